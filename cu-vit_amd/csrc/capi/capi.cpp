@@ -393,6 +393,22 @@ int layer_norm_cached(const std::uint16_t* input, const float* gamma, const floa
                     "layer_norm launch");
 }
 
+bool attention_long_supported(std::int64_t pairs, int tokens, int heads, int head_dim, int element_size) {
+    return detail::attention_long_supported(pairs, tokens, heads, head_dim, element_size);
+}
+
+int attention_long(const float* qkv, float* context, int images, int heads, int tokens,
+                   hipStream_t stream) {
+    return from_hip(detail::attention_long_f32(qkv, context, images, heads, tokens, stream),
+                    "attention launch");
+}
+
+int attention_long(const std::uint16_t* qkv, std::uint16_t* context, int images, int heads, int tokens,
+                   hipStream_t stream) {
+    return from_hip(detail::attention_long_bf16(qkv, context, images, heads, tokens, stream),
+                    "attention launch");
+}
+
 } // namespace cuvit::capi
 
 using namespace cuvit;

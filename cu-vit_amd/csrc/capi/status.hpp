@@ -62,6 +62,15 @@ int extract_patches_f32_to_bf16(const float* images, std::uint16_t* patches, int
                                 int channels, int height, int width, int patch,
                                 hipStream_t stream, bool* fused);
 
+/// Attention beyond cuvit_attention_supported()'s 256 tokens for the model's
+/// blocks (attention_long.hip): whether the shape is covered, and the launch.
+/// The C ABI's attention keeps its limits.
+bool attention_long_supported(std::int64_t pairs, int tokens, int heads, int head_dim, int element_size);
+int attention_long(const float* qkv, float* context, int images, int heads, int tokens,
+                   hipStream_t stream);
+int attention_long(const std::uint16_t* qkv, std::uint16_t* context, int images, int heads, int tokens,
+                   hipStream_t stream);
+
 /// The checks of preprocess (image.cpp:96-104, 126-128), in its order: an
 /// empty image, a non-positive size, a crop fraction outside (0, 1], a zero
 /// standard deviation.

@@ -7,7 +7,8 @@
 // the reference's Q.K^T GEMM (alpha 1/sqrt(head_dim), split batch over
 // (image, head)) -> softmax in place -> attention.V GEMM written straight into
 // [tokens, heads * head_dim]; where the shape allows it runs as one fused
-// launch with bitwise the same result and no logits buffer.
+// launch with bitwise the same result and no logits buffer, or beyond 256
+// tokens as one launch with a running softmax (attention_long.hip).
 // Around the blocks (forward, vit.cu:263-317): patch gather -> embedding GEMM
 // into rows 1.. of each image -> class token into row 0 -> positional add ->
 // blocks -> final LN -> head GEMM on the class rows only. Here the positional
@@ -317,6 +318,13 @@ template <typename T> void VisionTransformer::reserve_activations(Stored<T>& sto
                        static_cast<std::int64_t>(max_batch_) * config_.heads <= 65535 &&
                        static_cast<std::int64_t>(config_.token_count()) * 3 * config_.embed_dim *
                                static_cast<std::int64_t>(sizeof(T)) <= 0x7FFFFFF0;
+    // Beyond the fused kernels' tokens, the one-pass kernel. Against the three
+    // launches it replaces at 577 tokens: 8 images of 6 heads in bf16 125 -> 14
+    // us a layer, 8 of 5 in fp32 109 -> 44.
+    long_attention_ = cuvit_attention_supported(config_.token_count(), config_.head_dim()) == 0 &&
+                      capi::attention_long_supported(static_cast<std::int64_t>(max_batch_) * config_.heads,
+                                                     config_.token_count(), config_.heads, config_.head_dim(),
+                                                     static_cast<int>(sizeof(T)));
 
     const Extent images = max_batch_;
     const Extent embed = config_.embed_dim;
@@ -329,7 +337,7 @@ template <typename T> void VisionTransformer::reserve_activations(Stored<T>& sto
         images * tokens * embed,                                              // residual stream
         images * tokens * embed,                                              // normalized
         images * tokens * 3 * embed,                                          // packed q, k, v
-        fused_attention_ ? 0 : images * config_.heads * tokens * tokens,      // attention logits
+        fused_attention_ || long_attention_ ? 0 : images * config_.heads * tokens * tokens, // attention logits
         images * tokens * embed,                                              // attention context
         images * tokens * hidden,                                             // MLP hidden
         kFloat ? 0 : images * config_.classes,                                // logits in bf16
@@ -426,6 +434,8 @@ void VisionTransformer::run_block(const BlockWeights& block,
             throw_on_error(cuvit_attention_bf16(stored.qkv, stored.context, batch, heads,
                                                 token_count, head_dim, as_c(stream)));
         }
+    } else if (long_attention_) {
+        throw_on_error(capi::attention_long(stored.qkv, stored.context, batch, heads, token_count, stream));
     } else {
         attention_unfused(stored, batch, stream);
     }

@@ -28,8 +28,7 @@
 // owns one (image, head) and up to kWaves query tiles of 16 rows; K and V of
 // that (image, head) sit in LDS as [key][head_dim + 4] fp32 (padded rows give
 // conflict-free 16-byte fragment reads).
-#include "device_common.hpp"
-#include "gemm_kernel.hpp"
+#include "attention_common.hpp"
 #include "launch.hpp"
 
 #include <cmath>
@@ -37,33 +36,14 @@
 namespace cuvit::detail {
 namespace {
 
+using namespace attention;
 using namespace cuvit::device;
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
-constexpr int kHeadDim = 64;          // head_dim this kernel handles
 constexpr int kPitch = kHeadDim + 4;  // floats per LDS row
 constexpr int kMaxKeyTiles = 16;      // up to 256 tokens
 constexpr float kLog2e = 1.4426950408889634F;
-
-/// op(value of lanes 16 k + i, value of lanes 16 (k + 1) + i) for k = 0 and
-/// k = 2, in both lanes of each pair (@p kRows 16: rows of 16 lanes, by
-/// v_permlane16_swap), or op(lower half, upper half) (@p kRows 32, by
-/// v_permlane32_swap): a swap of the value with itself leaves each lane its
-/// own value and its partner's, the lower one first in both lanes, with no LDS
-/// round trip. op is max or + here, which give the same bits as
-/// op(own, partner) in either order.
-template <int kRows, typename Op> __device__ __forceinline__ float combine_rows(float value, Op op) {
-    const std::uint32_t bits = __float_as_uint(value);
-    if constexpr (kRows == 16) {
-        const auto swapped = __builtin_amdgcn_permlane16_swap(bits, bits, false, false);
-        return op(__uint_as_float(swapped[0]), __uint_as_float(swapped[1]));
-    } else {
-        static_assert(kRows == 32, "rows of 16 or halves of 32 lanes");
-        const auto swapped = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
-        return op(__uint_as_float(swapped[0]), __uint_as_float(swapped[1]));
-    }
-}
 
 template <int KT, int Waves>
 __global__ __launch_bounds__(Waves * kWave) void attention_kernel(const float* __restrict__ qkv,

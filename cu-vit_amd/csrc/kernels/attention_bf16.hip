@@ -50,8 +50,7 @@
 // (the transposed layout this replaces took eight 2-byte stores a chunk,
 // about half of the kernel's LDS cycles lost to bank conflicts). Q fragments
 // are read straight from global memory (16 contiguous bytes).
-#include "device_common.hpp"
-#include "gemm_kernel.hpp"
+#include "attention_common.hpp"
 #include "launch.hpp"
 #include "softmax_terms.hpp"
 
@@ -60,13 +59,13 @@
 namespace cuvit::detail {
 namespace {
 
+using namespace attention;
 using namespace cuvit::device;
 using gemm::Mma;
 
 using Bf16Mma = Mma<std::uint16_t>;
 using Acc = Bf16Mma::Acc;
 
-constexpr int kHeadDim = 64;
 constexpr int kEdge = 32;        // MFMA tile edge: 32 queries x 32 keys (or dims)
 constexpr int kKBlock = 16;      // k per MFMA
 constexpr int kStage = 64;       // the GEMM's k stage
@@ -79,69 +78,12 @@ constexpr int kWavesPerGroup = 4;
 constexpr float kScaledLog2e = kLog2e * 0.125F;
 static_assert(kHeadDim == 64, "the logits' scale is 1/8");
 
-/// Elements per LDS row of K ([key][head_dim + 8]).
-constexpr int kKeyPitch = kHeadDim + 8;
 /// 16-byte chunks of one key's K or V row.
 constexpr int kChunksPerKey = kHeadDim / 8;
 
 /// V ([key][head_dim]), then K.
 __host__ __device__ constexpr std::size_t lds_bytes(int key_tiles) {
     return static_cast<std::size_t>(key_tiles) * kEdge * (kHeadDim + kKeyPitch) * 2;
-}
-
-/// Element offset of V[key][dim] in its LDS tile: 16-byte chunk dim / 8 of
-/// the key's row sits at chunk (dim / 8) ^ 4 ((key >> 1) & 1).
-__device__ __forceinline__ int value_slot(int key, int dim) {
-    return key * kHeadDim + 8 * ((dim >> 3) ^ (4 * ((key >> 1) & 1))) + (dim & 7);
-}
-
-/// Four 16-bit elements in LDS, the operand type of ds_read_b64_tr_b16.
-typedef short Short4 __attribute__((vector_size(4 * sizeof(short))));
-using Lds4x16 = __attribute__((address_space(3))) Short4;
-
-/// The weights.V B fragment of k-block @p kb, dims @p d0 + 0..31: lane l
-/// holds dim d0 + l % 32, keys 16 kb + 8 (l / 32) + 0..7, the layout a
-/// 16-byte row of transposed V would give it.
-__device__ __forceinline__ Vec16 value_fragment(const std::uint16_t* values, int kb, int d0,
-                                                int lane) {
-    const int j = lane & 15;
-    const int dim = d0 + 16 * ((lane >> 4) & 1) + 4 * (j & 3);
-    Vec16 fragment;
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-        const int key = kb * 16 + 8 * (lane >> 5) + 4 * s + (j >> 2);
-        // `values` points into LDS; the C-style cast is the address-space
-        // conversion the builtin's operand needs.
-        const auto part =
-            __builtin_amdgcn_ds_read_tr16_b64_v4i16((Lds4x16*)(values + value_slot(key, dim)));
-        fragment.w[2 * s] = static_cast<std::uint16_t>(part[0]) |
-                            (static_cast<std::uint32_t>(static_cast<std::uint16_t>(part[1])) << 16);
-        fragment.w[2 * s + 1] = static_cast<std::uint16_t>(part[2]) |
-                                (static_cast<std::uint32_t>(static_cast<std::uint16_t>(part[3])) << 16);
-    }
-    return fragment;
-}
-
-/// 16 bytes at @p element of the pair's packed projection, through the
-/// buffer resource @p resource (based at that element 0), or zero when
-/// @p inside is false: the offset is then one the resource drops, so the load
-/// needs no branch. Element offsets stay far inside 32 bits (at most 256
-/// tokens of 3 * heads * 64 elements).
-__device__ __forceinline__ Vec16 load_or_zero(__amdgpu_buffer_rsrc_t resource, std::int64_t element,
-                                              bool inside) {
-    return gemm::buffer_load16(resource, inside ? static_cast<unsigned int>(element * 2) : gemm::kOutside);
-}
-
-/// op(the lower half's value, the upper half's value) in lanes l and l ^ 32
-/// alike: one v_permlane32_swap of the value with itself leaves a lane of the
-/// lower half its own value and its partner's, and a lane of the upper half
-/// its partner's and its own, lower half first in both (no LDS round trip).
-/// The two halves then hold the same bits; op is max or + here, which give
-/// the same bits as op(own, partner) in either order.
-template <typename Op> __device__ __forceinline__ float combine_halves(float value, Op op) {
-    const std::uint32_t bits = __float_as_uint(value);
-    const auto swapped = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
-    return op(__uint_as_float(swapped[0]), __uint_as_float(swapped[1]));
 }
 
 __device__ __forceinline__ std::uint32_t pack_bf16(float low, float high) {

@@ -129,6 +129,16 @@ bool attention_bf16_supported(int tokens, int head_dim);
 hipError_t attention_bf16(const std::uint16_t* qkv, std::uint16_t* context, int images, int heads,
                           int tokens, int head_dim, hipStream_t stream);
 
+/// The same for any number of tokens (attention_long.hip): one pass over the
+/// keys with a running softmax, so not bitwise the three launches, whose
+/// rounded bf16 logits it does not round. Bases 16-byte aligned, head_dim 64;
+/// attention_long_supported() gives the limits.
+bool attention_long_supported(std::int64_t pairs, int tokens, int heads, int head_dim, int element_size);
+hipError_t attention_long_f32(const float* qkv, float* context, int images, int heads, int tokens,
+                              hipStream_t stream);
+hipError_t attention_long_bf16(const std::uint16_t* qkv, std::uint16_t* context, int images, int heads,
+                               int tokens, hipStream_t stream);
+
 // Device facts used to shape grids, cached per device.
 int compute_units();
 

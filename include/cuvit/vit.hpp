@@ -134,7 +134,8 @@ class VisionTransformer final {
     VitConfig config_;
     int max_batch_ = 1;
     Precision precision_ = Precision::kFloat32;
-    bool fused_attention_ = false;
+    bool fused_attention_ = false; // at most 256 tokens: bitwise the three launches
+    bool long_attention_ = false;  // more tokens: one launch, running softmax
 
     DeviceArena weights_;
     DeviceArena activations_;
