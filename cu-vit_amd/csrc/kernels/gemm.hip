@@ -5,25 +5,23 @@
 //        linear layers and patch embedding); else the tiled kernel
 //        (gemm_kernel.hpp), 32 x 32 tiles, 64 x 64 once a problem has work
 //        for more than 32 small tiles per compute unit.
-//   bf16 (32 x 32 MFMA): the wide kernel (gemm_wide.hpp, 128 x 256 tiles)
-//        for large products without accumulation (ViT-Base FC1, QKV); the
-//        tiled kernel's twelve-wavefront 256 x 192 tile when one round of it
-//        covers a product that 128 x 128 tiles would need more than two per
-//        compute unit for (ViT-Base FC2, projection, patch embedding); else
-//        128 x 128 once a problem fills every compute unit twice with it
-//        (32-deep stages up to K = 1024), else 64 x 64.
+//   bf16 (32 x 32 MFMA): B as [N, K] with 16-byte rows runs on direct-to-LDS
+//        loads, in the persistent kernel (gemm_dma.hpp, up to 320 x 256 tiles)
+//        where its tiles fill the chip and in the ring kernel (gemm_ring.hpp,
+//        64 x 64 to 128 x 128 tiles) otherwise, by a cost fitted to both; else
+//        (B as [K, N], odd rows) the tiled kernel, 128 x 128 once a problem
+//        fills every compute unit twice with it (32-deep stages up to K =
+//        1024), else 64 x 64.
 // Every kernel of a type runs the same MFMA over K in the same order, so the
 // choice never changes a result.
 #include "gemm_dma.hpp"
 #include "gemm_kernel.hpp"
 #include "gemm_panel.hpp"
-#include "gemm_wide.hpp"
 
 namespace cuvit::detail {
 namespace {
 
 using cuvit::device::aligned16;
-using gemm::kThreads;
 using gemm::Shape;
 
 constexpr int kMaxGridY = 65535;
@@ -271,67 +269,12 @@ hipError_t gemm_f32(const float* a, const float* b, const float* bias, float* c,
     return pick_flags<float, 2, 2, 1, 1, 32>(a, b, bias, c, args, stream);
 }
 
-/// The wide-tile kernel (gemm_wide.hpp) for a problem it covers: B as [N, K],
-/// A and B vector operands within one descriptor's span, C written whole in
-/// 16-byte pieces (N, ldc and the C strides multiples of 8, C 16-byte aligned),
-/// no accumulation and no addend, and enough 128 x 256 tiles to fill every
-/// CU's two slots. Returns hipErrorNotSupported otherwise.
-template <int TM, int TN>
-hipError_t launch_wide(const std::uint16_t* a, const std::uint16_t* b, const float* bias,
-                       std::uint16_t* c, const GemmArgs& args, hipStream_t stream) {
-    using S = gemm::WideShape<TM, TN>;
-    const bool split = args.inner > 0;
-    const bool eligible =
-        args.transposed && !args.accumulate && args.addend == nullptr &&
-        vector_operand(a, args.lda, args.k, args.stride_a, args.outer_stride_a, split) &&
-        vector_operand(b, args.ldb, args.k, args.stride_b, args.outer_stride_b, split) &&
-        static_cast<std::int64_t>(S::kBM) * args.lda * 2 < gemm::kMaxSpan &&
-        static_cast<std::int64_t>(S::kBN) * args.ldb * 2 < gemm::kMaxSpan && aligned16(c) &&
-        args.n % 8 == 0 && args.ldc % 8 == 0 && args.stride_c % 8 == 0 &&
-        (!split || args.outer_stride_c % 8 == 0) &&
-        tile_count(args, S::kBM, S::kBN) >= static_cast<std::int64_t>(compute_units()) * 2;
-    if (!eligible) {
-        return hipErrorNotSupported;
-    }
-    const gemm::TileMap map = tile_map(args, S::kBM, S::kBN, 2);
-    const std::int64_t tiles_m = (args.m + S::kBM - 1) / S::kBM;
-    const std::int64_t tiles_n = (args.n + S::kBN - 1) / S::kBN;
-    const std::int64_t tiles = map.px > 0 ? 8 * ((tiles_m + map.px - 1) / map.px) *
-                                                ((tiles_n + map.py - 1) / map.py)
-                                          : tiles_m * tiles_n;
-    if (tiles > 0x7FFFFFFF) {
-        return hipErrorNotSupported;
-    }
-    const dim3 grid(static_cast<unsigned int>(tiles),
-                    static_cast<unsigned int>(args.count < kMaxGridY ? args.count : kMaxGridY));
-    auto run = [&](auto kernel) -> hipError_t {
-        static std::atomic<std::uint64_t> opted_in{0};
-        if (const hipError_t opted =
-                allow_lds(reinterpret_cast<const void*>(kernel), S::kLdsBytes, opted_in);
-            opted != hipSuccess) {
-            return opted;
-        }
-        kernel<<<grid, kThreads, S::kLdsBytes, stream>>>(a, b, bias, c, args, map);
-        return hipGetLastError();
-    };
-    auto pick = [&](auto with_alpha) -> hipError_t {
-        constexpr bool kAlpha = decltype(with_alpha)::value;
-        if (bias != nullptr) {
-            return args.gelu ? run(gemm::gemm_wide_kernel<TM, TN, true, true, kAlpha>)
-                             : run(gemm::gemm_wide_kernel<TM, TN, true, false, kAlpha>);
-        }
-        return args.gelu ? run(gemm::gemm_wide_kernel<TM, TN, false, true, kAlpha>)
-                         : run(gemm::gemm_wide_kernel<TM, TN, false, false, kAlpha>);
-    };
-    return args.alpha == 1.0F ? pick(std::false_type{}) : pick(std::true_type{});
-}
-
 /// The XCD split for a persistent kernel whose @p turns workgroups per XCD
 /// take an XCD's tiles in turn: fewest rounds (the largest block's tiles over
 /// @p turns), then the fewest bytes moved into the L2 caches (tile_map's
 /// measure). Measured at ViT-Base FC2 on 192 x 256 tiles: a byte-only choice
 /// left one XCD 34 tiles for its 32 workgroups, 139 against 88 us.
-gemm::TileMap balanced_map(const GemmArgs& args, int bm, int bn, int turns) {
+gemm::TileMap balanced_map(const GemmArgs& args, int bm, int bn, int turns, int* rounds_out) {
     const int tiles_m = (args.m + bm - 1) / bm;
     const int tiles_n = (args.n + bn - 1) / bn;
     const double a_bytes = static_cast<double>(tiles_m) * bm * args.k * 2;
@@ -357,6 +300,50 @@ gemm::TileMap balanced_map(const GemmArgs& args, int bm, int bn, int turns) {
             best_rounds = rounds;
         }
     }
+    *rounds_out = best_rounds;
+    return best;
+}
+
+/// Relative times of the bf16 kernels with B as [N, K], one 64 x 64 ring tile
+/// per CU without GELU being 1, all proportional to K: a CU's row of ring tiles
+/// takes ceil(tiles / CUs) times the tile's cost, the persistent kernel rounds x
+/// BM times its cost per row of a 256-wide tile. Fitted to MI355X times at K =
+/// 384 and 768, M from 197 to 12608 (us at K = 768: a 64 x 64 tile 2.65, 128 x
+/// 64 4.4, 128 x 128 7.7, a persistent 192-row tile 16.7; at K = 384: 1.6, 2.6,
+/// 4.2). The GELU weighs more where fewer wavefronts share a SIMD.
+constexpr double kRingCost[3] = {1.0, 1.65, 2.9};
+constexpr double kRingCostGelu[3] = {1.1, 1.85, 3.3};
+constexpr double kDmaRow = 0.035;
+constexpr double kDmaRowGelu = 0.043;
+
+struct RingChoice {
+    RingTile tile;
+    int bm;
+    int bn;
+    double cost;
+};
+
+/// The ring kernel's cheapest tile for a problem. A 128 x 128 tile that is
+/// alone on its CU takes three stages once K is long (768 x 3072 on 4616 rows:
+/// 31 -> 27 us; two tiles per CU with two stages each beat one at a time with
+/// three, 40 against 51 us on 6304 rows).
+RingChoice choose_ring(const GemmArgs& args) {
+    constexpr RingTile kTiles[3] = {RingTile::k64x64, RingTile::k128x64, RingTile::k128x128};
+    constexpr int kHeights[3] = {64, 128, 128};
+    constexpr int kWidths[3] = {64, 64, 128};
+    const std::int64_t units = compute_units();
+    RingChoice best{RingTile::k64x64, 64, 64, 0.0};
+    for (int i = 0; i < 3; ++i) {
+        const std::int64_t tiles = tile_count(args, kHeights[i], kWidths[i]);
+        const double cost = static_cast<double>((tiles + units - 1) / units) *
+                            (args.gelu ? kRingCostGelu[i] : kRingCost[i]);
+        if (i == 0 || cost < best.cost) {
+            best = RingChoice{kTiles[i], kHeights[i], kWidths[i], cost};
+            if (i == 2 && tiles <= units && args.k >= 1024) {
+                best.tile = RingTile::k128x128Deep;
+            }
+        }
+    }
     return best;
 }
 
@@ -365,15 +352,15 @@ gemm::TileMap balanced_map(const GemmArgs& args, int bm, int bn, int turns) {
 /// vector A and B, C written in 16-byte pieces, every operand tile within one
 /// descriptor's span, the CUs a multiple of 8 (one persistent workgroup per
 /// CU, eight per XCD) and BM x 256 tiles for at least half the CUs. BM is the
-/// height with the fewest rounds x BM (ViT-Base b64: 320 for FC1, 256 for QKV,
-/// 192 for FC2 and the projection). Returns hipErrorNotSupported otherwise.
+/// height with the fewest rounds x BM, the rounds as balanced_map's split
+/// gives them (ViT-Base b64: 320 for FC1, 256 for QKV, 192 for FC2 and the
+/// projection). Returns hipErrorNotSupported otherwise, and where the ring
+/// kernel's @p ring_cost is the smaller one.
 hipError_t launch_dma(const std::uint16_t* a, const std::uint16_t* b, const float* bias,
-                      std::uint16_t* c, const GemmArgs& problem, hipStream_t stream) {
+                      std::uint16_t* c, const GemmArgs& args, double ring_cost, hipStream_t stream) {
     const int units = compute_units();
-    // A batch whose entries share B and follow one another in A runs as one
-    // problem, each row stored back in its entry: the patch embedding, with
-    // its positional addend (the instance that takes entries).
-    const GemmArgs args = as_one_problem(problem);
+    // Entries run as one problem, each row stored back in its entry: the patch
+    // embedding, with its positional addend (the instance that takes entries).
     const bool with_addend = args.addend != nullptr;
     const bool entries = args.rows_per_entry > 0;
     // The addend only in the combination the model uses (bias, no alpha, no
@@ -392,24 +379,28 @@ hipError_t launch_dma(const std::uint16_t* a, const std::uint16_t* b, const floa
     if (!eligible) {
         return hipErrorNotSupported;
     }
+    const int turns = units / 8;
     int bm = 0;
-    std::int64_t best = 0;
+    int rounds = 0;
+    gemm::TileMap map{0, 0};
     for (const int height : {192, 256, 320}) {
         if (with_addend && height == 320) {
             continue;  // the addend's registers would spill at 320 rows
         }
-        const std::int64_t tiles = tile_count(args, height, 256);
-        const std::int64_t cost = (tiles + units - 1) / units * height;
-        if (bm == 0 || cost < best) {
+        if (2 * tile_count(args, height, 256) < units) {
+            continue;  // fewer tiles than half the CUs: the ring kernel
+        }
+        int height_rounds = 0;
+        const gemm::TileMap split = balanced_map(args, height, 256, turns, &height_rounds);
+        if (bm == 0 || height_rounds * height < rounds * bm) {
             bm = height;
-            best = cost;
+            rounds = height_rounds;
+            map = split;
         }
     }
-    if (2 * tile_count(args, bm, 256) < units) {
-        return hipErrorNotSupported;  // fewer tiles than half the CUs: the other kernels
+    if (bm == 0 || ring_cost < rounds * bm * (args.gelu ? kDmaRowGelu : kDmaRow)) {
+        return hipErrorNotSupported;
     }
-    const int turns = units / 8;
-    const gemm::TileMap map = balanced_map(args, bm, 256, turns);
     auto run = [&](auto kernel, std::size_t lds_bytes) -> hipError_t {
         static std::atomic<std::uint64_t> opted_in{0};
         if (const hipError_t opted = allow_lds(reinterpret_cast<const void*>(kernel), lds_bytes, opted_in);
@@ -456,58 +447,41 @@ hipError_t launch_dma(const std::uint16_t* a, const std::uint16_t* b, const floa
 
 hipError_t gemm_bf16(const std::uint16_t* a, const std::uint16_t* b, const float* bias,
                      std::uint16_t* c, const GemmArgs& args, hipStream_t stream) {
-    // The direct-to-LDS kernel where it applies (ViT-Base b64 against the
-    // kernels below, same bits, two input sets: FC1 + GELU 99 -> 87 us, QKV
-    // 61 -> 50, FC2 accumulating 81 -> 67, the projection 38 -> 26; the patch
-    // embedding 51 -> 29 inside the forward. With A from HBM now 78, 52, 68
-    // and 27 us).
-    if (const hipError_t dma = launch_dma(a, b, bias, c, args, stream); dma != hipErrorNotSupported) {
-        return dma;
-    }
-    // 128 x 256 tiles with 64 x 128 per wavefront (ViT-Base FC1 + GELU 137 ->
-    // 110 us), where they apply; bitwise the same results as the tiles below.
-    if (const hipError_t wide = launch_wide<2, 4>(a, b, bias, c, args, stream);
-        wide != hipErrorNotSupported) {
-        return wide;
-    }
-    // One round of 256 x 192 tiles, twelve wavefronts of 64 x 64 (three per
-    // SIMD), for products with B as [N, K] that would need more than two
-    // 128 x 128 tiles per CU: each CU then streams one tile's whole K, with
-    // three wavefronts per SIMD to cover the loads (ViT-Base FC2 12608 x 768 x
-    // 3072, accumulating: 110 -> 81 us; the projection, K = 768: 43 -> 40 us).
-    // Eight wavefronts of 64 x 96 ran FC2 in 92-95 us and the projection in
-    // 49: two per SIMD left the waves waiting on their loads 54% of the time.
-    // A batch whose entries' A rows follow one another and share B (the
-    // model's patch embedding: 196 rows per image into rows 1.. of its 197)
-    // runs as one problem of all the rows, so tiles do not stop at entry
-    // boundaries (ViT-Base b64 embedding 53 -> 41 us).
-    const std::int64_t units = compute_units();
+    // B as [N, K] with 16-byte rows: the persistent kernel (ViT-Base b64: FC1 +
+    // GELU 78 us, QKV 52, FC2 accumulating 68, the projection 27) or the ring
+    // kernel, whichever the costs above say is faster. A batch whose entries'
+    // A rows follow one another and share B (the patch embedding) runs as one
+    // problem of all the rows, so tiles do not stop at entry boundaries.
     const GemmArgs whole = as_one_problem(args);
-    if (whole.transposed && whole.k >= 512 && tile_count(whole, 256, 192) <= units &&
-        tile_count(whole, 128, 128) > 2 * units) {
-        using S = Shape<std::uint16_t, 4, 3, 2, 2, 64>;
-        const bool split = whole.inner > 0;
-        if (vector_operand(a, whole.lda, whole.k, whole.stride_a, whole.outer_stride_a, split) &&
-            vector_operand(b, whole.ldb, whole.k, whole.stride_b, whole.outer_stride_b, split) &&
-            static_cast<std::int64_t>(S::kBM) * whole.lda * 2 < gemm::kMaxSpan &&
-            static_cast<std::int64_t>(S::kBN) * whole.ldb * 2 < gemm::kMaxSpan) {
-            return launch<std::uint16_t, 4, 3, 2, 2, 64, 3, true, true, true>(
-                a, b, bias, c, whole, vector_output(c, whole), stream);
+    const bool split = whole.inner > 0;
+    const bool vector_c = aligned16(c) && whole.n % 8 == 0 && whole.ldc % 8 == 0 && whole.stride_c % 8 == 0 &&
+                          (!split || whole.outer_stride_c % 8 == 0);
+    const bool addend_ok = whole.addend == nullptr ||
+                           (vector_c && bias != nullptr && !whole.gelu && !whole.accumulate &&
+                            aligned16(whole.addend) && whole.ld_addend % 4 == 0);
+    if (whole.transposed && addend_ok &&
+        vector_operand(a, whole.lda, whole.k, whole.stride_a, whole.outer_stride_a, split) &&
+        vector_operand(b, whole.ldb, whole.k, whole.stride_b, whole.outer_stride_b, split) &&
+        static_cast<std::int64_t>(128) * whole.lda * 2 < gemm::kMaxSpan &&
+        static_cast<std::int64_t>(128) * whole.ldb * 2 < gemm::kMaxSpan) {
+        const RingChoice ring = choose_ring(whole);
+        if (const hipError_t dma = launch_dma(a, b, bias, c, whole, ring.cost, stream);
+            dma != hipErrorNotSupported) {
+            return dma;
         }
+        const gemm::TileMap map = tile_map(whole, ring.bm, ring.bn, 2);
+        return gemm_ring_bf16(ring.tile, a, b, bias, c, whole, map.px, map.py, vector_c, stream);
     }
+    const std::int64_t units = compute_units();
     if (tile_count(args, 128, 128) >= units * 2) {
         // Up to K = 1024, 32-deep stages with registers for three workgroups
-        // per CU beat 64-deep ones at two (ViT-Base FC1 + GELU 146 -> 136 us,
-        // QKV 103 -> 96, projection 45.5 -> 38.4); FC2 (K = 3072) keeps the
-        // 64-deep stages (95 against 99 us).
+        // per CU; 64-deep stages beyond.
         if (args.k <= 1024) {
             return pick_flags<std::uint16_t, 2, 2, 2, 2, 32, 3>(a, b, bias, c, args, stream);
         }
         return pick_flags<std::uint16_t, 2, 2, 2, 2, 64>(a, b, bias, c, args, stream);
     }
-    // 64 x 64: 32-deep stages for short K (ViT-Tiny FC1 6304 x 768 x 192 with
-    // GELU: 13.4 against 16.1 us), 64-deep beyond (FC2, K = 768: 10.9 against
-    // 11.7 us).
+    // 64 x 64: 32-deep stages for short K, 64-deep beyond.
     if (args.k <= 512) {
         return pick_flags<std::uint16_t, 2, 2, 1, 1, 32>(a, b, bias, c, args, stream);
     }

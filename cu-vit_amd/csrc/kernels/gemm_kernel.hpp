@@ -9,8 +9,7 @@
 // (entry * stride) or split into (entry / inner, entry % inner) with outer
 // strides (gemm.cu:58-72); every operand has its own leading dimension.
 //
-// Structure. A workgroup of WM x WN wavefronts (four, or twelve for the
-// largest bf16 tile) owns a BM x BN tile of C; each
+// Structure. A workgroup of four (WM x WN) wavefronts owns a BM x BN tile of C; each
 // wavefront owns (TM * E) x (TN * E) of it as TM x TN MFMA tiles of edge E.
 // K is walked in BK-wide stages. Both operand tiles sit in LDS as
 // [rows][BK] (k contiguous), rows padded by 16 bytes so that the sixteen
@@ -55,9 +54,6 @@ using namespace cuvit::device;
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-
-/// Threads of a four-wavefront workgroup (the wide and tiled bf16 kernels).
-constexpr int kThreads = 256;
 
 /// The MFMA of each storage type. kEdge is the MFMA tile's edge; a lane's
 /// accumulator holds kRuns runs of four consecutive columns of row
@@ -236,7 +232,7 @@ __device__ __forceinline__ void store4(std::uint16_t* p, const float (&value)[4]
 
 /// Compile-time shape of one kernel instance.
 template <typename T, int WM, int WN, int TM, int TN, int BK> struct Shape {
-    static_assert(WM * WN == 4 || WM * WN == 12, "four or twelve wavefronts per workgroup");
+    static_assert(WM * WN == 4, "four wavefronts per workgroup");
     static constexpr int kThreads = kWave * WM * WN;
     static constexpr int kE = Mma<T>::kEdge;
     static constexpr int kBM = WM * TM * kE;
@@ -304,9 +300,6 @@ __global__ __launch_bounds__(kWave * WM * WN) __attribute__((amdgpu_waves_per_eu
                                                         const float* __restrict__ bias, T* c,
                                                         GemmArgs args, TileMap map, bool vector_c) {
     using S = Shape<T, WM, WN, TM, TN, BK>;
-    // Explicit MFMA / memory interleave for the bf16 tiles whose stages are
-    // whole 16-byte chunks written as such (vector A and B, B as [N, K]).
-    constexpr bool kInterleave = sizeof(T) == 2 && VecA && VecB && TransB && TM * TN >= 4;
     constexpr int BM = S::kBM;
     constexpr int BN = S::kBN;
     constexpr int P = S::kPitch;
@@ -485,44 +478,13 @@ __global__ __launch_bounds__(kWave * WM * WN) __attribute__((amdgpu_waves_per_eu
 
         // One stage of the loop: the MFMAs over LDS buffer @p buffer, the
         // next stage's registers into the other buffer, and the loads of the
-        // stage two further on into the registers just freed. With
-        // kInterleave the MFMA stream is ordered explicitly: the first
-        // k-block's fragments, then one MFMA per fragment read for the
-        // following k-blocks, and the LDS writes and global loads spread
-        // over the last k-block's MFMAs (measured on the ViT-Base bf16
-        // GEMMs: FC1 + GELU 165 -> 147 us, FC2 107 -> 94 us). The order of
-        // the MFMAs, and so every result bit, is the same either way.
+        // stage two further on into the registers just freed.
         auto advance = [&](const Vec16 (&ra)[S::kAPerThread], const Vec16 (&rb)[S::kBPerThread],
                            Vec16 (&la)[S::kAPerThread], Vec16 (&lb)[S::kBPerThread], int buffer,
                            int next_fetch) {
-            if constexpr (kInterleave) {
-                compute(buffer);
-                stage(ra, rb, buffer ^ 1);
-                fetch(la, lb, next_fetch);
-                constexpr int kBlocks = BK / S::kKBlock;
-                constexpr int kMfma = TM * TN * kBlocks;
-                constexpr int kReads = (TM + TN) * kBlocks;
-                constexpr int kPaired = kReads - (TM + TN);
-                constexpr int kRest = kMfma - kPaired;
-                constexpr int kWrites = (S::kAPerThread + S::kBPerThread + kRest - 1) / kRest;
-                static_assert(kRest > 0, "more MFMAs than fragment reads");
-                __builtin_amdgcn_sched_group_barrier(0x100, TM + TN, 0); // DS reads
-#pragma unroll
-                for (int i = 0; i < kPaired; ++i) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); // MFMA
-                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0); // DS read
-                }
-#pragma unroll
-                for (int i = 0; i < kRest; ++i) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);        // MFMA
-                    __builtin_amdgcn_sched_group_barrier(0x200, kWrites, 0);  // DS write
-                    __builtin_amdgcn_sched_group_barrier(0x020, kWrites, 0);  // VMEM read
-                }
-            } else {
-                stage(ra, rb, buffer ^ 1);
-                fetch(la, lb, next_fetch);
-                compute(buffer);
-            }
+            stage(ra, rb, buffer ^ 1);
+            fetch(la, lb, next_fetch);
+            compute(buffer);
         };
 
         // Stage s sits in LDS buffer s % 2. Register set 0 carries even

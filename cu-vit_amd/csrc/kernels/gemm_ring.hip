@@ -1,0 +1,68 @@
+// Launch of the LDS-ring bf16 GEMM (gemm_ring.hpp): its instances, one
+// translation unit of their own.
+#include "gemm_ring.hpp"
+
+namespace cuvit::detail {
+namespace {
+
+constexpr int kMaxGridY = 65535;
+
+template <typename S>
+hipError_t launch(const std::uint16_t* a, const std::uint16_t* b, const float* bias, std::uint16_t* c,
+                  const GemmArgs& args, const gemm::TileMap& map, bool vector_c, hipStream_t stream) {
+    const std::int64_t tiles_m = (args.m + S::kBM - 1) / S::kBM;
+    const std::int64_t tiles_n = (args.n + S::kBN - 1) / S::kBN;
+    const std::int64_t tiles = map.px > 0 ? 8 * ((tiles_m + map.px - 1) / map.px) *
+                                                ((tiles_n + map.py - 1) / map.py)
+                                          : tiles_m * tiles_n;
+    if (tiles > 0x7FFFFFFF) {
+        return hipErrorInvalidConfiguration;
+    }
+    auto run = [&](auto kernel) -> hipError_t {
+        static std::atomic<std::uint64_t> opted_in{0};
+        if (const hipError_t opted =
+                allow_lds(reinterpret_cast<const void*>(kernel), S::kLdsBytes, opted_in);
+            opted != hipSuccess) {
+            return opted;
+        }
+        // A grid's y extent is limited: more entries than that take several launches.
+        for (int first = 0; first < args.count; first += kMaxGridY) {
+            const int entries = args.count - first < kMaxGridY ? args.count - first : kMaxGridY;
+            const dim3 grid(static_cast<unsigned int>(tiles), static_cast<unsigned int>(entries));
+            kernel<<<grid, S::kThreads, S::kLdsBytes, stream>>>(a, b, bias, c, args, map, vector_c, first);
+            if (const hipError_t launched = hipGetLastError(); launched != hipSuccess) {
+                return launched;
+            }
+        }
+        return hipSuccess;
+    };
+    if (args.addend != nullptr) {
+        return run(gemm::gemm_ring_kernel<S, true, false, false, true>);
+    }
+    auto with_gelu = [&](auto with_bias) -> hipError_t {
+        constexpr bool kB = decltype(with_bias)::value;
+        if (args.gelu) {
+            return args.accumulate ? run(gemm::gemm_ring_kernel<S, kB, true, true>)
+                                   : run(gemm::gemm_ring_kernel<S, kB, true, false>);
+        }
+        return args.accumulate ? run(gemm::gemm_ring_kernel<S, kB, false, true>)
+                               : run(gemm::gemm_ring_kernel<S, kB, false, false>);
+    };
+    return bias != nullptr ? with_gelu(std::true_type{}) : with_gelu(std::false_type{});
+}
+
+} // namespace
+
+hipError_t gemm_ring_bf16(RingTile tile, const std::uint16_t* a, const std::uint16_t* b,
+                          const float* bias, std::uint16_t* c, const GemmArgs& args, int px, int py,
+                          bool vector_c, hipStream_t stream) {
+    const gemm::TileMap map{px, py};
+    switch (tile) {
+    case RingTile::k64x64: return launch<gemm::RingShape<2, 2, 1, 1, 2>>(a, b, bias, c, args, map, vector_c, stream);
+    case RingTile::k128x64: return launch<gemm::RingShape<2, 2, 2, 1, 2>>(a, b, bias, c, args, map, vector_c, stream);
+    case RingTile::k128x128: return launch<gemm::RingShape<4, 2, 1, 2, 2>>(a, b, bias, c, args, map, vector_c, stream);
+    default: return launch<gemm::RingShape<4, 2, 1, 2, 3>>(a, b, bias, c, args, map, vector_c, stream);
+    }
+}
+
+} // namespace cuvit::detail

@@ -1,0 +1,333 @@
+// The bf16 GEMM for products with B given as [N, K] that the persistent kernel
+// (gemm_dma.hpp) has too few tiles or no whole 256-column tiles for: one tile
+// per workgroup, operands brought into an LDS ring by direct-to-LDS loads.
+//
+// What bounds these. Tiles are few and K is short (6 to 48 stages of 64), so
+// a tile's time is the latency of its first loads, its LDS traffic and its
+// epilogue; and a CU's LDS, not its MFMAs, is the busiest unit: a 64-deep
+// stage of a 128 x 128 tile writes 32 KB and reads 96 KB of fragments for 512
+// cycles of MFMA per SIMD. Loads through registers (gemm_kernel.hpp) hold
+// registers and add a write instruction per 16 bytes; here the loads land by
+// themselves and two stages per workgroup leave room for two (128 x 128) to
+// four (64 x 64) workgroups per CU, which cover each other's waits. Measured
+// on MI355X with two, three, four and eight stages: two are the fastest of
+// each tile, except for a tile alone on its CU with a long K, which has
+// nothing but its own loads to hide behind and takes three (4616 x 768 x
+// 3072: 31 -> 27 us). Eight wavefronts of 32 x 64 beat four of 64 x 64 on the
+// 128 x 128 tile by a few percent (3152 x 2304 x 768: 16.1 against 16.2 us).
+// Before (gemm_kernel.hpp and gemm_dma.hpp) and now, bf16, us:
+//   4616 x 1152 x 384          18.0 ->  9.9    197 x 768 x 768 (+=)    8.6 -> 5.2
+//   4616 x 384 x 1536 (+=)     17.5 -> 10.6    1576 x 2304 x 768      17.4 -> 9.4
+//   4616 x 1536 x 384 (GELU)   18.2 -> 13.8    3152 x 2304 x 768      19.2 -> 16.1
+//   6304 x 192 x 768 (+=)      11.4 ->  6.5    12608 x 1152 x 384     38.2 -> 19.6
+//
+// Stages are 64 deep, rows of 128 bytes: chunk c of row r sits in 16-byte slot
+// c ^ ((r >> 1) & 7) of its row, conflict-free for the fragment reads (lane l:
+// row l % 32, chunk 2 kb + l / 32). One buffer_load_dwordx4 ... lds moves
+// eight rows; every wavefront loads the same number of pieces of A and of B
+// for each stage and waits for its own (vmcnt, the newest kSlots - 2 stages
+// staying in flight) before the stage's barrier. Loads past the last stage go
+// out too, with an offset past the descriptor's range (zeros, no traffic), so
+// that the count in flight is the same in every trip.
+//
+// Epilogue and arithmetic are gemm_dma.hpp's: 32 rows at a time through the
+// wavefront's own piece of the drained ring, stored as 16-byte pieces (single
+// elements where C's rows are not 16-byte aligned); the same MFMA over the
+// same K order, then alpha, bias, addend, GELU, old C, one rounding, so the
+// results are bitwise those of the other bf16 kernels. Old C is read before
+// the k loop.
+#pragma once
+
+#include "gemm_dma.hpp"
+
+namespace cuvit::detail::gemm {
+
+/// WM x WN wavefronts of TM x TN MFMA tiles (32 x 32), Slots stages in the ring.
+template <int WM, int WN, int TM, int TN, int Slots> struct RingShape {
+    static constexpr int kWaves = WM * WN;
+    static constexpr int kThreads = kWave * kWaves;
+    static constexpr int kWN = WN;
+    static constexpr int kTM = TM;
+    static constexpr int kTN = TN;
+    static constexpr int kBK = 64;
+    static constexpr int kBM = 32 * WM * TM;
+    static constexpr int kBN = 32 * WN * TN;
+    static constexpr int kSlots = Slots;
+    static constexpr int kRowBytes = 2 * kBK;
+    static constexpr int kChunks = kBK / 8;                  // 16-byte chunks per row
+    static constexpr int kLoadRows = 1024 / kRowBytes;       // rows of one load instruction
+    static constexpr int kLoadsA = kBM / kLoadRows / kWaves; // per wavefront and stage
+    static constexpr int kLoadsB = kBN / kLoadRows / kWaves;
+    static constexpr int kLoads = kLoadsA + kLoadsB;
+    static constexpr int kStageBytes = (kBM + kBN) * kRowBytes;
+    static constexpr int kBiasOffset = Slots * kStageBytes;
+    static constexpr int kLdsBytes = kBiasOffset + kBN * 4;
+    static constexpr int kStagingBytes = 32 * TN * 64; // 32 rows of a wavefront's columns
+    static_assert(kBM % (kLoadRows * kWaves) == 0 && kBN % (kLoadRows * kWaves) == 0,
+                  "every wavefront loads whole pieces of both operands");
+    static_assert(kBN <= kThreads, "one thread per bias value");
+    static_assert(kWaves * kLoadRows % 16 == 0, "a lane's placement is the same in all its pieces");
+    static_assert(Slots >= 2 && (Slots - 2) * kLoads <= 63, "vmcnt");
+    static_assert(kBiasOffset >= kWaves * kStagingBytes, "the ring holds every wavefront's staging");
+    static_assert(kLdsBytes <= 160 * 1024, "LDS");
+
+    __device__ __forceinline__ static int place(int row, int chunk) { return chunk ^ ((row >> 1) & 7); }
+};
+
+/// The epilogue's parts as in gemm_dma_kernel (alpha is always multiplied in:
+/// 1 * x is x, bit for bit). Batch entry @p first_entry + blockIdx.y; with
+/// args.rows_per_entry > 0 the rows are entries run as one problem. Without
+/// @p vector_c C's rows are not 16-byte aligned or N is no multiple of 8, and
+/// its elements are read and written one by one.
+template <typename S, bool kBias, bool kGelu, bool kAccumulate, bool kAddend = false>
+__global__ __launch_bounds__(S::kThreads) void gemm_ring_kernel(const std::uint16_t* __restrict__ a,
+                                                                const std::uint16_t* __restrict__ b,
+                                                                const float* __restrict__ bias,
+                                                                std::uint16_t* c, GemmArgs args,
+                                                                TileMap map, bool vector_c, int first_entry) {
+    constexpr int BM = S::kBM;
+    constexpr int BN = S::kBN;
+    constexpr int TM = S::kTM;
+    constexpr int TN = S::kTN;
+    constexpr int BK = S::kBK;
+    const Offsets entry = entry_offsets(args, first_entry + static_cast<int>(blockIdx.y));
+    a += entry.a;
+    b += entry.b;
+    c += entry.c;
+    extern __shared__ Vec16 lds_vectors[];
+    unsigned char* const lds = reinterpret_cast<unsigned char*>(lds_vectors);
+    const unsigned int lds_base = __builtin_amdgcn_readfirstlane(lds_address(lds));
+
+    const int lane = lane_id();
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
+    const int wave_m = wave / S::kWN;
+    const int wave_n = wave % S::kWN;
+
+    const int tiles_n = (args.n + BN - 1) / BN;
+    int tile_m = static_cast<int>(blockIdx.x) / tiles_n;
+    int tile_n = static_cast<int>(blockIdx.x) % tiles_n;
+    if (map.px > 0) {
+        const int tiles_m = (args.m + BM - 1) / BM;
+        const int block = static_cast<int>(blockIdx.x) % 8;
+        const int index = static_cast<int>(blockIdx.x) / 8;
+        const int m_lo = split_point(tiles_m, map.px, block / map.py);
+        const int m_hi = split_point(tiles_m, map.px, block / map.py + 1);
+        const int n_lo = split_point(tiles_n, map.py, block % map.py);
+        const int n_hi = split_point(tiles_n, map.py, block % map.py + 1);
+        const int width = n_hi - n_lo;
+        if (index >= (m_hi - m_lo) * width) {
+            return; // fewer tiles than the grid allows: the whole workgroup, before any barrier
+        }
+        tile_m = m_lo + index / width;
+        tile_n = n_lo + index % width;
+    }
+    const int row0 = __builtin_amdgcn_readfirstlane(tile_m * BM);
+    const int col0 = __builtin_amdgcn_readfirstlane(tile_n * BN);
+
+    // Old C, one 16-byte piece per lane and row group, issued ahead of the
+    // stage loads (so older than they are in every wait below).
+    constexpr int kRowChunks = 4 * TN;                // 16-byte pieces of a wavefront's row
+    constexpr int kRowsPerStore = kWave / kRowChunks; // rows one store instruction covers
+    constexpr int kStores = 32 / kRowsPerStore;
+    const int store_row = lane / kRowChunks;
+    const int store_chunk = lane % kRowChunks;
+    const int store_col = col0 + wave_n * 32 * TN + 8 * store_chunk;
+    auto group_row = [&](int i, int k) {
+        return row0 + (wave_m * TM + i) * 32 + kRowsPerStore * k + store_row;
+    };
+    // Output row -> its element offset in C (in its entry when entries run as one).
+    auto c_offset = [&](int row) -> std::int64_t {
+        if (args.rows_per_entry > 0) {
+            const int index = row / args.rows_per_entry;
+            return index * args.stride_c + static_cast<std::int64_t>(row - index * args.rows_per_entry) * args.ldc;
+        }
+        return static_cast<std::int64_t>(row) * args.ldc;
+    };
+    Vec16 old_rows[kAccumulate ? TM : 1][kStores];
+    if constexpr (kAccumulate) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int k = 0; k < kStores; ++k) {
+                const int row = group_row(i, k);
+                old_rows[i][k] = Vec16{{0U, 0U, 0U, 0U}};
+                if (row < args.m && store_col < args.n) {
+                    const std::uint16_t* const from = c + c_offset(row) + store_col;
+                    old_rows[i][k] = vector_c ? load16(from) : load_chunk_scalar(from, 0, 0, 1, 0, args.n - store_col);
+                }
+            }
+    }
+    // The tile's bias into LDS (read by the epilogue, many barriers later).
+    float* const bias_slot = reinterpret_cast<float*>(lds + S::kBiasOffset);
+    if (kBias && static_cast<int>(threadIdx.x) < BN) {
+        const int col = col0 + static_cast<int>(threadIdx.x);
+        bias_slot[threadIdx.x] = col < args.n ? bias[col] : 0.F;
+    }
+
+    // -- stage loads: piece p of wavefront w holds stage rows
+    // (p kWaves + w) kLoadRows .. + kLoadRows; lane l lands in row l / kChunks,
+    // slot l % kChunks of it.
+    const int rows_a = min(args.m - row0, BM);
+    const int rows_b = min(args.n - col0, BN);
+    const sgpr4 resource_a = scalar_resource(a + static_cast<std::int64_t>(row0) * args.lda,
+                                             static_cast<unsigned int>(rows_a * args.lda * 2));
+    const sgpr4 resource_b = scalar_resource(b + static_cast<std::int64_t>(col0) * args.ldb,
+                                             static_cast<unsigned int>(rows_b * args.ldb * 2));
+    const int load_row = wave * S::kLoadRows + lane / S::kChunks;
+    const int load_k = 8 * S::place(load_row, lane % S::kChunks);
+    const unsigned int offset_a = static_cast<unsigned int>((load_row * args.lda + load_k) * 2);
+    const unsigned int offset_b = static_cast<unsigned int>((load_row * args.ldb + load_k) * 2);
+    const unsigned int step_a =
+        static_cast<unsigned int>(__builtin_amdgcn_readfirstlane(S::kWaves * S::kLoadRows * args.lda * 2));
+    const unsigned int step_b =
+        static_cast<unsigned int>(__builtin_amdgcn_readfirstlane(S::kWaves * S::kLoadRows * args.ldb * 2));
+    auto issue = [&](int k0, int slot) {
+        const bool inside = load_k + k0 < args.k;
+        const unsigned int from_a = inside ? offset_a + static_cast<unsigned int>(k0) * 2U : kOutside;
+        const unsigned int from_b = inside ? offset_b + static_cast<unsigned int>(k0) * 2U : kOutside;
+        const unsigned int m0 = lds_base + static_cast<unsigned int>(slot * S::kStageBytes + wave * 1024);
+#pragma unroll
+        for (int p = 0; p < S::kLoadsA; ++p) {
+            load_to_lds(m0 + static_cast<unsigned int>(p * S::kWaves * 1024),
+                        from_a + static_cast<unsigned int>(p) * step_a, resource_a);
+        }
+#pragma unroll
+        for (int p = 0; p < S::kLoadsB; ++p) {
+            load_to_lds(m0 + static_cast<unsigned int>(BM * S::kRowBytes + p * S::kWaves * 1024),
+                        from_b + static_cast<unsigned int>(p) * step_b, resource_b);
+        }
+    };
+
+    const unsigned int a_fragment = static_cast<unsigned int>((wave_m * 32 * TM + (lane & 31)) * S::kRowBytes);
+    const unsigned int b_fragment =
+        static_cast<unsigned int>((BM + wave_n * 32 * TN + (lane & 31)) * S::kRowBytes);
+    unsigned int fragment_column[BK / 16];
+#pragma unroll
+    for (int kb = 0; kb < BK / 16; ++kb) {
+        fragment_column[kb] = static_cast<unsigned int>(S::place(lane & 31, 2 * kb + (lane >> 5)) * 16);
+    }
+    floatx16 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                acc[i][j][r] = 0.F;
+    auto compute = [&](int slot) {
+        const unsigned char* const base = lds + slot * S::kStageBytes;
+#pragma unroll
+        for (int kb = 0; kb < BK / 16; ++kb) {
+            Vec16 fa[TM];
+            Vec16 fb[TN];
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+                fa[i] = *reinterpret_cast<const Vec16*>(base + a_fragment + i * 32 * S::kRowBytes +
+                                                        fragment_column[kb]);
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+                fb[j] = *reinterpret_cast<const Vec16*>(base + b_fragment + j * 32 * S::kRowBytes +
+                                                        fragment_column[kb]);
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+                    Mma<std::uint16_t>::run(acc[i][j], fb[j], fa[i]);
+        }
+    };
+
+    const int stages = (args.k + 127) / 128 * (128 / BK);
+#pragma unroll
+    for (int g = 0; g < S::kSlots - 1; ++g) {
+        issue(g * BK, g);
+    }
+    int slot = 0;
+    int free_slot = S::kSlots - 1;
+    for (int g = 0; g < stages; ++g) {
+        // Stage g landed (each wavefront waits for its own pieces) and every
+        // wavefront is done reading stage g - 1, whose slot is refilled.
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"((S::kSlots - 2) * S::kLoads) : "memory");
+        issue((g + S::kSlots - 1) * BK, free_slot);
+        compute(slot);
+        free_slot = slot;
+        slot = slot + 1 == S::kSlots ? 0 : slot + 1;
+    }
+    // No load in flight and no wavefront reading: the ring becomes staging.
+    stage_barrier(true);
+
+    unsigned char* const staging = lds + wave * S::kStagingBytes;
+    auto staged = [&](int r, int chunk) {
+        return staging + r * (64 * TN) + ((chunk ^ ((r >> (TN == 2 ? 1 : 2)) & (kRowChunks - 1))) * 16);
+    };
+    const int r = lane & 31;
+    static_for<TM>([&](auto tile_i) {
+        constexpr int i = decltype(tile_i)::value;
+        if constexpr (kAccumulate) {
+#pragma unroll
+            for (int k = 0; k < kStores; ++k) {
+                *reinterpret_cast<Vec16*>(staged(kRowsPerStore * k + store_row, store_chunk)) = old_rows[i][k];
+            }
+        }
+        const int row = row0 + (wave_m * TM + i) * 32 + r;
+        Vec16 addend_runs[kAddend ? TN * 4 : 1];
+        if constexpr (kAddend) {
+            const int local = row >= args.m ? 0 : args.rows_per_entry > 0 ? row % args.rows_per_entry : row;
+            const float* const addend_row = args.addend + static_cast<std::int64_t>(local) * args.ld_addend;
+            static_for<TN * 4>([&](auto run) {
+                constexpr int q = decltype(run)::value;
+                const int col = col0 + wave_n * 32 * TN + 32 * (q / 4) + Mma<std::uint16_t>::column(lane, q % 4);
+                addend_runs[q] = row < args.m && col < args.n ? load16(addend_row + col) : Vec16{{0U, 0U, 0U, 0U}};
+            });
+        }
+        static_for<TN * 4>([&](auto run) {
+            constexpr int j = decltype(run)::value / 4;
+            constexpr int q = decltype(run)::value % 4;
+            uint2* const at = reinterpret_cast<uint2*>(staged(r, 4 * j + q) + 8 * (lane >> 5));
+            Vec16 bias_run{{0U, 0U, 0U, 0U}};
+            if constexpr (kBias) {
+                bias_run = load16(bias_slot + wave_n * 32 * TN + 32 * j + Mma<std::uint16_t>::column(lane, q));
+            }
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+#pragma clang fp contract(off)
+                float x = args.alpha * acc[i][j][4 * q + e];
+                if constexpr (kBias) {
+                    x += __uint_as_float(bias_run.w[e]);
+                }
+                if constexpr (kAddend) {
+                    x += __uint_as_float(addend_runs[4 * j + q].w[e]);
+                }
+                v[e] = kGelu ? gelu(x) : x;
+            }
+            if constexpr (kAccumulate) {
+                const uint2 old = *at;
+                v[0] = add_unfused(bf16_to_float(static_cast<std::uint16_t>(old.x & 0xFFFFU)), v[0]);
+                v[1] = add_unfused(bf16_to_float(static_cast<std::uint16_t>(old.x >> 16)), v[1]);
+                v[2] = add_unfused(bf16_to_float(static_cast<std::uint16_t>(old.y & 0xFFFFU)), v[2]);
+                v[3] = add_unfused(bf16_to_float(static_cast<std::uint16_t>(old.y >> 16)), v[3]);
+            }
+            *at = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+        });
+#pragma unroll
+        for (int k = 0; k < kStores; ++k) {
+            const int out_row = group_row(i, k);
+            const Vec16 v = *reinterpret_cast<const Vec16*>(staged(kRowsPerStore * k + store_row, store_chunk));
+            if (out_row < args.m && store_col < args.n) {
+                std::uint16_t* const to = c + c_offset(out_row) + store_col;
+                if (vector_c) {
+                    store16(to, v);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        if (store_col + e < args.n) {
+                            Elem<std::uint16_t>::store_bits(to + e, v, e);
+                        }
+                    }
+                }
+            }
+        }
+    });
+}
+
+} // namespace cuvit::detail::gemm

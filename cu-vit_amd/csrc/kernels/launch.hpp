@@ -117,6 +117,14 @@ hipError_t gemm_f32(const float* a, const float* b, const float* bias, float* c,
 hipError_t gemm_bf16(const std::uint16_t* a, const std::uint16_t* b, const float* bias,
                      std::uint16_t* c, const GemmArgs& args, hipStream_t stream);
 
+/// gemm_ring.hip: the bf16 LDS-ring kernel on one of its tiles, for a problem
+/// gemm.hip found to fit it. px x py is the tile grid's split over the XCDs
+/// (0: none); @p vector_c tells that C may be stored in 16-byte pieces.
+enum class RingTile { k64x64, k128x64, k128x128, k128x128Deep };
+hipError_t gemm_ring_bf16(RingTile tile, const std::uint16_t* a, const std::uint16_t* b,
+                          const float* bias, std::uint16_t* c, const GemmArgs& args, int px, int py,
+                          bool vector_c, hipStream_t stream);
+
 /// Fused softmax(Q.K^T / sqrt(head_dim)).V per (image, head) from the packed
 /// [images, tokens, 3, heads, head_dim] projection into [images, tokens,
 /// heads, head_dim]; bitwise equal to the GEMM -> softmax -> GEMM sequence.
