@@ -244,11 +244,182 @@ __global__ __launch_bounds__(Waves * kWave) void attention_kernel(const float* _
     }
 }
 
+constexpr int kSplitWaves = 4;
+
+/// The same attention with a query tile's work split over four wavefronts: wavefront w computes the logits of key tiles w, w + 4, ... and
+/// the 16 context columns 16 w .. + 15, so that no wavefront's chain is longer
+/// than about a quarter of a query tile's MFMAs. K's and V's fragments go from
+/// global memory straight into the wavefronts' registers, all loads in flight
+/// at once (each is used by one wavefront only); the row maxima and then the
+/// exponentials pass through LDS, in the layout in which every lane needs them
+/// back. Every output is computed by attention_kernel's operations in its
+/// order, so the bits are the same.
+template <int KT>
+__global__ __launch_bounds__(kSplitWaves * kWave) void attention_split_kernel(
+    const float* __restrict__ qkv, float* __restrict__ context, int heads, int tokens, float scale) {
+    static_assert(kSplitWaves * 16 == kHeadDim, "one wavefront per 16 context columns");
+    constexpr int KW = (KT + kSplitWaves - 1) / kSplitWaves; // key tiles per wavefront
+    __shared__ floatx4 weights[KT][kWave];
+    __shared__ float maxima[kSplitWaves][kWave];
+
+    const int lane = lane_id();
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
+    const int row_in_tile = lane & 15;
+    const int group = lane >> 4;
+
+    const int pair = blockIdx.y;
+    const int image = pair / heads;
+    const int head = pair - image * heads;
+    const int embed = heads * kHeadDim;
+    const std::int64_t qkv_row = 3 * static_cast<std::int64_t>(embed);
+    const float* const q_base = qkv + static_cast<std::int64_t>(image) * tokens * qkv_row + head * kHeadDim;
+    const auto resource = gemm::buffer_resource(q_base);
+    const unsigned int row_bytes = static_cast<unsigned int>(qkv_row * 4);
+    const int q0 = static_cast<int>(blockIdx.x) * 16;
+
+    // Q: row q0 + l % 16 (clamped), chunk l / 16 of each k-block; K: the same
+    // of this wavefront's key tiles (rows past the tokens read as zero); V: keys 16 jt + 4 (l / 16) + e, column 16 wave + l % 16.
+    Vec16 qf[kHeadDim / 16];
+    const int q_row = min(q0 + row_in_tile, tokens - 1);
+#pragma unroll
+    for (int kb = 0; kb < kHeadDim / 16; ++kb) {
+        qf[kb] = gemm::buffer_load16(
+            resource, static_cast<unsigned int>(q_row) * row_bytes + 64U * kb + 16U * static_cast<unsigned int>(group));
+    }
+    Vec16 kf[KW][kHeadDim / 16];
+#pragma unroll
+    for (int i = 0; i < KW; ++i) {
+        const int key = 16 * (wave + kSplitWaves * i) + row_in_tile;
+        const unsigned int from = key < tokens ? static_cast<unsigned int>(key) * row_bytes + 4U * embed +
+                                                     16U * static_cast<unsigned int>(group)
+                                               : gemm::kOutside;
+#pragma unroll
+        for (int kb = 0; kb < kHeadDim / 16; ++kb) {
+            kf[i][kb] = gemm::buffer_load16(resource, from + 64U * kb);
+        }
+    }
+    float vf[KT][4];
+#pragma unroll
+    for (int jt = 0; jt < KT; ++jt) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int key = 16 * jt + 4 * group + e;
+            const unsigned int from = static_cast<unsigned int>(key) * row_bytes + 8U * embed +
+                                      4U * static_cast<unsigned int>(16 * wave + row_in_tile);
+            vf[jt][e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                resource, jt < KT - 1 || key < tokens ? from : gemm::kOutside, 0, 0));
+        }
+    }
+
+    // Logits of this wavefront's key tiles, alpha * sum rounded on its own,
+    // and the row maxima over the valid keys.
+    floatx4 s[KW];
+#pragma unroll
+    for (int i = 0; i < KW; ++i) {
+#pragma unroll
+        for (int kb = 0; kb < kHeadDim / 16; ++kb) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                s[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                    __uint_as_float(kf[i][kb].w[e]), __uint_as_float(qf[kb].w[e]),
+                    kb == 0 && e == 0 ? floatx4{0.F, 0.F, 0.F, 0.F} : s[i], 0, 0, 0);
+            }
+        }
+    }
+    const auto larger = [](float a, float b) { return fmaxf(a, b); };
+    float maximum = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < KW; ++i) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+#pragma clang fp contract(off)
+            s[i][r] = scale * s[i][r];
+            if (16 * (wave + kSplitWaves * i) + 4 * group + r < tokens) {
+                maximum = fmaxf(maximum, s[i][r]);
+            }
+        }
+    }
+    maxima[wave][lane] = combine_rows<32>(combine_rows<16>(maximum, larger), larger);
+    __syncthreads();
+
+    // Exponentials of this wavefront's tiles; keys past the tokens become
+    // exact zeros.
+    maximum = fmaxf(fmaxf(maxima[0][lane], maxima[1][lane]),
+                    fmaxf(maxima[2][lane], maxima[3][lane]));
+#pragma unroll
+    for (int i = 0; i < KW; ++i) {
+        const int jt = wave + kSplitWaves * i;
+        floatx4 e;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float value = __builtin_amdgcn_exp2f((s[i][r] - maximum) * kLog2e);
+            e[r] = 16 * jt + 4 * group + r < tokens ? value : 0.F;
+        }
+        if (jt < KT) {
+            weights[jt][lane] = e;
+        }
+    }
+    __syncthreads();
+
+    // The softmax's sum in its order (see attention_kernel), the weights, and
+    // weights.V for this wavefront's columns.
+    floatx4 out;
+    floatx4 w[KT];
+    float partial[4] = {0.F, 0.F, 0.F, 0.F};
+#pragma unroll
+    for (int jt = 0; jt < KT; ++jt) {
+        w[jt] = weights[jt][lane];
+    }
+#pragma unroll
+    for (int jt = 0; jt < KT; ++jt) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            partial[r] += w[jt][r];
+        }
+    }
+    const float quad = (partial[0] + partial[1]) + (partial[2] + partial[3]);
+    const auto add = [](float a, float b) { return a + b; };
+    const float inverse = 1.0F / combine_rows<32>(combine_rows<16>(quad, add), add);
+#pragma unroll
+    for (int jt = 0; jt < KT; ++jt) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            w[jt][r] *= inverse;
+        }
+    }
+#pragma unroll
+    for (int jt = 0; jt < KT; ++jt) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            out = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                vf[jt][e], w[jt][e], jt == 0 && e == 0 ? floatx4{0.F, 0.F, 0.F, 0.F} : out, 0, 0, 0);
+        }
+    }
+    const int row = q0 + row_in_tile;
+    if (row < tokens) {
+        *reinterpret_cast<floatx4*>(context + (static_cast<std::int64_t>(image) * tokens + row) * embed +
+                                    head * kHeadDim + 16 * wave + 4 * group) = out;
+    }
+}
+
 constexpr int kWaves = 8;
 
 template <int KT>
 hipError_t launch(const float* qkv, float* context, int images, int heads, int tokens,
                   hipStream_t stream) {
+    // One query tile per workgroup while that makes at most three workgroups
+    // per compute unit (fewer of few key tiles, whose chains are short either
+    // way). Measured at 197 tokens, against the whole tiles below: 3 pairs 17.5
+    // -> 6.7 us, 24 17.6 -> 10.1, 48 18.4 -> 14.7, 96 pairs (beyond the line)
+    // 18.8 against 21.0; at 50 tokens 12 pairs 5.2 -> 3.5, 192 5.4 against 6.2.
+    const std::int64_t split_groups = static_cast<std::int64_t>(images) * heads * KT;
+    if (split_groups <= compute_units() * (KT < 8 ? 3.0 / 8.0 * KT : 3.0)) {
+        const dim3 split_grid(KT, static_cast<unsigned int>(images * heads));
+        const float split_scale = 1.0F / std::sqrt(static_cast<float>(kHeadDim));
+        attention_split_kernel<KT><<<split_grid, kSplitWaves * kWave, 0, stream>>>(qkv, context, heads, tokens,
+                                                                                  split_scale);
+        return hipGetLastError();
+    }
     constexpr std::size_t kLds = 2 * static_cast<std::size_t>(KT) * 16 * kPitch * sizeof(float);
     auto kernel = attention_kernel<KT, kWaves>;
     static std::atomic<std::uint64_t> opted_in{0};
