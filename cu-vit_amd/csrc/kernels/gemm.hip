@@ -1,10 +1,11 @@
 // Host dispatch of the batched GEMM. The kernels, all measured on MI355X at
 // the ViT shapes and picked in this order:
 //   fp32 (16 x 16 MFMA): the resident-panel kernel (gemm_panel.hpp) for
-//        tall products with B as [N, K] and K of 192 or 768 (the ViT-Tiny
-//        linear layers and patch embedding); else the tiled kernel
-//        (gemm_kernel.hpp), 32 x 32 tiles, 64 x 64 once a problem has work
-//        for more than 32 small tiles per compute unit.
+//        tall products with B as [N, K] and K of 192, or 768 into few columns
+//        (the ViT-Tiny linear layers and patch embedding); the ring kernel
+//        (gemm_ring.hpp) for the others with B as [N, K] and 16-byte rows; else
+//        the tiled kernel (gemm_kernel.hpp), 32 x 32 tiles, 64 x 64 once a
+//        problem has work for more than 32 small tiles per compute unit.
 //   bf16 (32 x 32 MFMA): B as [N, K] with 16-byte rows runs on direct-to-LDS
 //        loads, in the persistent kernel (gemm_dma.hpp, up to 320 x 256 tiles)
 //        where its tiles fill the chip and in the ring kernel (gemm_ring.hpp,
@@ -238,6 +239,32 @@ hipError_t launch_panel(const float* a, const float* b, const float* bias, float
     return bias != nullptr ? with_gelu(std::true_type{}) : with_gelu(std::false_type{});
 }
 
+/// The fp32 ring kernel's tile for a problem, by relative times of a CU's row
+/// of tiles fitted to MI355X at K = 768 (us: 32 x 32 3.8, 64 x 32 6.9, 64 x 64
+/// 13.7 each, more for a tile alone on its CU; these are MFMA-bound, so larger
+/// tiles gain little and lose it to a last row of tiles that is not full).
+/// Three stages for 32 x 32 tiles alone on a CU (197 x 192 x 768: 8.4 -> 7.6).
+RingTileF32 choose_ring_f32(const GemmArgs& args) {
+    constexpr RingTileF32 kTiles[3] = {RingTileF32::k32x32, RingTileF32::k64x32, RingTileF32::k64x64};
+    constexpr int kHeights[3] = {32, 64, 64};
+    constexpr int kWidths[3] = {32, 32, 64};
+    constexpr double kCost[3] = {1.0, 1.8, 3.56};
+    constexpr double kAlone[3] = {1.5, 2.45, 4.0};
+    const std::int64_t units = compute_units();
+    RingTileF32 best = RingTileF32::k32x32;
+    double best_cost = 0.0;
+    for (int i = 0; i < 3; ++i) {
+        const std::int64_t tiles = tile_count(args, kHeights[i], kWidths[i]);
+        const double cost =
+            tiles <= units ? kAlone[i] : static_cast<double>((tiles + units - 1) / units) * kCost[i];
+        if (i == 0 || cost < best_cost) {
+            best = i == 0 && tiles <= units ? RingTileF32::k32x32Deep : kTiles[i];
+            best_cost = cost;
+        }
+    }
+    return best;
+}
+
 hipError_t gemm_f32(const float* a, const float* b, const float* bias, float* c,
                     const GemmArgs& args, hipStream_t stream) {
     // Tall single products with B as [N, K] (the model's linear layers): the
@@ -259,9 +286,21 @@ hipError_t gemm_f32(const float* a, const float* b, const float* bias, float* c,
                panel != hipErrorNotSupported) {
         return panel;
     }
-    if (const hipError_t panel = launch_panel<48, 32, 2, 4, 12>(a, b, bias, c, whole, stream);
-        panel != hipErrorNotSupported) {
-        return panel;
+    // K = 768 into wide outputs is the ring kernel's (3152 x 2304 114 -> 107 us,
+    // 3152 x 768 40 -> 37); into 192 columns the panels stay ahead (6304 rows:
+    // 23.1 against 25.0 us).
+    if (whole.n < 512) {
+        if (const hipError_t panel = launch_panel<48, 32, 2, 4, 12>(a, b, bias, c, whole, stream);
+            panel != hipErrorNotSupported) {
+            return panel;
+        }
+    }
+    const bool split = whole.inner > 0;
+    if (whole.transposed && vector_operand(a, whole.lda, whole.k, whole.stride_a, whole.outer_stride_a, split) &&
+        vector_operand(b, whole.ldb, whole.k, whole.stride_b, whole.outer_stride_b, split) &&
+        static_cast<std::int64_t>(64) * whole.lda * 4 < gemm::kMaxSpan &&
+        static_cast<std::int64_t>(64) * whole.ldb * 4 < gemm::kMaxSpan) {
+        return gemm_ring_f32(choose_ring_f32(whole), a, b, bias, c, whole, vector_output(c, whole), stream);
     }
     if (tile_count(args, 32, 32) > static_cast<std::int64_t>(compute_units()) * 32) {
         return pick_flags<float, 2, 2, 2, 2, 32>(a, b, bias, c, args, stream);
@@ -313,6 +352,9 @@ gemm::TileMap balanced_map(const GemmArgs& args, int bm, int bn, int turns, int*
 /// 4.2). The GELU weighs more where fewer wavefronts share a SIMD.
 constexpr double kRingCost[3] = {1.0, 1.65, 2.9};
 constexpr double kRingCostGelu[3] = {1.1, 1.85, 3.3};
+/// A tile alone on its CU, with nothing beside it to cover its waits (128 x 64:
+/// 4616 x 384 x 384 5.7 us against 5.3 with two 64 x 64 tiles per CU).
+constexpr double kRingCostAlone[3] = {1.3, 2.1, 3.0};
 constexpr double kDmaRow = 0.035;
 constexpr double kDmaRowGelu = 0.043;
 
@@ -323,10 +365,12 @@ struct RingChoice {
     double cost;
 };
 
-/// The ring kernel's cheapest tile for a problem. A 128 x 128 tile that is
-/// alone on its CU takes three stages once K is long (768 x 3072 on 4616 rows:
-/// 31 -> 27 us; two tiles per CU with two stages each beat one at a time with
-/// three, 40 against 51 us on 6304 rows).
+/// The ring kernel's cheapest tile for a problem. Where a CU has few tiles and
+/// K is long, the tile's own loads are all there is to hide behind, and it
+/// takes three stages: 64 x 64 tiles up to two per CU (768 x 3072 on 788 rows
+/// 22.0 -> 14.5 us, on 1576 rows 24.0 -> 19.3), 128 x 128 alone on a CU (768 x
+/// 3072 on 4616 rows 31 -> 27 us; two with two stages each beat one at a time
+/// with three, 40 against 51 us on 6304 rows).
 RingChoice choose_ring(const GemmArgs& args) {
     constexpr RingTile kTiles[3] = {RingTile::k64x64, RingTile::k128x64, RingTile::k128x128};
     constexpr int kHeights[3] = {64, 128, 128};
@@ -335,11 +379,14 @@ RingChoice choose_ring(const GemmArgs& args) {
     RingChoice best{RingTile::k64x64, 64, 64, 0.0};
     for (int i = 0; i < 3; ++i) {
         const std::int64_t tiles = tile_count(args, kHeights[i], kWidths[i]);
-        const double cost = static_cast<double>((tiles + units - 1) / units) *
-                            (args.gelu ? kRingCostGelu[i] : kRingCost[i]);
+        const double cost = tiles <= units ? kRingCostAlone[i]
+                                           : static_cast<double>((tiles + units - 1) / units) *
+                                                 (args.gelu ? kRingCostGelu[i] : kRingCost[i]);
         if (i == 0 || cost < best.cost) {
             best = RingChoice{kTiles[i], kHeights[i], kWidths[i], cost};
-            if (i == 2 && tiles <= units && args.k >= 1024) {
+            if (i == 0 && tiles <= 2 * units && args.k >= 1024) {
+                best.tile = RingTile::k64x64Deep;
+            } else if (i == 2 && tiles <= units && args.k >= 1024) {
                 best.tile = RingTile::k128x128Deep;
             }
         }

@@ -1,5 +1,5 @@
-// Launch of the LDS-ring bf16 GEMM (gemm_ring.hpp): its instances, one
-// translation unit of their own.
+// Launch of the LDS-ring GEMM (gemm_ring.hpp): its instances, one translation
+// unit of their own.
 #include "gemm_ring.hpp"
 
 namespace cuvit::detail {
@@ -7,9 +7,12 @@ namespace {
 
 constexpr int kMaxGridY = 65535;
 
-template <typename S>
-hipError_t launch(const std::uint16_t* a, const std::uint16_t* b, const float* bias, std::uint16_t* c,
-                  const GemmArgs& args, const gemm::TileMap& map, bool vector_c, hipStream_t stream) {
+/// Launches @p kernel over the tile grid, one workgroup per tile (per slot of
+/// the largest XCD block with a split) and batch entry.
+template <typename S, typename Kernel, typename T>
+hipError_t run_tiles(Kernel kernel, std::atomic<std::uint64_t>& opted_in, const T* a, const T* b,
+                     const float* bias, T* c, const GemmArgs& args, const gemm::TileMap& map, bool vector_c,
+                     hipStream_t stream) {
     const std::int64_t tiles_m = (args.m + S::kBM - 1) / S::kBM;
     const std::int64_t tiles_n = (args.n + S::kBN - 1) / S::kBN;
     const std::int64_t tiles = map.px > 0 ? 8 * ((tiles_m + map.px - 1) / map.px) *
@@ -18,23 +21,28 @@ hipError_t launch(const std::uint16_t* a, const std::uint16_t* b, const float* b
     if (tiles > 0x7FFFFFFF) {
         return hipErrorInvalidConfiguration;
     }
+    if (const hipError_t opted = allow_lds(reinterpret_cast<const void*>(kernel), S::kLdsBytes, opted_in);
+        opted != hipSuccess) {
+        return opted;
+    }
+    // A grid's y extent is limited: more entries than that take several launches.
+    for (int first = 0; first < args.count; first += kMaxGridY) {
+        const int entries = args.count - first < kMaxGridY ? args.count - first : kMaxGridY;
+        const dim3 grid(static_cast<unsigned int>(tiles), static_cast<unsigned int>(entries));
+        kernel<<<grid, S::kThreads, S::kLdsBytes, stream>>>(a, b, bias, c, args, map, vector_c, first);
+        if (const hipError_t launched = hipGetLastError(); launched != hipSuccess) {
+            return launched;
+        }
+    }
+    return hipSuccess;
+}
+
+template <typename S>
+hipError_t launch(const std::uint16_t* a, const std::uint16_t* b, const float* bias, std::uint16_t* c,
+                  const GemmArgs& args, const gemm::TileMap& map, bool vector_c, hipStream_t stream) {
     auto run = [&](auto kernel) -> hipError_t {
         static std::atomic<std::uint64_t> opted_in{0};
-        if (const hipError_t opted =
-                allow_lds(reinterpret_cast<const void*>(kernel), S::kLdsBytes, opted_in);
-            opted != hipSuccess) {
-            return opted;
-        }
-        // A grid's y extent is limited: more entries than that take several launches.
-        for (int first = 0; first < args.count; first += kMaxGridY) {
-            const int entries = args.count - first < kMaxGridY ? args.count - first : kMaxGridY;
-            const dim3 grid(static_cast<unsigned int>(tiles), static_cast<unsigned int>(entries));
-            kernel<<<grid, S::kThreads, S::kLdsBytes, stream>>>(a, b, bias, c, args, map, vector_c, first);
-            if (const hipError_t launched = hipGetLastError(); launched != hipSuccess) {
-                return launched;
-            }
-        }
-        return hipSuccess;
+        return run_tiles<S>(kernel, opted_in, a, b, bias, c, args, map, vector_c, stream);
     };
     if (args.addend != nullptr) {
         return run(gemm::gemm_ring_kernel<S, true, false, false, true>);
@@ -57,11 +65,32 @@ hipError_t gemm_ring_bf16(RingTile tile, const std::uint16_t* a, const std::uint
                           const float* bias, std::uint16_t* c, const GemmArgs& args, int px, int py,
                           bool vector_c, hipStream_t stream) {
     const gemm::TileMap map{px, py};
+    using T = std::uint16_t;
     switch (tile) {
-    case RingTile::k64x64: return launch<gemm::RingShape<2, 2, 1, 1, 2>>(a, b, bias, c, args, map, vector_c, stream);
-    case RingTile::k128x64: return launch<gemm::RingShape<2, 2, 2, 1, 2>>(a, b, bias, c, args, map, vector_c, stream);
-    case RingTile::k128x128: return launch<gemm::RingShape<4, 2, 1, 2, 2>>(a, b, bias, c, args, map, vector_c, stream);
-    default: return launch<gemm::RingShape<4, 2, 1, 2, 3>>(a, b, bias, c, args, map, vector_c, stream);
+    case RingTile::k64x64: return launch<gemm::RingShape<T, 2, 2, 1, 1, 2>>(a, b, bias, c, args, map, vector_c, stream);
+    case RingTile::k64x64Deep:
+        return launch<gemm::RingShape<T, 2, 2, 1, 1, 3, true>>(a, b, bias, c, args, map, vector_c, stream);
+    case RingTile::k128x64:
+        return launch<gemm::RingShape<T, 4, 2, 1, 1, 2, true>>(a, b, bias, c, args, map, vector_c, stream);
+    case RingTile::k128x128:
+        return launch<gemm::RingShape<T, 4, 2, 1, 2, 2>>(a, b, bias, c, args, map, vector_c, stream);
+    default: return launch<gemm::RingShape<T, 4, 2, 1, 2, 3>>(a, b, bias, c, args, map, vector_c, stream);
+    }
+}
+
+hipError_t gemm_ring_f32(RingTileF32 tile, const float* a, const float* b, const float* bias, float* c,
+                         const GemmArgs& args, bool vector_c, hipStream_t stream) {
+    auto launch_f32 = [&](auto shape) -> hipError_t {
+        using S = decltype(shape);
+        static std::atomic<std::uint64_t> opted_in{0};
+        return run_tiles<S>(gemm::gemm_ring_f32_kernel<S>, opted_in, a, b, bias, c, args, gemm::TileMap{0, 0},
+                            vector_c, stream);
+    };
+    switch (tile) {
+    case RingTileF32::k32x32: return launch_f32(gemm::RingShape<float, 2, 2, 1, 1, 2, true>{});
+    case RingTileF32::k32x32Deep: return launch_f32(gemm::RingShape<float, 2, 2, 1, 1, 3, true>{});
+    case RingTileF32::k64x32: return launch_f32(gemm::RingShape<float, 2, 2, 2, 1, 2, true>{});
+    default: return launch_f32(gemm::RingShape<float, 2, 2, 2, 2, 2, true>{});
     }
 }
 

@@ -1,5 +1,6 @@
-// The bf16 GEMM for products with B given as [N, K] that the persistent kernel
-// (gemm_dma.hpp) has too few tiles or no whole 256-column tiles for: one tile
+// The GEMM for products with B given as [N, K] that the persistent bf16 kernel
+// (gemm_dma.hpp) and the fp32 panels (gemm_panel.hpp) do not take: in bf16 those
+// with too few tiles for the persistent kernel or no whole 256-column tiles. One tile
 // per workgroup, operands brought into an LDS ring by direct-to-LDS loads.
 //
 // What bounds these. Tiles are few and K is short (6 to 48 stages of 64), so
@@ -14,16 +15,24 @@
 // each tile, except for a tile alone on its CU with a long K, which has
 // nothing but its own loads to hide behind and takes three (4616 x 768 x
 // 3072: 31 -> 27 us). Eight wavefronts of 32 x 64 beat four of 64 x 64 on the
-// 128 x 128 tile by a few percent (3152 x 2304 x 768: 16.1 against 16.2 us).
+// 128 x 128 tile (4616 x 2304 x 768: 24.7 against 25.7 us).
 // Before (gemm_kernel.hpp and gemm_dma.hpp) and now, bf16, us:
 //   4616 x 1152 x 384          18.0 ->  9.9    197 x 768 x 768 (+=)    8.6 -> 5.2
 //   4616 x 384 x 1536 (+=)     17.5 -> 10.6    1576 x 2304 x 768      17.4 -> 9.4
 //   4616 x 1536 x 384 (GELU)   18.2 -> 13.8    3152 x 2304 x 768      19.2 -> 16.1
 //   6304 x 192 x 768 (+=)      11.4 ->  6.5    12608 x 1152 x 384     38.2 -> 19.6
+// and fp32 (MFMA-bound from a few tiles per CU on):
+//   197 x 192 x 768 (+=)        8.5 ->  7.6    1576 x 2304 x 768      60.3 -> 54.7
+//   788 x 3072 x 768 (GELU)    45.6 -> 36.0    3152 x 768 x 3072      158  -> 126
 //
-// Stages are 64 deep, rows of 128 bytes: chunk c of row r sits in 16-byte slot
-// c ^ ((r >> 1) & 7) of its row, conflict-free for the fragment reads (lane l:
-// row l % 32, chunk 2 kb + l / 32). One buffer_load_dwordx4 ... lds moves
+// With kAhead a stage's fragments are read during the stage before, and its
+// loads go out between two k-blocks' MFMAs: a wavefront waits about 85 cycles
+// to issue one, which its MFMAs in flight then cover. It pays where few
+// wavefronts share a SIMD, and costs the registers of a second set.
+//
+// Stages are rows of 128 bytes (64 bf16 or 32 fp32 of k): chunk c of row r sits in 16-byte slot
+// c ^ ((r >> 1) & 7) of its row, conflict-free for the fragment reads (bf16 lane
+// l: row l % 32, chunk 2 kb + l / 32; fp32: row l % 16, chunk 4 kb + l / 16). One buffer_load_dwordx4 ... lds moves
 // eight rows; every wavefront loads the same number of pieces of A and of B
 // for each stage and waits for its own (vmcnt, the newest kSlots - 2 stages
 // staying in flight) before the stage's barrier. Loads past the last stage go
@@ -42,19 +51,22 @@
 
 namespace cuvit::detail::gemm {
 
-/// WM x WN wavefronts of TM x TN MFMA tiles (32 x 32), Slots stages in the ring.
-template <int WM, int WN, int TM, int TN, int Slots> struct RingShape {
+/// WM x WN wavefronts of TM x TN MFMA tiles of type @p T (bf16 32 x 32, fp32
+/// 16 x 16), Slots stages in the ring.
+template <typename T, int WM, int WN, int TM, int TN, int Slots, bool Ahead = false> struct RingShape {
+    static constexpr bool kAhead = Ahead;
+    static constexpr int kEdge = Mma<T>::kEdge;
     static constexpr int kWaves = WM * WN;
     static constexpr int kThreads = kWave * kWaves;
     static constexpr int kWN = WN;
     static constexpr int kTM = TM;
     static constexpr int kTN = TN;
-    static constexpr int kBK = 64;
-    static constexpr int kBM = 32 * WM * TM;
-    static constexpr int kBN = 32 * WN * TN;
+    static constexpr int kBM = kEdge * WM * TM;
+    static constexpr int kBN = kEdge * WN * TN;
     static constexpr int kSlots = Slots;
-    static constexpr int kRowBytes = 2 * kBK;
-    static constexpr int kChunks = kBK / 8;                  // 16-byte chunks per row
+    static constexpr int kRowBytes = 128;                    // of a stage, either type
+    static constexpr int kBK = kRowBytes / sizeof(T);        // k of a stage
+    static constexpr int kChunks = kRowBytes / 16;           // 16-byte chunks per row
     static constexpr int kLoadRows = 1024 / kRowBytes;       // rows of one load instruction
     static constexpr int kLoadsA = kBM / kLoadRows / kWaves; // per wavefront and stage
     static constexpr int kLoadsB = kBN / kLoadRows / kWaves;
@@ -62,17 +74,213 @@ template <int WM, int WN, int TM, int TN, int Slots> struct RingShape {
     static constexpr int kStageBytes = (kBM + kBN) * kRowBytes;
     static constexpr int kBiasOffset = Slots * kStageBytes;
     static constexpr int kLdsBytes = kBiasOffset + kBN * 4;
-    static constexpr int kStagingBytes = 32 * TN * 64; // 32 rows of a wavefront's columns
+    static constexpr int kStagingBytes = kEdge * TN * 64; // bf16: 32 rows of a wavefront's columns
     static_assert(kBM % (kLoadRows * kWaves) == 0 && kBN % (kLoadRows * kWaves) == 0,
                   "every wavefront loads whole pieces of both operands");
     static_assert(kBN <= kThreads, "one thread per bias value");
     static_assert(kWaves * kLoadRows % 16 == 0, "a lane's placement is the same in all its pieces");
-    static_assert(Slots >= 2 && (Slots - 2) * kLoads <= 63, "vmcnt");
+    static_assert(Slots >= 2 && (Slots - 1) * kLoads <= 63, "vmcnt");
     static_assert(kBiasOffset >= kWaves * kStagingBytes, "the ring holds every wavefront's staging");
     static_assert(kLdsBytes <= 160 * 1024, "LDS");
 
     __device__ __forceinline__ static int place(int row, int chunk) { return chunk ^ ((row >> 1) & 7); }
 };
+
+/// The tile of workgroup blockIdx.x, or false where its XCD's block of the
+/// tile grid (TileMap) has fewer tiles than the grid allows.
+template <typename S>
+__device__ __forceinline__ bool ring_tile(const GemmArgs& args, const TileMap& map, int& row0, int& col0) {
+    const int tiles_n = (args.n + S::kBN - 1) / S::kBN;
+    int tile_m = static_cast<int>(blockIdx.x) / tiles_n;
+    int tile_n = static_cast<int>(blockIdx.x) % tiles_n;
+    if (map.px > 0) {
+        const int tiles_m = (args.m + S::kBM - 1) / S::kBM;
+        // px py = 8, both powers of two: the split points as shifts, since a
+        // tile has little time for five integer divisions.
+        const int block = static_cast<int>(blockIdx.x & 7U);
+        const int index = static_cast<int>(blockIdx.x >> 3);
+        const int log_m = 31 - __builtin_clz(static_cast<unsigned int>(map.px));
+        const int log_n = 3 - log_m;
+        const int part_m = block >> log_n;
+        const int part_n = block & (map.py - 1);
+        const int m_lo = tiles_m * part_m >> log_m;
+        const int m_hi = tiles_m * (part_m + 1) >> log_m;
+        const int n_lo = tiles_n * part_n >> log_n;
+        const int n_hi = tiles_n * (part_n + 1) >> log_n;
+        const int width = n_hi - n_lo;
+        if (index >= (m_hi - m_lo) * width) {
+            return false;
+        }
+        tile_m = m_lo + index / width;
+        tile_n = n_lo + index % width;
+    }
+    row0 = __builtin_amdgcn_readfirstlane(tile_m * S::kBM);
+    col0 = __builtin_amdgcn_readfirstlane(tile_n * S::kBN);
+    return true;
+}
+
+/// The stage loads of one wavefront: piece p of wavefront w holds stage rows
+/// (p kWaves + w) kLoadRows .. + kLoadRows; lane l lands in row l / kChunks,
+/// slot l % kChunks of it. Rows past the problem and k past K read as zero.
+template <typename T, typename S> struct RingLoads {
+    sgpr4 resource_a;
+    sgpr4 resource_b;
+    unsigned int offset_a;
+    unsigned int offset_b;
+    unsigned int step_a;
+    unsigned int step_b;
+    unsigned int lds_base;
+    int load_k;
+    int depth;
+
+    __device__ __forceinline__ RingLoads(const T* a, const T* b, const GemmArgs& args, int row0, int col0,
+                                         int wave, int lane, unsigned int lds) {
+        constexpr int kSize = static_cast<int>(sizeof(T));
+        const int rows_a = min(args.m - row0, S::kBM);
+        const int rows_b = min(args.n - col0, S::kBN);
+        resource_a = scalar_resource(a + static_cast<std::int64_t>(row0) * args.lda,
+                                     static_cast<unsigned int>(rows_a * args.lda * kSize));
+        resource_b = scalar_resource(b + static_cast<std::int64_t>(col0) * args.ldb,
+                                     static_cast<unsigned int>(rows_b * args.ldb * kSize));
+        const int load_row = wave * S::kLoadRows + lane / S::kChunks;
+        load_k = 16 / kSize * S::place(load_row, lane % S::kChunks);
+        offset_a = static_cast<unsigned int>((load_row * args.lda + load_k) * kSize);
+        offset_b = static_cast<unsigned int>((load_row * args.ldb + load_k) * kSize);
+        step_a = static_cast<unsigned int>(__builtin_amdgcn_readfirstlane(S::kWaves * S::kLoadRows * args.lda * kSize));
+        step_b = static_cast<unsigned int>(__builtin_amdgcn_readfirstlane(S::kWaves * S::kLoadRows * args.ldb * kSize));
+        lds_base = lds + static_cast<unsigned int>(wave * 1024);
+        depth = args.k;
+    }
+
+    /// Stage @p g into ring slot @p slot.
+    __device__ __forceinline__ void issue(int g, int slot) const {
+        const int k0 = g * S::kBK;
+        const bool inside = load_k + k0 < depth;
+        const unsigned int at = static_cast<unsigned int>(k0) * static_cast<unsigned int>(sizeof(T));
+        const unsigned int from_a = inside ? offset_a + at : kOutside;
+        const unsigned int from_b = inside ? offset_b + at : kOutside;
+        const unsigned int m0 = lds_base + static_cast<unsigned int>(slot * S::kStageBytes);
+#pragma unroll
+        for (int p = 0; p < S::kLoadsA; ++p) {
+            load_to_lds(m0 + static_cast<unsigned int>(p * S::kWaves * 1024),
+                        from_a + static_cast<unsigned int>(p) * step_a, resource_a);
+        }
+#pragma unroll
+        for (int p = 0; p < S::kLoadsB; ++p) {
+            load_to_lds(m0 + static_cast<unsigned int>(S::kBM * S::kRowBytes + p * S::kWaves * 1024),
+                        from_b + static_cast<unsigned int>(p) * step_b, resource_b);
+        }
+    }
+};
+
+/// The k loop: acc += A.B^T over @p stages stages, the ring kept kSlots - 1
+/// stages ahead. On return no load is in flight and no wavefront reads the
+/// ring.
+template <typename T, typename S>
+__device__ __forceinline__ void ring_multiply(const RingLoads<T, S>& loads, const unsigned char* lds, int wave_m,
+                                              int wave_n, int lane, int stages,
+                                              typename Mma<T>::Acc (&acc)[S::kTM][S::kTN]) {
+    constexpr int E = S::kEdge;
+    constexpr int kBlocks = S::kBK / kKBlock<T>;  // k-blocks per stage
+    constexpr int kPerBlock = kWave / E;          // 16-byte chunks of a row per k-block
+    const unsigned int a_fragment = static_cast<unsigned int>((wave_m * E * S::kTM + lane % E) * S::kRowBytes);
+    const unsigned int b_fragment =
+        static_cast<unsigned int>((S::kBM + wave_n * E * S::kTN + lane % E) * S::kRowBytes);
+    // E rows further on the placement is the same (its period is 16 rows).
+    unsigned int fragment_column[kBlocks];
+#pragma unroll
+    for (int kb = 0; kb < kBlocks; ++kb) {
+        fragment_column[kb] = static_cast<unsigned int>(S::place(lane % E, kPerBlock * kb + lane / E) * 16);
+    }
+#pragma unroll
+    for (int i = 0; i < S::kTM; ++i)
+#pragma unroll
+        for (int j = 0; j < S::kTN; ++j)
+#pragma unroll
+            for (int r = 0; r < 4 * Mma<T>::kRuns; ++r)
+                acc[i][j][r] = 0.F;
+    struct Fragments {
+        Vec16 a[kBlocks][S::kTM];
+        Vec16 b[kBlocks][S::kTN];
+    };
+    auto read_block = [&](const unsigned char* base, int kb, Vec16 (&fa)[S::kTM], Vec16 (&fb)[S::kTN]) {
+#pragma unroll
+        for (int i = 0; i < S::kTM; ++i)
+            fa[i] = load16(base + a_fragment + i * E * S::kRowBytes + fragment_column[kb]);
+#pragma unroll
+        for (int j = 0; j < S::kTN; ++j)
+            fb[j] = load16(base + b_fragment + j * E * S::kRowBytes + fragment_column[kb]);
+    };
+    auto multiply_block = [&](const Vec16 (&fa)[S::kTM], const Vec16 (&fb)[S::kTN]) {
+#pragma unroll
+        for (int i = 0; i < S::kTM; ++i)
+#pragma unroll
+            for (int j = 0; j < S::kTN; ++j)
+                Mma<T>::run(acc[i][j], fb[j], fa[i]);
+    };
+    if constexpr (S::kAhead) {
+        // A stage's fragments are read during the MFMAs of the stage before it
+        // (two register sets), so a stage costs its MFMAs and a barrier, with
+        // no LDS latency between them; its slot is free one stage earlier and
+        // the ring runs kSlots stages ahead of the registers.
+        Fragments set[2];
+        auto read = [&](Fragments& f, int slot) {
+#pragma unroll
+            for (int kb = 0; kb < kBlocks; ++kb)
+                read_block(lds + slot * S::kStageBytes, kb, f.a[kb], f.b[kb]);
+        };
+#pragma unroll
+        for (int g = 0; g < S::kSlots; ++g) {
+            loads.issue(g, g);
+        }
+        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"((S::kSlots - 1) * S::kLoads) : "memory");
+        read(set[0], 0);
+        int slot = 0;
+        auto step = [&](int g, Fragments& now, Fragments& next) {
+            // Stage g + 1 landed, and every wavefront holds stage g in registers.
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"((S::kSlots - 2) * S::kLoads) : "memory");
+            const int free_slot = slot;
+            slot = slot + 1 == S::kSlots ? 0 : slot + 1;
+            read(next, slot);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply_block(now.a[0], now.b[0]);
+            __builtin_amdgcn_sched_barrier(0);
+            loads.issue(g + S::kSlots, free_slot); // while the MFMAs before run
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int kb = 1; kb < kBlocks; ++kb)
+                multiply_block(now.a[kb], now.b[kb]);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        for (int g = 0; g < stages; g += 2) { // K's spans are whole pairs of stages
+            step(g, set[0], set[1]);
+            step(g + 1, set[1], set[0]);
+        }
+    } else {
+#pragma unroll
+        for (int g = 0; g < S::kSlots - 1; ++g) {
+            loads.issue(g, g);
+        }
+        int slot = 0;
+        int free_slot = S::kSlots - 1;
+        for (int g = 0; g < stages; ++g) {
+            // Stage g landed (each wavefront waits for its own pieces) and every
+            // wavefront is done reading stage g - 1, whose slot is refilled.
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"((S::kSlots - 2) * S::kLoads) : "memory");
+            loads.issue(g + S::kSlots - 1, free_slot);
+#pragma unroll
+            for (int kb = 0; kb < kBlocks; ++kb) {
+                Vec16 fa[S::kTM];
+                Vec16 fb[S::kTN];
+                read_block(lds + slot * S::kStageBytes, kb, fa, fb);
+                multiply_block(fa, fb);
+            }
+            free_slot = slot;
+            slot = slot + 1 == S::kSlots ? 0 : slot + 1;
+        }
+    }
+    stage_barrier(true);
+}
 
 /// The epilogue's parts as in gemm_dma_kernel (alpha is always multiplied in:
 /// 1 * x is x, bit for bit). Batch entry @p first_entry + blockIdx.y; with
@@ -89,7 +297,6 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring_kernel(const std::uint1
     constexpr int BN = S::kBN;
     constexpr int TM = S::kTM;
     constexpr int TN = S::kTN;
-    constexpr int BK = S::kBK;
     const Offsets entry = entry_offsets(args, first_entry + static_cast<int>(blockIdx.y));
     a += entry.a;
     b += entry.b;
@@ -103,26 +310,10 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring_kernel(const std::uint1
     const int wave_m = wave / S::kWN;
     const int wave_n = wave % S::kWN;
 
-    const int tiles_n = (args.n + BN - 1) / BN;
-    int tile_m = static_cast<int>(blockIdx.x) / tiles_n;
-    int tile_n = static_cast<int>(blockIdx.x) % tiles_n;
-    if (map.px > 0) {
-        const int tiles_m = (args.m + BM - 1) / BM;
-        const int block = static_cast<int>(blockIdx.x) % 8;
-        const int index = static_cast<int>(blockIdx.x) / 8;
-        const int m_lo = split_point(tiles_m, map.px, block / map.py);
-        const int m_hi = split_point(tiles_m, map.px, block / map.py + 1);
-        const int n_lo = split_point(tiles_n, map.py, block % map.py);
-        const int n_hi = split_point(tiles_n, map.py, block % map.py + 1);
-        const int width = n_hi - n_lo;
-        if (index >= (m_hi - m_lo) * width) {
-            return; // fewer tiles than the grid allows: the whole workgroup, before any barrier
-        }
-        tile_m = m_lo + index / width;
-        tile_n = n_lo + index % width;
+    int row0, col0;
+    if (!ring_tile<S>(args, map, row0, col0)) {
+        return; // the whole workgroup, before any barrier
     }
-    const int row0 = __builtin_amdgcn_readfirstlane(tile_m * BM);
-    const int col0 = __builtin_amdgcn_readfirstlane(tile_n * BN);
 
     // Old C, one 16-byte piece per lane and row group, issued ahead of the
     // stage loads (so older than they are in every wait below).
@@ -164,97 +355,11 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring_kernel(const std::uint1
         bias_slot[threadIdx.x] = col < args.n ? bias[col] : 0.F;
     }
 
-    // -- stage loads: piece p of wavefront w holds stage rows
-    // (p kWaves + w) kLoadRows .. + kLoadRows; lane l lands in row l / kChunks,
-    // slot l % kChunks of it.
-    const int rows_a = min(args.m - row0, BM);
-    const int rows_b = min(args.n - col0, BN);
-    const sgpr4 resource_a = scalar_resource(a + static_cast<std::int64_t>(row0) * args.lda,
-                                             static_cast<unsigned int>(rows_a * args.lda * 2));
-    const sgpr4 resource_b = scalar_resource(b + static_cast<std::int64_t>(col0) * args.ldb,
-                                             static_cast<unsigned int>(rows_b * args.ldb * 2));
-    const int load_row = wave * S::kLoadRows + lane / S::kChunks;
-    const int load_k = 8 * S::place(load_row, lane % S::kChunks);
-    const unsigned int offset_a = static_cast<unsigned int>((load_row * args.lda + load_k) * 2);
-    const unsigned int offset_b = static_cast<unsigned int>((load_row * args.ldb + load_k) * 2);
-    const unsigned int step_a =
-        static_cast<unsigned int>(__builtin_amdgcn_readfirstlane(S::kWaves * S::kLoadRows * args.lda * 2));
-    const unsigned int step_b =
-        static_cast<unsigned int>(__builtin_amdgcn_readfirstlane(S::kWaves * S::kLoadRows * args.ldb * 2));
-    auto issue = [&](int k0, int slot) {
-        const bool inside = load_k + k0 < args.k;
-        const unsigned int from_a = inside ? offset_a + static_cast<unsigned int>(k0) * 2U : kOutside;
-        const unsigned int from_b = inside ? offset_b + static_cast<unsigned int>(k0) * 2U : kOutside;
-        const unsigned int m0 = lds_base + static_cast<unsigned int>(slot * S::kStageBytes + wave * 1024);
-#pragma unroll
-        for (int p = 0; p < S::kLoadsA; ++p) {
-            load_to_lds(m0 + static_cast<unsigned int>(p * S::kWaves * 1024),
-                        from_a + static_cast<unsigned int>(p) * step_a, resource_a);
-        }
-#pragma unroll
-        for (int p = 0; p < S::kLoadsB; ++p) {
-            load_to_lds(m0 + static_cast<unsigned int>(BM * S::kRowBytes + p * S::kWaves * 1024),
-                        from_b + static_cast<unsigned int>(p) * step_b, resource_b);
-        }
-    };
-
-    const unsigned int a_fragment = static_cast<unsigned int>((wave_m * 32 * TM + (lane & 31)) * S::kRowBytes);
-    const unsigned int b_fragment =
-        static_cast<unsigned int>((BM + wave_n * 32 * TN + (lane & 31)) * S::kRowBytes);
-    unsigned int fragment_column[BK / 16];
-#pragma unroll
-    for (int kb = 0; kb < BK / 16; ++kb) {
-        fragment_column[kb] = static_cast<unsigned int>(S::place(lane & 31, 2 * kb + (lane >> 5)) * 16);
-    }
+    const RingLoads<std::uint16_t, S> loads(a, b, args, row0, col0, wave, lane, lds_base);
     floatx16 acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r)
-                acc[i][j][r] = 0.F;
-    auto compute = [&](int slot) {
-        const unsigned char* const base = lds + slot * S::kStageBytes;
-#pragma unroll
-        for (int kb = 0; kb < BK / 16; ++kb) {
-            Vec16 fa[TM];
-            Vec16 fb[TN];
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-                fa[i] = *reinterpret_cast<const Vec16*>(base + a_fragment + i * 32 * S::kRowBytes +
-                                                        fragment_column[kb]);
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-                fb[j] = *reinterpret_cast<const Vec16*>(base + b_fragment + j * 32 * S::kRowBytes +
-                                                        fragment_column[kb]);
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int j = 0; j < TN; ++j)
-                    Mma<std::uint16_t>::run(acc[i][j], fb[j], fa[i]);
-        }
-    };
+    ring_multiply<std::uint16_t, S>(loads, lds, wave_m, wave_n, lane, (args.k + 127) / 128 * (128 / S::kBK), acc);
 
-    const int stages = (args.k + 127) / 128 * (128 / BK);
-#pragma unroll
-    for (int g = 0; g < S::kSlots - 1; ++g) {
-        issue(g * BK, g);
-    }
-    int slot = 0;
-    int free_slot = S::kSlots - 1;
-    for (int g = 0; g < stages; ++g) {
-        // Stage g landed (each wavefront waits for its own pieces) and every
-        // wavefront is done reading stage g - 1, whose slot is refilled.
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"((S::kSlots - 2) * S::kLoads) : "memory");
-        issue((g + S::kSlots - 1) * BK, free_slot);
-        compute(slot);
-        free_slot = slot;
-        slot = slot + 1 == S::kSlots ? 0 : slot + 1;
-    }
-    // No load in flight and no wavefront reading: the ring becomes staging.
-    stage_barrier(true);
-
+    // The drained ring becomes staging.
     unsigned char* const staging = lds + wave * S::kStagingBytes;
     auto staged = [&](int r, int chunk) {
         return staging + r * (64 * TN) + ((chunk ^ ((r >> (TN == 2 ? 1 : 2)) & (kRowChunks - 1))) * 16);
@@ -328,6 +433,99 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring_kernel(const std::uint1
             }
         }
     });
+}
+
+/// The fp32 kernel: stages 32 deep (two k-blocks of 16), K rounded up to 64 as
+/// in the other fp32 kernels, results stored from the registers (a lane holds
+/// four consecutive columns; without @p vector_c, C's rows not 16-byte aligned, or
+/// where N cuts a run they go element by element).
+template <typename S>
+__global__ __launch_bounds__(S::kThreads) void gemm_ring_f32_kernel(const float* __restrict__ a,
+                                                                    const float* __restrict__ b,
+                                                                    const float* __restrict__ bias, float* c,
+                                                                    GemmArgs args, TileMap map, bool vector_c,
+                                                                    int first_entry) {
+    constexpr int TM = S::kTM;
+    constexpr int TN = S::kTN;
+    constexpr int E = S::kEdge;
+    const Offsets entry = entry_offsets(args, first_entry + static_cast<int>(blockIdx.y));
+    extern __shared__ Vec16 lds_vectors[];
+    unsigned char* const lds = reinterpret_cast<unsigned char*>(lds_vectors);
+    const unsigned int lds_base = __builtin_amdgcn_readfirstlane(lds_address(lds));
+    const int lane = lane_id();
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
+    const int wave_m = wave / S::kWN;
+    const int wave_n = wave % S::kWN;
+    int row0, col0;
+    if (!ring_tile<S>(args, map, row0, col0)) {
+        return; // the whole workgroup, before any barrier
+    }
+
+    // The epilogue's operands ahead of the stage loads: the bias of this
+    // lane's runs and old C.
+    const int first_row = row0 + wave_m * E * TM + lane % E;
+    const int first_col = col0 + wave_n * E * TN + Mma<float>::column(lane, 0);
+    float run_bias[TN][4];
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int col = first_col + E * j + r;
+            run_bias[j][r] = bias != nullptr && col < args.n ? bias[col] : 0.F;
+        }
+    auto local_row = [&](int row) { return args.rows_per_entry > 0 ? row % args.rows_per_entry : row; };
+    auto c_row = [&](int row) -> float* {
+        const std::int64_t from =
+            args.rows_per_entry > 0 ? static_cast<std::int64_t>(row / args.rows_per_entry) * args.stride_c : 0;
+        return c + entry.c + from + static_cast<std::int64_t>(local_row(row)) * args.ldc;
+    };
+    floatx4 old[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const int row = first_row + E * i;
+            const int col = first_col + E * j;
+            old[i][j] = floatx4{0.F, 0.F, 0.F, 0.F};
+            if (args.accumulate && vector_c && row < args.m && col + 3 < args.n) {
+                old[i][j] = *reinterpret_cast<const floatx4*>(c_row(row) + col);
+            }
+        }
+
+    const RingLoads<float, S> loads(a + entry.a, b + entry.b, args, row0, col0, wave, lane, lds_base);
+    floatx4 acc[TM][TN];
+    ring_multiply<float, S>(loads, lds, wave_m, wave_n, lane, (args.k + 63) / 64 * (64 / S::kBK), acc);
+
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+        const int row = first_row + E * i;
+        if (row >= args.m) {
+            continue;
+        }
+        const int local = local_row(row);
+        float* const to = c_row(row);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const int col = first_col + E * j;
+            float value[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                value[r] = col + r < args.n ? epilogue_value(acc[i][j][r], bias != nullptr, run_bias[j][r], local,
+                                                             col + r, args)
+                                            : 0.F;
+            }
+            if (vector_c && col + 3 < args.n) {
+                store4(to + col, value, args.accumulate, old[i][j]);
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    if (col + r < args.n) {
+                        to[col + r] = args.accumulate ? add_unfused(to[col + r], value[r]) : value[r];
+                    }
+                }
+            }
+        }
+    }
 }
 
 } // namespace cuvit::detail::gemm

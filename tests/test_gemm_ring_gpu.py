@@ -118,3 +118,68 @@ def test_ring_runs_a_shared_weight_batch_as_one_problem(cuvit, device):
             expected = start[i].clone()
             run(cuvit, a[i], b.t().contiguous(), bias, expected, one, False)
             assert np.array_equal(c[i].cpu().view(torch.int16).numpy(), expected.cpu().view(torch.int16).numpy())
+
+
+F32_CASES = [
+    # m, n, k, bias, gelu, accumulate, alpha, C's padding
+    (1, 8, 4, True, False, False, 1.0, 0),           # one tile, one chunk of K
+    (31, 33, 64, True, True, False, 1.0, 3),         # odd rows of C
+    (33, 65, 68, True, False, True, 1.0, 0),         # past a tile, past a span of K; element-wise C
+    (197, 192, 772, False, False, True, -0.5, 4),    # 32 x 32 tiles alone on a CU
+    (788, 384, 320, True, True, True, 1.0, 0),       # several 32 x 32 tiles a CU
+    (1003, 1152, 100, True, False, False, 1.0, 0),   # 64 x 32 or 64 x 64 tiles with tails
+    (3151, 1540, 196, False, True, False, 2.0, 0),   # 64 x 64 tiles, GELU without bias
+]
+
+
+@pytest.mark.parametrize("m,n,k,with_bias,gelu,accumulate,alpha,pad", F32_CASES)
+def test_f32_ring_equals_the_tiled_kernel(cuvit, device, m, n, k, with_bias, gelu, accumulate, alpha, pad):
+    a = normal(m + k, (m, k), 1.0, device, torch.float32)
+    b = normal(n + k, (n, k), 0.05, device, torch.float32)
+    bias = normal(n, (n,), 0.5, device, torch.float32) if with_bias else None
+    start = normal(7, (m, n + pad), 1.0, device, torch.float32) if accumulate else \
+        torch.full((m, n + pad), float("nan"), device=device)
+    results = []
+    for transposed in (True, False):
+        problem = cuvit.gemm_problem(m, n, k, cuvit.TRANSPOSED)
+        problem.alpha, problem.ldc = alpha, n + pad
+        problem.epilogue.gelu, problem.epilogue.accumulate = int(gelu), int(accumulate)
+        c = start.clone()
+        run(cuvit, a, b if transposed else b.t().contiguous(), bias, c, problem, transposed)
+        results.append(c.cpu().view(torch.int32))
+    assert torch.equal(results[0], results[1])
+    assert torch.equal(results[0][:, n:], start.cpu().view(torch.int32)[:, n:])
+
+    a64, b64 = a.cpu().double(), b.cpu().double()
+    expected = alpha * (a64 @ b64.t())
+    scale = abs(alpha) * (a64.abs() @ b64.abs().t())
+    if with_bias:
+        expected = expected + bias.cpu().double()
+    if gelu:
+        expected = torch.nn.functional.gelu(expected)
+    if accumulate:
+        expected = expected + start.cpu().double()[:, :n]
+    actual = results[0].view(torch.float32)[:, :n].double()
+    # fp32 sums of k terms (k 2^-24 of their sizes at most, GELU's slope at
+    # most 1.13), a few roundings of the result and the GELU's own 4e-7.
+    limit = 2.0 ** -22 * expected.abs() + 1.2 * (k + 4) * 2.0 ** -24 * (scale + 1.0) + 1e-6
+    assert bool(((actual - expected).abs() <= limit).all())
+
+
+@pytest.mark.parametrize("count,inner,m,n,k", [(3, 0, 33, 36, 68), (6, 3, 50, 50, 64), (4, 2, 17, 65, 64)])
+def test_f32_ring_batches(cuvit, device, count, inner, m, n, k):
+    a, b = normal(1, (count, m, k), 1.0, device, torch.float32), normal(2, (count, n, k), 0.1, device, torch.float32)
+    results = []
+    for transposed in (True, False):
+        problem = cuvit.gemm_problem(m, n, k, cuvit.TRANSPOSED)
+        problem.batch.count, problem.batch.inner = count, inner
+        problem.batch.stride_a, problem.batch.stride_b, problem.batch.stride_c = m * k, n * k, m * n
+        if inner:
+            problem.batch.outer_stride_a = inner * m * k
+            problem.batch.outer_stride_b = inner * n * k
+            problem.batch.outer_stride_c = inner * m * n
+        c = torch.full((count, m, n), float("nan"), device=device)
+        run(cuvit, a, b if transposed else b.transpose(1, 2).contiguous(), None, c, problem, transposed)
+        results.append(c.cpu().view(torch.int32))
+    assert torch.equal(results[0], results[1])
+    assert not bool(results[0].view(torch.float32).isnan().any())
