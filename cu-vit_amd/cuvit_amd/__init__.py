@@ -16,6 +16,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import sys
 from typing import Optional
 
 __all__ = [
@@ -244,6 +245,38 @@ def library() -> ctypes.CDLL:
     return _lib
 
 
+_NATIVE_FUNCTIONS = (
+    "cuvit_layer_norm_f32", "cuvit_layer_norm_bf16", "cuvit_softmax_f32", "cuvit_softmax_bf16",
+    "cuvit_extract_patches_f32", "cuvit_extract_patches_bf16", "cuvit_gemm_f32", "cuvit_gemm_bf16",
+    "cuvit_attention_f32", "cuvit_attention_bf16", "cuvit_preprocess_u8", "cuvit_vit_forward",
+)
+
+
+class _NativeCalls:
+    """The launchers' plain case in native code (csrc/binding/native.cpp): each
+    takes a launcher's arguments and returns the library's status, or -1 where
+    they are not plain GPU tensors and whole numbers that pass every check.
+    The module is loaded with the first launcher that can be given a tensor:
+    a program without torch has none. Host time of a LayerNorm call 8 -> 1 us
+    beside the launch itself."""
+
+    def __getattr__(self, name):
+        if "torch" not in sys.modules:
+            return lambda *arguments: -1
+        from . import _native
+
+        lib = library()
+        _native.bind(GemmProblem, Preprocessing,
+                     *(ctypes.cast(getattr(lib, f), _P).value for f in _NATIVE_FUNCTIONS))
+        for call in ("layer_norm", "softmax", "extract_patches", "gemm", "attention", "preprocess",
+                     "vit_forward"):
+            setattr(self, call, getattr(_native, call))
+        return getattr(_native, name)
+
+
+_native_calls = _NativeCalls()
+
+
 def check(status: int) -> None:
     """Raises the exception matching a C-ABI status."""
     if status == OK:
@@ -376,6 +409,9 @@ def gemm_problem(m: int, n: int, k: int, layout: int = NO_TRANSPOSE) -> GemmProb
 
 
 def gemm(a, b, bias, c, problem: GemmProblem, stream=None, bf16: Optional[bool] = None) -> None:
+    status = _native_calls.gemm(a, b, bias, c, problem, stream, bf16)
+    if status >= 0:
+        return check(status)
     bf16 = bf16 if bf16 is not None else _bf16(a)
     fn = library().cuvit_gemm_bf16 if bf16 else library().cuvit_gemm_f32
     pa, pb, pbias, pc = _gemm_operands(a, b, bias, c, problem, bf16)
@@ -384,6 +420,9 @@ def gemm(a, b, bias, c, problem: GemmProblem, stream=None, bf16: Optional[bool] 
 
 def layer_norm(x, gamma, beta, out, rows: int, columns: int, epsilon: float = 1.0e-6,
                stream=None, bf16: Optional[bool] = None) -> None:
+    status = _native_calls.layer_norm(x, gamma, beta, out, rows, columns, epsilon, stream, bf16)
+    if status >= 0:
+        return check(status)
     bf16 = bf16 if bf16 is not None else _bf16(x)
     fn = library().cuvit_layer_norm_bf16 if bf16 else library().cuvit_layer_norm_f32
     if _positive(rows, columns):
@@ -396,6 +435,9 @@ def layer_norm(x, gamma, beta, out, rows: int, columns: int, epsilon: float = 1.
 
 
 def softmax(x, out, rows: int, columns: int, stream=None, bf16: Optional[bool] = None) -> None:
+    status = _native_calls.softmax(x, out, rows, columns, stream, bf16)
+    if status >= 0:
+        return check(status)
     bf16 = bf16 if bf16 is not None else _bf16(x)
     fn = library().cuvit_softmax_bf16 if bf16 else library().cuvit_softmax_f32
     if _positive(rows, columns):
@@ -414,6 +456,10 @@ def gelu(x, out, count: int, stream=None, bf16: Optional[bool] = None) -> None:
 
 def extract_patches(images, patches, batch: int, channels: int, height: int, width: int,
                     patch: int, stream=None, bf16: Optional[bool] = None) -> None:
+    status = _native_calls.extract_patches(images, patches, batch, channels, height, width, patch,
+                                            stream, bf16)
+    if status >= 0:
+        return check(status)
     bf16 = bf16 if bf16 is not None else _bf16(images)
     fn = library().cuvit_extract_patches_bf16 if bf16 else library().cuvit_extract_patches_f32
     if _positive(batch, channels, height, width, patch):
@@ -488,6 +534,9 @@ def attention(qkv, context, images: int, heads: int, tokens: int, head_dim: int,
     [images, tokens, 3, heads, head_dim] projection into
     [images, tokens, heads, head_dim]; an extension replacing the reference's
     three attention launches (vit.cu:205-245) with bitwise the same result."""
+    status = _native_calls.attention(qkv, context, images, heads, tokens, head_dim, stream)
+    if status >= 0:
+        return check(status)
     bf16 = _bf16(qkv)
     fn = library().cuvit_attention_bf16 if bf16 else library().cuvit_attention_f32
     if _positive(images, heads, tokens, head_dim):
@@ -628,6 +677,10 @@ class VisionTransformer:
 
     def forward(self, images, logits, batch: int, stream=None) -> None:
         c = self.config
+        status = _native_calls.vit_forward(self._handle.value if self._handle else None, images, logits, batch,
+                                           c.channels * c.image_size * c.image_size, c.classes, stream)
+        if status >= 0:
+            return check(status)
         if _positive(batch):
             images = _operand(images, "images", "float32",
                               batch * c.channels * c.image_size * c.image_size)
@@ -706,6 +759,9 @@ def preprocess(pixels, tensor, batch: int, width: int, height: int,
     uint8 into the device tensor [batch, 3, size, size] float (the reference's
     preprocess, image.cpp:95-135, batched on the GPU)."""
     settings = settings if settings is not None else Preprocessing()
+    status = _native_calls.preprocess(pixels, tensor, batch, width, height, settings, stream)
+    if status >= 0:
+        return check(status)
     if _positive(batch, width, height, settings.size):
         pixels = _operand(pixels, "pixels", "uint8", batch * height * width * 3)
         tensor = _operand(tensor, "tensor", "float32", batch * 3 * settings.size * settings.size)
