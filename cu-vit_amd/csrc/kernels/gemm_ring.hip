@@ -79,12 +79,12 @@ hipError_t gemm_ring_bf16(RingTile tile, const std::uint16_t* a, const std::uint
 }
 
 hipError_t gemm_ring_f32(RingTileF32 tile, const float* a, const float* b, const float* bias, float* c,
-                         const GemmArgs& args, bool vector_c, hipStream_t stream) {
+                         const GemmArgs& args, hipStream_t stream) {
     auto launch_f32 = [&](auto shape) -> hipError_t {
         using S = decltype(shape);
         static std::atomic<std::uint64_t> opted_in{0};
-        return run_tiles<S>(gemm::gemm_ring_f32_kernel<S>, opted_in, a, b, bias, c, args, gemm::TileMap{0, 0},
-                            vector_c, stream);
+        return run_tiles<S>(gemm::gemm_ring_f32_kernel<S>, opted_in, a, b, bias, c, args, gemm::TileMap{0, 0}, true,
+                            stream);
     };
     switch (tile) {
     case RingTileF32::k32x32: return launch_f32(gemm::RingShape<float, 2, 2, 1, 1, 2, true>{});

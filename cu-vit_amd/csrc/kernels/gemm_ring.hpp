@@ -437,13 +437,13 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring_kernel(const std::uint1
 
 /// The fp32 kernel: stages 32 deep (two k-blocks of 16), K rounded up to 64 as
 /// in the other fp32 kernels, results stored from the registers (a lane holds
-/// four consecutive columns; without @p vector_c, C's rows not 16-byte aligned, or
-/// where N cuts a run they go element by element).
+/// four consecutive columns, one store at any alignment; a run that N cuts goes
+/// element by element).
 template <typename S>
 __global__ __launch_bounds__(S::kThreads) void gemm_ring_f32_kernel(const float* __restrict__ a,
                                                                     const float* __restrict__ b,
                                                                     const float* __restrict__ bias, float* c,
-                                                                    GemmArgs args, TileMap map, bool vector_c,
+                                                                    GemmArgs args, TileMap map, bool /* four at once: always */,
                                                                     int first_entry) {
     constexpr int TM = S::kTM;
     constexpr int TN = S::kTN;
@@ -487,8 +487,8 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring_f32_kernel(const float*
             const int row = first_row + E * i;
             const int col = first_col + E * j;
             old[i][j] = floatx4{0.F, 0.F, 0.F, 0.F};
-            if (args.accumulate && vector_c && row < args.m && col + 3 < args.n) {
-                old[i][j] = *reinterpret_cast<const floatx4*>(c_row(row) + col);
+            if (args.accumulate && row < args.m && col + 3 < args.n) {
+                old[i][j] = *reinterpret_cast<const floatx4_unaligned*>(c_row(row) + col);
             }
         }
 
@@ -514,7 +514,7 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring_f32_kernel(const float*
                                                              col + r, args)
                                             : 0.F;
             }
-            if (vector_c && col + 3 < args.n) {
+            if (col + 3 < args.n) {
                 store4(to + col, value, args.accumulate, old[i][j]);
             } else {
 #pragma unroll

@@ -124,10 +124,10 @@ enum class RingTile { k64x64, k64x64Deep, k128x64, k128x128, k128x128Deep };
 hipError_t gemm_ring_bf16(RingTile tile, const std::uint16_t* a, const std::uint16_t* b,
                           const float* bias, std::uint16_t* c, const GemmArgs& args, int px, int py,
                           bool vector_c, hipStream_t stream);
-/// Its fp32 form (@p vector_c: four results at once, as float4).
+/// Its fp32 form.
 enum class RingTileF32 { k32x32, k32x32Deep, k64x32, k64x64 };
 hipError_t gemm_ring_f32(RingTileF32 tile, const float* a, const float* b, const float* bias, float* c,
-                         const GemmArgs& args, bool vector_c, hipStream_t stream);
+                         const GemmArgs& args, hipStream_t stream);
 
 /// Fused softmax(Q.K^T / sqrt(head_dim)).V per (image, head) from the packed
 /// [images, tokens, 3, heads, head_dim] projection into [images, tokens,
