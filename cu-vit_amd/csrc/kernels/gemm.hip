@@ -248,7 +248,11 @@ hipError_t launch_panel(const float* a, const float* b, const float* bias, float
 /// of tiles fitted to MI355X at K = 768 (us: 32 x 32 3.8, 64 x 32 6.9, 64 x 64
 /// 13.7 each, more for a tile alone on its CU; these are MFMA-bound, so larger
 /// tiles gain little and lose it to a last row of tiles that is not full).
-/// Three stages for 32 x 32 tiles alone on a CU (197 x 192 x 768: 8.4 -> 7.6).
+/// Three stages for 32 x 32 tiles where few of them share a CU or K is long
+/// (1576 x 192 x 768 14.3 -> 11.3 us, 394 x 768 x 3072 47 -> 35), two elsewhere
+/// (788 x 768 x 768: 13.7 against 14.3). While 32 x 16 tiles are alone on their
+/// CUs, those, with loading wavefronts beside the computing ones (197 x 192 x
+/// 768 7.6 -> 6.6, 197 x 576 x 192 4.0 -> 3.6).
 RingTileF32 choose_ring_f32(const GemmArgs& args) {
     constexpr RingTileF32 kTiles[3] = {RingTileF32::k32x32, RingTileF32::k64x32, RingTileF32::k64x64};
     constexpr int kHeights[3] = {32, 64, 64};
@@ -256,6 +260,9 @@ RingTileF32 choose_ring_f32(const GemmArgs& args) {
     constexpr double kCost[3] = {1.0, 1.8, 3.56};
     constexpr double kAlone[3] = {1.5, 2.45, 4.0};
     const std::int64_t units = compute_units();
+    if (tile_count(args, 32, 16) <= units) {
+        return RingTileF32::k32x16Alone;
+    }
     RingTileF32 best = RingTileF32::k32x32;
     double best_cost = 0.0;
     for (int i = 0; i < 3; ++i) {
@@ -263,7 +270,8 @@ RingTileF32 choose_ring_f32(const GemmArgs& args) {
         const double cost =
             tiles <= units ? kAlone[i] : static_cast<double>((tiles + units - 1) / units) * kCost[i];
         if (i == 0 || cost < best_cost) {
-            best = i == 0 && tiles <= units ? RingTileF32::k32x32Deep : kTiles[i];
+            const bool deep = i == 0 && ((tiles <= 2 * units && args.k >= 512) || args.k >= 1024);
+            best = deep ? RingTileF32::k32x32Deep : kTiles[i];
             best_cost = cost;
         }
     }
@@ -375,7 +383,10 @@ struct RingChoice {
 /// takes three stages: 64 x 64 tiles up to two per CU (768 x 3072 on 788 rows
 /// 22.0 -> 14.5 us, on 1576 rows 24.0 -> 19.3), 128 x 128 alone on a CU (768 x
 /// 3072 on 4616 rows 31 -> 27 us; two with two stages each beat one at a time
-/// with three, 40 against 51 us on 6304 rows).
+/// with three, 40 against 51 us on 6304 rows). Tiles that are alone on their
+/// CUs have loading wavefronts beside the computing ones (64 x 32 tiles: 197 x
+/// 768 x 768 5.3 -> 4.4 us, 197 x 768 x 3072 11.6 -> 8.5; 64 x 64 from K = 768
+/// on: 197 x 2304 x 768 5.5 -> 4.7; at K = 384 788 x 1152 lost, 4.7 -> 5.3).
 RingChoice choose_ring(const GemmArgs& args) {
     constexpr RingTile kTiles[3] = {RingTile::k64x64, RingTile::k128x64, RingTile::k128x128};
     constexpr int kHeights[3] = {64, 128, 128};
@@ -389,7 +400,11 @@ RingChoice choose_ring(const GemmArgs& args) {
                                                  (args.gelu ? kRingCostGelu[i] : kRingCost[i]);
         if (i == 0 || cost < best.cost) {
             best = RingChoice{kTiles[i], kHeights[i], kWidths[i], cost};
-            if (i == 0 && tiles <= 2 * units && args.k >= 1024) {
+            if (i == 0 && tile_count(args, 64, 32) <= units) {
+                best = RingChoice{RingTile::k64x32Alone, 64, 32, cost};
+            } else if (i == 0 && tiles <= units && args.k >= 768) {
+                best.tile = RingTile::k64x64Alone;
+            } else if (i == 0 && tiles <= 2 * units && args.k >= 1024) {
                 best.tile = RingTile::k64x64Deep;
             } else if (i == 2 && tiles <= units && args.k >= 1024) {
                 best.tile = RingTile::k128x128Deep;

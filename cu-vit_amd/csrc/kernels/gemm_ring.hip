@@ -68,6 +68,10 @@ hipError_t gemm_ring_bf16(RingTile tile, const std::uint16_t* a, const std::uint
     using T = std::uint16_t;
     switch (tile) {
     case RingTile::k64x64: return launch<gemm::RingShape<T, 2, 2, 1, 1, 2>>(a, b, bias, c, args, map, vector_c, stream);
+    case RingTile::k64x32Alone:
+        return launch<gemm::RingShape<T, 2, 1, 1, 1, 4, true, true>>(a, b, bias, c, args, map, vector_c, stream);
+    case RingTile::k64x64Alone:
+        return launch<gemm::RingShape<T, 2, 2, 1, 1, 3, true, true>>(a, b, bias, c, args, map, vector_c, stream);
     case RingTile::k64x64Deep:
         return launch<gemm::RingShape<T, 2, 2, 1, 1, 3, true>>(a, b, bias, c, args, map, vector_c, stream);
     case RingTile::k128x64:
@@ -87,6 +91,7 @@ hipError_t gemm_ring_f32(RingTileF32 tile, const float* a, const float* b, const
                             stream);
     };
     switch (tile) {
+    case RingTileF32::k32x16Alone: return launch_f32(gemm::RingShape<float, 2, 1, 1, 1, 3, true, true>{});
     case RingTileF32::k32x32: return launch_f32(gemm::RingShape<float, 2, 2, 1, 1, 2, true>{});
     case RingTileF32::k32x32Deep: return launch_f32(gemm::RingShape<float, 2, 2, 1, 1, 3, true>{});
     case RingTileF32::k64x32: return launch_f32(gemm::RingShape<float, 2, 2, 2, 1, 2, true>{});

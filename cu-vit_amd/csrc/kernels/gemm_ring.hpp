@@ -1,7 +1,7 @@
 // The GEMM for products with B given as [N, K] that the persistent bf16 kernel
 // (gemm_dma.hpp) and the fp32 panels (gemm_panel.hpp) do not take: in bf16 those
-// with too few tiles for the persistent kernel or no whole 256-column tiles. One tile
-// per workgroup, operands brought into an LDS ring by direct-to-LDS loads.
+// with too few tiles for the persistent kernel or no whole 256-column tiles. One
+// tile per workgroup, operands brought into an LDS ring by direct-to-LDS loads.
 //
 // What bounds these. Tiles are few and K is short (6 to 48 stages of 64), so
 // a tile's time is the latency of its first loads, its LDS traffic and its
@@ -17,24 +17,27 @@
 // 3072: 31 -> 27 us). Eight wavefronts of 32 x 64 beat four of 64 x 64 on the
 // 128 x 128 tile (4616 x 2304 x 768: 24.7 against 25.7 us).
 // Before (gemm_kernel.hpp and gemm_dma.hpp) and now, bf16, us:
-//   4616 x 1152 x 384          18.0 ->  9.9    197 x 768 x 768 (+=)    8.6 -> 5.2
+//   4616 x 1152 x 384          18.0 ->  9.9    197 x 768 x 768 (+=)    8.6 -> 4.4
 //   4616 x 384 x 1536 (+=)     17.5 -> 10.6    1576 x 2304 x 768      17.4 -> 9.4
 //   4616 x 1536 x 384 (GELU)   18.2 -> 13.8    3152 x 2304 x 768      19.2 -> 16.1
 //   6304 x 192 x 768 (+=)      11.4 ->  6.5    12608 x 1152 x 384     38.2 -> 19.6
 // and fp32 (MFMA-bound from a few tiles per CU on):
-//   197 x 192 x 768 (+=)        8.5 ->  7.6    1576 x 2304 x 768      60.3 -> 54.7
+//   197 x 192 x 768 (+=)        8.5 ->  6.6    1576 x 2304 x 768      60.3 -> 54.7
 //   788 x 3072 x 768 (GELU)    45.6 -> 36.0    3152 x 768 x 3072      158  -> 126
 //
 // With kAhead a stage's fragments are read during the stage before, and its
 // loads go out between two k-blocks' MFMAs: a wavefront waits about 85 cycles
 // to issue one, which its MFMAs in flight then cover. It pays where few
-// wavefronts share a SIMD, and costs the registers of a second set.
+// wavefronts share a SIMD, and costs the registers of a second set. With
+// kLoaders as many wavefronts again do nothing but load, for tiles alone on
+// their CU.
 //
-// Stages are rows of 128 bytes (64 bf16 or 32 fp32 of k): chunk c of row r sits in 16-byte slot
-// c ^ ((r >> 1) & 7) of its row, conflict-free for the fragment reads (bf16 lane
-// l: row l % 32, chunk 2 kb + l / 32; fp32: row l % 16, chunk 4 kb + l / 16). One buffer_load_dwordx4 ... lds moves
-// eight rows; every wavefront loads the same number of pieces of A and of B
-// for each stage and waits for its own (vmcnt, the newest kSlots - 2 stages
+// Stages are rows of 128 bytes (64 bf16 or 32 fp32 of k): chunk c of row r sits
+// in 16-byte slot c ^ ((r >> 1) & 7) of its row, conflict-free for the fragment
+// reads (bf16 lane l: row l % 32, chunk 2 kb + l / 32; fp32: row l % 16, chunk 4
+// kb + l / 16). One buffer_load_dwordx4 ... lds moves eight rows; every loading
+// wavefront loads the same number of pieces of A and of B for each stage and
+// waits for its own (vmcnt, the newest kSlots - 2 stages
 // staying in flight) before the stage's barrier. Loads past the last stage go
 // out too, with an offset past the descriptor's range (zeros, no traffic), so
 // that the count in flight is the same in every trip.
@@ -53,11 +56,14 @@ namespace cuvit::detail::gemm {
 
 /// WM x WN wavefronts of TM x TN MFMA tiles of type @p T (bf16 32 x 32, fp32
 /// 16 x 16), Slots stages in the ring.
-template <typename T, int WM, int WN, int TM, int TN, int Slots, bool Ahead = false> struct RingShape {
+template <typename T, int WM, int WN, int TM, int TN, int Slots, bool Ahead = false, bool Loaders = false>
+struct RingShape {
     static constexpr bool kAhead = Ahead;
+    static constexpr bool kLoaders = Loaders;
+    static_assert(Ahead || !Loaders, "loading wavefronts go with fragments read ahead");
     static constexpr int kEdge = Mma<T>::kEdge;
     static constexpr int kWaves = WM * WN;
-    static constexpr int kThreads = kWave * kWaves;
+    static constexpr int kThreads = kWave * kWaves * (Loaders ? 2 : 1);
     static constexpr int kWN = WN;
     static constexpr int kTM = TM;
     static constexpr int kTN = TN;
@@ -178,7 +184,7 @@ template <typename T, typename S> struct RingLoads {
 /// ring.
 template <typename T, typename S>
 __device__ __forceinline__ void ring_multiply(const RingLoads<T, S>& loads, const unsigned char* lds, int wave_m,
-                                              int wave_n, int lane, int stages,
+                                              int wave_n, int lane, bool loading, int stages,
                                               typename Mma<T>::Acc (&acc)[S::kTM][S::kTN]) {
     constexpr int E = S::kEdge;
     constexpr int kBlocks = S::kBK / kKBlock<T>;  // k-blocks per stage
@@ -229,24 +235,53 @@ __device__ __forceinline__ void ring_multiply(const RingLoads<T, S>& loads, cons
             for (int kb = 0; kb < kBlocks; ++kb)
                 read_block(lds + slot * S::kStageBytes, kb, f.a[kb], f.b[kb]);
         };
+        if (!S::kLoaders || loading) {
 #pragma unroll
-        for (int g = 0; g < S::kSlots; ++g) {
-            loads.issue(g, g);
+            for (int g = 0; g < S::kSlots; ++g) {
+                loads.issue(g, g);
+            }
         }
-        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"((S::kSlots - 1) * S::kLoads) : "memory");
+        if (S::kLoaders && loading) {
+            // Half of the wavefronts only load: what a load costs at issue then
+            // delays no MFMA. A stage's slot is free after the barrier that
+            // follows its fragment reads.
+            asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"((S::kSlots - 1) * S::kLoads) : "memory");
+            int slot = 0;
+            for (int g = 0; g < stages; ++g) {
+                asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"((S::kSlots - 2) * S::kLoads) : "memory");
+                loads.issue(g + S::kSlots, slot);
+                slot = slot + 1 == S::kSlots ? 0 : slot + 1;
+            }
+            stage_barrier(true);
+            return;
+        }
+        if constexpr (S::kLoaders) {
+            asm volatile("s_barrier" : : : "memory");
+        } else {
+            asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"((S::kSlots - 1) * S::kLoads) : "memory");
+        }
         read(set[0], 0);
         int slot = 0;
         auto step = [&](int g, Fragments& now, Fragments& next) {
             // Stage g + 1 landed, and every wavefront holds stage g in registers.
-            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"((S::kSlots - 2) * S::kLoads) : "memory");
+            if constexpr (S::kLoaders) {
+                asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory");
+            } else {
+                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier"
+                             :
+                             : "n"((S::kSlots - 2) * S::kLoads)
+                             : "memory");
+            }
             const int free_slot = slot;
             slot = slot + 1 == S::kSlots ? 0 : slot + 1;
             read(next, slot);
             __builtin_amdgcn_sched_barrier(0);
             multiply_block(now.a[0], now.b[0]);
             __builtin_amdgcn_sched_barrier(0);
-            loads.issue(g + S::kSlots, free_slot); // while the MFMAs before run
-            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (!S::kLoaders) {
+                loads.issue(g + S::kSlots, free_slot); // while the MFMAs before run
+                __builtin_amdgcn_sched_barrier(0);
+            }
 #pragma unroll
             for (int kb = 1; kb < kBlocks; ++kb)
                 multiply_block(now.a[kb], now.b[kb]);
@@ -306,7 +341,9 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring_kernel(const std::uint1
     const unsigned int lds_base = __builtin_amdgcn_readfirstlane(lds_address(lds));
 
     const int lane = lane_id();
-    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
+    const int wavefront = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
+    const bool loading = S::kLoaders && wavefront >= S::kWaves;
+    const int wave = loading ? wavefront - S::kWaves : wavefront;
     const int wave_m = wave / S::kWN;
     const int wave_n = wave % S::kWN;
 
@@ -357,7 +394,11 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring_kernel(const std::uint1
 
     const RingLoads<std::uint16_t, S> loads(a, b, args, row0, col0, wave, lane, lds_base);
     floatx16 acc[TM][TN];
-    ring_multiply<std::uint16_t, S>(loads, lds, wave_m, wave_n, lane, (args.k + 127) / 128 * (128 / S::kBK), acc);
+    ring_multiply<std::uint16_t, S>(loads, lds, wave_m, wave_n, lane, loading, (args.k + 127) / 128 * (128 / S::kBK), acc);
+
+    if (loading) {
+        return; // no barrier follows
+    }
 
     // The drained ring becomes staging.
     unsigned char* const staging = lds + wave * S::kStagingBytes;
@@ -453,7 +494,9 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring_f32_kernel(const float*
     unsigned char* const lds = reinterpret_cast<unsigned char*>(lds_vectors);
     const unsigned int lds_base = __builtin_amdgcn_readfirstlane(lds_address(lds));
     const int lane = lane_id();
-    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
+    const int wavefront = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
+    const bool loading = S::kLoaders && wavefront >= S::kWaves;
+    const int wave = loading ? wavefront - S::kWaves : wavefront;
     const int wave_m = wave / S::kWN;
     const int wave_n = wave % S::kWN;
     int row0, col0;
@@ -494,7 +537,10 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring_f32_kernel(const float*
 
     const RingLoads<float, S> loads(a + entry.a, b + entry.b, args, row0, col0, wave, lane, lds_base);
     floatx4 acc[TM][TN];
-    ring_multiply<float, S>(loads, lds, wave_m, wave_n, lane, (args.k + 63) / 64 * (64 / S::kBK), acc);
+    ring_multiply<float, S>(loads, lds, wave_m, wave_n, lane, loading, (args.k + 63) / 64 * (64 / S::kBK), acc);
+    if (loading) {
+        return; // no barrier follows
+    }
 
 #pragma unroll
     for (int i = 0; i < TM; ++i) {

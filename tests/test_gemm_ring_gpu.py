@@ -35,7 +35,11 @@ CASES = [
     (65, 72, 136, True, False, True, 1.0, 8),         # a row and a chunk past; K past one span
     (64, 65, 128, True, False, True, 1.0, 0),         # odd N: element-wise C, accumulating
     (130, 199, 72, False, True, False, -0.5, 3),      # odd rows of C, GELU without bias, alpha
-    (197, 768, 192, True, False, True, 1.0, 0),       # 64 x 64 tiles
+    (197, 768, 3080, True, False, True, 1.0, 0),      # tiles alone on their CUs, long K
+    (65, 2304, 128, True, True, True, 1.0, 0),        # the same at one span of K
+    (197, 2304, 776, True, False, False, 1.0, 0),     # 64 x 64 alone, loading wavefronts
+    (1576, 1536, 200, True, False, True, 1.0, 0),     # several 64 x 64 tiles a CU
+    (1576, 768, 1032, True, False, True, 1.0, 0),     # 64 x 64 tiles with three stages
     (1576, 2304, 200, True, False, False, 1.0, 0),    # 128 x 64 tiles
     (1571, 3064, 64, True, True, True, 1.0, 1),       # 128 x 64 or 128 x 128, odd rows of C
     (6304, 1152, 384, True, False, False, 1.0, 0),    # 128 x 128 tiles
@@ -125,7 +129,8 @@ F32_CASES = [
     (1, 8, 4, True, False, False, 1.0, 0),           # one tile, one chunk of K
     (31, 33, 64, True, True, False, 1.0, 3),         # odd rows of C
     (33, 65, 68, True, False, True, 1.0, 0),         # past a tile, past a span of K; element-wise C
-    (197, 192, 772, False, False, True, -0.5, 4),    # 32 x 32 tiles alone on a CU
+    (197, 192, 772, False, False, True, -0.5, 4),    # tiles alone on their CUs
+    (230, 640, 772, True, False, False, 1.0, 0),     # 32 x 32 tiles with three stages
     (788, 384, 320, True, True, True, 1.0, 0),       # several 32 x 32 tiles a CU
     (1003, 1152, 100, True, False, False, 1.0, 0),   # 64 x 32 or 64 x 64 tiles with tails
     (3151, 1540, 196, False, True, False, 2.0, 0),   # 64 x 64 tiles, GELU without bias
