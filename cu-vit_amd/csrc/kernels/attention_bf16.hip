@@ -447,32 +447,39 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void attention_bf16_kernel(
 template <int KT>
 hipError_t launch(const std::uint16_t* qkv, std::uint16_t* context, int images, int heads,
                   int tokens, hipStream_t stream) {
-    // Query tiles per workgroup, measured on MI355X at 197 tokens: all of
-    // them (one K/V load per (image, head)) once there are two (image, head)
-    // pairs per compute unit (ViT-Base b64: 47.1 us against 49.9 with four),
-    // four below that (ViT-Tiny b32: 11.4 us against 14.8 with seven).
+    // Query tiles per workgroup: four while those workgroups are one per
+    // compute unit at most, else all of them, so that a pair's K and V are
+    // staged once and no compute unit gets two workgroups where another has
+    // one. Measured at 197 tokens, four against all: 96 pairs 7.1 against 8.5
+    // us, 132 9.9 against 8.7, 192 10.7 against 9.0, 252 12.0 against 9.7, 384
+    // 20.1 against 16.5, 504 23.8 against 18.7. Five and six query tiles keep
+    // four just past one pair per compute unit, where the second wavefronts of
+    // the few compute units with two pairs are soon through (264 pairs of six:
+    // 12.5 against 13.4, 384 15.9 against 14.1).
     const int query_tiles = (tokens + kEdge - 1) / kEdge;
     const std::int64_t pairs = static_cast<std::int64_t>(images) * heads;
-    const bool many = pairs >= 2 * static_cast<std::int64_t>(compute_units());
-    const int per_group = many ? kMaxWaves : kWavesPerGroup;
+    const std::int64_t units = compute_units();
+    const std::int64_t groups_of_four = pairs * ((query_tiles + kWavesPerGroup - 1) / kWavesPerGroup);
+    const bool just_past = query_tiles <= kWavesPerGroup + 2 && pairs > units && 10 * pairs < 13 * units;
+    const bool whole = pairs >= 2 * units || (query_tiles > kWavesPerGroup && groups_of_four > units && !just_past);
+    const int per_group = whole ? kMaxWaves : kWavesPerGroup;
     const int waves = query_tiles < per_group ? query_tiles : per_group;
     // (Up to 7 key tiles, 224 tokens: with 8 the prefetch registers spill.)
     if constexpr (KT <= 7) {
-    if (many && pairs <= 0x7FFFFFFF) {
+    if (whole && pairs > units) {
         // One workgroup per CU (the kernel's registers allow one of KT
         // wavefronts) looping over pairs, the next pair's K and V loaded into
         // registers during the current pair's work and into the second LDS
         // buffer after it: each CU's later pairs do not wait for their loads.
         // With waves = KT, a thread's share of a pair's K and V is 8 chunks.
         constexpr int kChunksPerThread = 2 * kEdge * kChunksPerKey / kWave;
-        const std::int64_t groups = compute_units() < pairs ? compute_units() : pairs;
         auto run = [&](auto kernel, std::atomic<std::uint64_t>& opted_in) -> hipError_t {
             if (const hipError_t opted =
                     allow_lds(reinterpret_cast<const void*>(kernel), 2 * lds_bytes(KT), opted_in);
                 opted != hipSuccess) {
                 return opted;
             }
-            kernel<<<dim3(1, static_cast<unsigned int>(groups)), query_tiles * kWave,
+            kernel<<<dim3(1, static_cast<unsigned int>(units)), query_tiles * kWave,
                      2 * lds_bytes(KT), stream>>>(qkv, context, heads, tokens, static_cast<int>(pairs));
             return hipGetLastError();
         };
