@@ -380,13 +380,14 @@ struct RingChoice {
 
 /// The ring kernel's cheapest tile for a problem. Where a CU has few tiles and
 /// K is long, the tile's own loads are all there is to hide behind, and it
-/// takes three stages: 64 x 64 tiles up to two per CU (768 x 3072 on 788 rows
-/// 22.0 -> 14.5 us, on 1576 rows 24.0 -> 19.3), 128 x 128 alone on a CU (768 x
-/// 3072 on 4616 rows 31 -> 27 us; two with two stages each beat one at a time
-/// with three, 40 against 51 us on 6304 rows). Tiles that are alone on their
-/// CUs have loading wavefronts beside the computing ones (64 x 32 tiles: 197 x
-/// 768 x 768 5.3 -> 4.4 us, 197 x 768 x 3072 11.6 -> 8.5; 64 x 64 from K = 768
-/// on: 197 x 2304 x 768 5.5 -> 4.7; at K = 384 788 x 1152 lost, 4.7 -> 5.3).
+/// takes three stages: 64 x 64 tiles up to two per CU (768 x 3072 on 1576 rows
+/// 24.0 -> 19.3 us; FC2 of 4616 rows, 384 x 1536, two microseconds inside its
+/// forward), 128 x 128 alone on a CU (768 x 3072 on 4616 rows 31 -> 27 us; two
+/// with two stages each beat one at a time with three, 40 against 51 us on 6304
+/// rows). Tiles that are alone on their CUs have loading wavefronts beside the
+/// computing ones (64 x 32 tiles: 197 x 768 x 768 5.3 -> 4.4 us, 197 x 768 x 3072
+/// 11.6 -> 8.5; 64 x 64 from K = 768 on: 197 x 2304 x 768 5.5 -> 4.7; at K = 384
+/// 788 x 1152 lost, 4.7 -> 5.3).
 RingChoice choose_ring(const GemmArgs& args) {
     constexpr RingTile kTiles[3] = {RingTile::k64x64, RingTile::k128x64, RingTile::k128x128};
     constexpr int kHeights[3] = {64, 128, 128};

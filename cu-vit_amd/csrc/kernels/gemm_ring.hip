@@ -75,7 +75,7 @@ hipError_t gemm_ring_bf16(RingTile tile, const std::uint16_t* a, const std::uint
     case RingTile::k64x64Deep:
         return launch<gemm::RingShape<T, 2, 2, 1, 1, 3, true>>(a, b, bias, c, args, map, vector_c, stream);
     case RingTile::k128x64:
-        return launch<gemm::RingShape<T, 4, 2, 1, 1, 2, true>>(a, b, bias, c, args, map, vector_c, stream);
+        return launch<gemm::RingShape<T, 4, 2, 1, 1, 2>>(a, b, bias, c, args, map, vector_c, stream);
     case RingTile::k128x128:
         return launch<gemm::RingShape<T, 4, 2, 1, 2, 2>>(a, b, bias, c, args, map, vector_c, stream);
     default: return launch<gemm::RingShape<T, 4, 2, 1, 2, 3>>(a, b, bias, c, args, map, vector_c, stream);
