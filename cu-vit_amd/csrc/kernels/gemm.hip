@@ -86,7 +86,7 @@ gemm::TileMap tile_map(const GemmArgs& args, int bm, int bn, std::size_t element
 template <typename T, int WM, int WN, int TM, int TN, int BK, int MinWaves, bool VecA, bool VecB,
           bool TransB>
 hipError_t launch(const T* a, const T* b, const float* bias, T* c, const GemmArgs& args,
-                  bool vector_c, hipStream_t stream) {
+                  bool vector_c, bool spans_a, bool spans_b, hipStream_t stream) {
     using S = Shape<T, WM, WN, TM, TN, BK>;
     const gemm::TileMap map = tile_map(args, S::kBM, S::kBN, sizeof(T));
     const std::int64_t tiles_m = (args.m + S::kBM - 1) / S::kBM;
@@ -111,7 +111,7 @@ hipError_t launch(const T* a, const T* b, const float* bias, T* c, const GemmArg
     }
     const dim3 grid(static_cast<unsigned int>(tiles),
                     static_cast<unsigned int>(args.count < kMaxGridY ? args.count : kMaxGridY));
-    kernel<<<grid, S::kThreads, S::kLdsBytes, stream>>>(a, b, bias, c, args, map, vector_c);
+    kernel<<<grid, S::kThreads, S::kLdsBytes, stream>>>(a, b, bias, c, args, map, vector_c, spans_a, spans_b);
     return hipGetLastError();
 }
 
@@ -121,21 +121,19 @@ hipError_t pick_flags(const T* a, const T* b, const float* bias, T* c, const Gem
     using S = Shape<T, WM, WN, TM, TN, BK>;
     const bool split = args.inner > 0;
     // Buffer offsets of a tile stay inside the span one descriptor addresses.
-    bool vec_a = vector_operand(a, args.lda, args.k, args.stride_a, args.outer_stride_a, split) &&
-                 static_cast<std::int64_t>(S::kBM) * args.lda * sizeof(T) < gemm::kMaxSpan;
-    bool vec_b;
-    if (args.transposed) {
-        vec_b = vector_operand(b, args.ldb, args.k, args.stride_b, args.outer_stride_b, split) &&
-                static_cast<std::int64_t>(S::kBN) * args.ldb * sizeof(T) < gemm::kMaxSpan;
-    } else {
-        vec_b = vector_operand(b, args.ldb, args.n, args.stride_b, args.outer_stride_b, split) &&
-                static_cast<std::int64_t>(args.k) * args.ldb * sizeof(T) < gemm::kMaxSpan;
-    }
+    const bool spans_a = static_cast<std::int64_t>(S::kBM) * args.lda * sizeof(T) < gemm::kMaxSpan;
+    const bool spans_b = (args.transposed ? static_cast<std::int64_t>(S::kBN) : static_cast<std::int64_t>(args.k)) *
+                             args.ldb * sizeof(T) <
+                         gemm::kMaxSpan;
+    const bool vec_a =
+        spans_a && vector_operand(a, args.lda, args.k, args.stride_a, args.outer_stride_a, split);
+    const bool vec_b = spans_b && vector_operand(b, args.ldb, args.transposed ? args.k : args.n, args.stride_b,
+                                                 args.outer_stride_b, split);
     const bool vec_c = vector_output(c, args);
 #define CUVIT_GEMM_LAUNCH(VA, VB)                                                                  \
     (args.transposed                                                                               \
-         ? launch<T, WM, WN, TM, TN, BK, MinWaves, VA, VB, true>(a, b, bias, c, args, vec_c, stream) \
-         : launch<T, WM, WN, TM, TN, BK, MinWaves, VA, VB, false>(a, b, bias, c, args, vec_c, stream))
+         ? launch<T, WM, WN, TM, TN, BK, MinWaves, VA, VB, true>(a, b, bias, c, args, vec_c, spans_a, spans_b, stream) \
+         : launch<T, WM, WN, TM, TN, BK, MinWaves, VA, VB, false>(a, b, bias, c, args, vec_c, spans_a, spans_b, stream))
     if (vec_a) {
         return vec_b ? CUVIT_GEMM_LAUNCH(true, true) : CUVIT_GEMM_LAUNCH(true, false);
     }

@@ -169,26 +169,40 @@ __device__ __forceinline__ unsigned int chunk_offset(int row, int rows, int ld, 
 typedef float floatx4_unaligned __attribute__((ext_vector_type(4), aligned(4)));
 
 /// Scalar path: one 16-byte chunk of a row-major [rows][depth] operand, row
-/// @p row, elements @p k .. + kPerVec, zero outside. A whole chunk of floats is
-/// one load all the same, whatever its row's alignment (the attention.V product
-/// of 24 heads at 577 tokens, odd rows of A: 29.9 -> 26.3 us).
+/// @p row, elements @p k .. + kPerVec, zero outside.
 template <typename T>
 __device__ __forceinline__ Vec16 load_chunk_scalar(const T* matrix, int ld, int row, int rows, int k,
                                                    int depth) {
     Vec16 v{{0U, 0U, 0U, 0U}};
     if (row < rows) {
         const T* p = matrix + static_cast<std::int64_t>(row) * ld;
-        if constexpr (sizeof(T) == 4) {
-            if (k + 3 < depth) {
-                return __builtin_bit_cast(Vec16, *reinterpret_cast<const floatx4_unaligned*>(p + k));
-            }
-        }
 #pragma unroll
         for (int e = 0; e < Mma<T>::kPerVec; ++e) {
             if (k + e < depth) {
                 Elem<T>::put_bits(v, e, p + k + e);
             }
         }
+    }
+    return v;
+}
+
+/// The same of an fp32 operand whose rows start at any float, through its buffer
+/// resource: with @p whole (uniform: no chunk of the stage is cut) one load,
+/// which needs 4-byte alignment only, else one per element, without a branch on
+/// the lane either way, so that a stage's loads stay in flight like the vector
+/// path's. The element-wise scalar path waited out a memory latency a stage
+/// (attention by launches at 577 tokens, 24 heads, whose weights.V product has
+/// odd rows of A: 64.6 -> 61.5 us for the three launches, with whole chunks
+/// already loaded at once on that path).
+__device__ __forceinline__ Vec16 load_chunk_unaligned(__amdgpu_buffer_rsrc_t resource, int row, int rows, int ld,
+                                                      int k, int depth, bool whole) {
+    if (whole) {
+        return buffer_load16(resource, chunk_offset<float>(row, rows, ld, k, depth));
+    }
+    Vec16 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        v.w[e] = __builtin_amdgcn_raw_buffer_load_b32(resource, chunk_offset<float>(row, rows, ld, k + e, depth), 0, 0);
     }
     return v;
 }
@@ -303,6 +317,8 @@ __device__ __forceinline__ int split_point(int n, int parts, int i) { return n *
 /// in pairs; bf16 stages are 32 or 64 deep and run to a multiple of 128.
 template <typename T> constexpr int kSpan = sizeof(T) == 2 ? 128 : 64;
 
+/// @p spans_a, @p spans_b: an operand that is no vector operand (VecA, VecB
+/// false) still has its tile within one resource's span.
 /// @tparam MinWaves wavefronts per SIMD the register allocation must allow
 /// (amdgpu_waves_per_eu); 1 leaves the compiler free.
 template <typename T, int WM, int WN, int TM, int TN, int BK, bool VecA, bool VecB, bool TransB,
@@ -310,7 +326,8 @@ template <typename T, int WM, int WN, int TM, int TN, int BK, bool VecA, bool Ve
 __global__ __launch_bounds__(kWave * WM * WN) __attribute__((amdgpu_waves_per_eu(MinWaves))) void gemm_kernel(const T* __restrict__ a,
                                                         const T* __restrict__ b,
                                                         const float* __restrict__ bias, T* c,
-                                                        GemmArgs args, TileMap map, bool vector_c) {
+                                                        GemmArgs args, TileMap map, bool vector_c,
+                                                        bool spans_a, bool spans_b) {
     using S = Shape<T, WM, WN, TM, TN, BK>;
     constexpr int BM = S::kBM;
     constexpr int BN = S::kBN;
@@ -391,7 +408,12 @@ __global__ __launch_bounds__(kWave * WM * WN) __attribute__((amdgpu_waves_per_eu
                         ra[p] = buffer_load16(a_resource,
                                               chunk_offset<T>(row, a_rows, args.lda, k, args.k));
                     } else {
-                        ra[p] = load_chunk_scalar(a_tile, args.lda, row, a_rows, k, args.k);
+                        if (sizeof(T) == 4 && spans_a) {
+                            ra[p] = load_chunk_unaligned(a_resource, row, a_rows, args.lda, k, args.k,
+                                                         k0 + BK <= args.k);
+                        } else {
+                            ra[p] = load_chunk_scalar(a_tile, args.lda, row, a_rows, k, args.k);
+                        }
                     }
                 }
             }
@@ -406,7 +428,12 @@ __global__ __launch_bounds__(kWave * WM * WN) __attribute__((amdgpu_waves_per_eu
                             rb[p] = buffer_load16(b_resource,
                                                   chunk_offset<T>(row, b_rows, args.ldb, k, args.k));
                         } else {
-                            rb[p] = load_chunk_scalar(b_tile, args.ldb, row, b_rows, k, args.k);
+                            if (sizeof(T) == 4 && spans_b) {
+                                rb[p] = load_chunk_unaligned(b_resource, row, b_rows, args.ldb, k, args.k,
+                                                             k0 + BK <= args.k);
+                            } else {
+                                rb[p] = load_chunk_scalar(b_tile, args.ldb, row, b_rows, k, args.k);
+                            }
                         }
                     } else {
                         // [BK][BN] in global order: chunk q is k row q / (BN / V),
@@ -417,7 +444,12 @@ __global__ __launch_bounds__(kWave * WM * WN) __attribute__((amdgpu_waves_per_eu
                             rb[p] = buffer_load16(b_resource,
                                                   chunk_offset<T>(k, args.k, args.ldb, n, b_rows));
                         } else {
-                            rb[p] = load_chunk_scalar(b_tile, args.ldb, k, args.k, n, b_rows);
+                            if (sizeof(T) == 4 && spans_b) {
+                                rb[p] = load_chunk_unaligned(b_resource, k, args.k, args.ldb, n, b_rows,
+                                                             BN <= b_rows);
+                            } else {
+                                rb[p] = load_chunk_scalar(b_tile, args.ldb, k, args.k, n, b_rows);
+                            }
                         }
                     }
                 }
