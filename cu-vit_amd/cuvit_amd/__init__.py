@@ -1,8 +1,9 @@
 """Python binding of libcuvit_amd.so, the MI355X (gfx950) layer-kernel library.
 
 The library's interface is the C ABI in include/cuvit/capi.h; this module binds
-it with ctypes so tests and the benchmark can drive the HIP kernels on device
-tensors that PyTorch allocates. PyTorch provides device memory and the stream
+it with ctypes, and the launchers' plain case with the native module beside it
+(_native.so), so programs can drive the HIP kernels on device tensors that
+PyTorch allocates. PyTorch provides device memory and the stream
 handle only; every computation runs in the library's own HIP kernels. There is
 no fallback: if the library is not built, loading raises.
 
@@ -257,8 +258,8 @@ class _NativeCalls:
     takes a launcher's arguments and returns the library's status, or -1 where
     they are not plain GPU tensors and whole numbers that pass every check.
     The module is loaded with the first launcher that can be given a tensor:
-    a program without torch has none. Host time of a LayerNorm call 8 -> 1 us
-    beside the launch itself."""
+    a program without torch has none. A LayerNorm call of 197 rows takes 4.0 us
+    of a stream of calls so, 10.4 through the Python code."""
 
     def __getattr__(self, name):
         if "torch" not in sys.modules:
