@@ -102,11 +102,9 @@ hipError_t launch(const T* a, const T* b, const float* bias, T* c, const GemmArg
     // The occupancy hint caps registers; the element-wise operand paths need
     // more than it leaves, so they take the default.
     constexpr int kMinWaves = VecA && VecB ? MinWaves : 1;
-    auto kernel = gemm::gemm_kernel<T, WM, WN, TM, TN, BK, VecA, VecB, TransB, kMinWaves>;
+    constexpr auto kernel = gemm::gemm_kernel<T, WM, WN, TM, TN, BK, VecA, VecB, TransB, kMinWaves>;
     // Above 64 KiB of LDS a kernel has to opt in, once per device.
-    static std::atomic<std::uint64_t> opted_in{0};
-    if (const hipError_t opted = allow_lds(reinterpret_cast<const void*>(kernel), S::kLdsBytes, opted_in);
-        opted != hipSuccess) {
+    if (const hipError_t opted = allow_lds<kernel>(S::kLdsBytes); opted != hipSuccess) {
         return opted;
     }
     const dim3 grid(static_cast<unsigned int>(tiles),
@@ -201,11 +199,9 @@ hipError_t launch_panel(const float* a, const float* b, const float* bias, float
     groups = groups < 1 ? 1 : groups > tiles_m ? tiles_m : groups;
     const dim3 grid(static_cast<unsigned int>(panels * groups));
     const int groups_argument = static_cast<int>(groups);
-    auto run = [&](auto kernel) -> hipError_t {
-        static std::atomic<std::uint64_t> opted_in{0};
-        if (const hipError_t opted =
-                allow_lds(reinterpret_cast<const void*>(kernel), S::kLdsBytes, opted_in);
-            opted != hipSuccess) {
+    auto run = [&](auto chosen) -> hipError_t {
+        constexpr auto kernel = decltype(chosen)::kValue;
+        if (const hipError_t opted = allow_lds<kernel>(S::kLdsBytes); opted != hipSuccess) {
             return opted;
         }
         kernel<<<grid, S::kThreads, S::kLdsBytes, stream>>>(a, b, bias, c, args, groups_argument);
@@ -214,16 +210,16 @@ hipError_t launch_panel(const float* a, const float* b, const float* bias, float
     // The epilogue's parts as template flags: alpha (when not 1), bias, GELU,
     // accumulate; the addend alone (the patch embedding's positional add).
     auto with_alpha = [&](auto alpha, auto with_bias, auto gelu, auto accumulate) -> hipError_t {
-        return run(gemm::gemm_panel_kernel<KB, BN, TN, KG, W, decltype(alpha)::value,
-                                           decltype(with_bias)::value, decltype(gelu)::value,
-                                           decltype(accumulate)::value>);
+        return run(KernelConstant<gemm::gemm_panel_kernel<KB, BN, TN, KG, W, decltype(alpha)::value,
+                                                          decltype(with_bias)::value, decltype(gelu)::value,
+                                                          decltype(accumulate)::value>>{});
     };
     if (with_addend) {
         auto with_bias = [&](auto alpha) -> hipError_t {
             constexpr bool kAlpha = decltype(alpha)::value;
             return bias != nullptr
-                       ? run(gemm::gemm_panel_kernel<KB, BN, TN, KG, W, kAlpha, true, false, false, true>)
-                       : run(gemm::gemm_panel_kernel<KB, BN, TN, KG, W, kAlpha, false, false, false, true>);
+                       ? run(KernelConstant<gemm::gemm_panel_kernel<KB, BN, TN, KG, W, kAlpha, true, false, false, true>>{})
+                       : run(KernelConstant<gemm::gemm_panel_kernel<KB, BN, TN, KG, W, kAlpha, false, false, false, true>>{});
         };
         return args.alpha == 1.0F ? with_bias(std::false_type{}) : with_bias(std::true_type{});
     }
@@ -467,10 +463,9 @@ hipError_t launch_dma(const std::uint16_t* a, const std::uint16_t* b, const floa
     if (bm == 0 || ring_cost < rounds * bm * (args.gelu ? kDmaRowGelu : kDmaRow)) {
         return hipErrorNotSupported;
     }
-    auto run = [&](auto kernel, std::size_t lds_bytes) -> hipError_t {
-        static std::atomic<std::uint64_t> opted_in{0};
-        if (const hipError_t opted = allow_lds(reinterpret_cast<const void*>(kernel), lds_bytes, opted_in);
-            opted != hipSuccess) {
+    auto run = [&](auto chosen, std::size_t lds_bytes) -> hipError_t {
+        constexpr auto kernel = decltype(chosen)::kValue;
+        if (const hipError_t opted = allow_lds<kernel>(lds_bytes); opted != hipSuccess) {
             return opted;
         }
         kernel<<<units, 512, lds_bytes, stream>>>(a, b, bias, c, args, map);
@@ -485,15 +480,15 @@ hipError_t launch_dma(const std::uint16_t* a, const std::uint16_t* b, const floa
             if constexpr (BM == 320) {
                 return hipErrorNotSupported;  // not chosen for an addend (see above)
             } else {
-                return run(gemm::gemm_dma_kernel<BM, true, false, false, false, true>, kLds);
+                return run(KernelConstant<gemm::gemm_dma_kernel<BM, true, false, false, false, true>>{}, kLds);
             }
         }
         auto with_flags = [&](auto with_bias, auto with_gelu, auto with_alpha) -> hipError_t {
             constexpr bool kB = decltype(with_bias)::value;
             constexpr bool kG = decltype(with_gelu)::value;
             constexpr bool kA = decltype(with_alpha)::value;
-            return args.accumulate ? run(gemm::gemm_dma_kernel<BM, kB, kG, kA, true>, kLds)
-                                   : run(gemm::gemm_dma_kernel<BM, kB, kG, kA, false>, kLds);
+            return args.accumulate ? run(KernelConstant<gemm::gemm_dma_kernel<BM, kB, kG, kA, true>>{}, kLds)
+                                   : run(KernelConstant<gemm::gemm_dma_kernel<BM, kB, kG, kA, false>>{}, kLds);
         };
         auto with_alpha = [&](auto with_bias, auto with_gelu) -> hipError_t {
             return args.alpha == 1.0F ? with_flags(with_bias, with_gelu, std::false_type{})

@@ -7,12 +7,11 @@ namespace {
 
 constexpr int kMaxGridY = 65535;
 
-/// Launches @p kernel over the tile grid, one workgroup per tile (per slot of
+/// Launches @p Kernel over the tile grid, one workgroup per tile (per slot of
 /// the largest XCD block with a split) and batch entry.
-template <typename S, typename Kernel, typename T>
-hipError_t run_tiles(Kernel kernel, std::atomic<std::uint64_t>& opted_in, const T* a, const T* b,
-                     const float* bias, T* c, const GemmArgs& args, const gemm::TileMap& map, bool vector_c,
-                     hipStream_t stream) {
+template <typename S, auto Kernel, typename T>
+hipError_t run_tiles(const T* a, const T* b, const float* bias, T* c, const GemmArgs& args,
+                     const gemm::TileMap& map, bool vector_c, hipStream_t stream) {
     const std::int64_t tiles_m = (args.m + S::kBM - 1) / S::kBM;
     const std::int64_t tiles_n = (args.n + S::kBN - 1) / S::kBN;
     const std::int64_t tiles = map.px > 0 ? 8 * ((tiles_m + map.px - 1) / map.px) *
@@ -21,15 +20,14 @@ hipError_t run_tiles(Kernel kernel, std::atomic<std::uint64_t>& opted_in, const 
     if (tiles > 0x7FFFFFFF) {
         return hipErrorInvalidConfiguration;
     }
-    if (const hipError_t opted = allow_lds(reinterpret_cast<const void*>(kernel), S::kLdsBytes, opted_in);
-        opted != hipSuccess) {
+    if (const hipError_t opted = allow_lds<Kernel>(S::kLdsBytes); opted != hipSuccess) {
         return opted;
     }
     // A grid's y extent is limited: more entries than that take several launches.
     for (int first = 0; first < args.count; first += kMaxGridY) {
         const int entries = args.count - first < kMaxGridY ? args.count - first : kMaxGridY;
         const dim3 grid(static_cast<unsigned int>(tiles), static_cast<unsigned int>(entries));
-        kernel<<<grid, S::kThreads, S::kLdsBytes, stream>>>(a, b, bias, c, args, map, vector_c, first);
+        Kernel<<<grid, S::kThreads, S::kLdsBytes, stream>>>(a, b, bias, c, args, map, vector_c, first);
         if (const hipError_t launched = hipGetLastError(); launched != hipSuccess) {
             return launched;
         }
@@ -41,20 +39,19 @@ template <typename S>
 hipError_t launch(const std::uint16_t* a, const std::uint16_t* b, const float* bias, std::uint16_t* c,
                   const GemmArgs& args, const gemm::TileMap& map, bool vector_c, hipStream_t stream) {
     auto run = [&](auto kernel) -> hipError_t {
-        static std::atomic<std::uint64_t> opted_in{0};
-        return run_tiles<S>(kernel, opted_in, a, b, bias, c, args, map, vector_c, stream);
+        return run_tiles<S, decltype(kernel)::kValue>(a, b, bias, c, args, map, vector_c, stream);
     };
     if (args.addend != nullptr) {
-        return run(gemm::gemm_ring_kernel<S, true, false, false, true>);
+        return run(KernelConstant<gemm::gemm_ring_kernel<S, true, false, false, true>>{});
     }
     auto with_gelu = [&](auto with_bias) -> hipError_t {
         constexpr bool kB = decltype(with_bias)::value;
         if (args.gelu) {
-            return args.accumulate ? run(gemm::gemm_ring_kernel<S, kB, true, true>)
-                                   : run(gemm::gemm_ring_kernel<S, kB, true, false>);
+            return args.accumulate ? run(KernelConstant<gemm::gemm_ring_kernel<S, kB, true, true>>{})
+                                   : run(KernelConstant<gemm::gemm_ring_kernel<S, kB, true, false>>{});
         }
-        return args.accumulate ? run(gemm::gemm_ring_kernel<S, kB, false, true>)
-                               : run(gemm::gemm_ring_kernel<S, kB, false, false>);
+        return args.accumulate ? run(KernelConstant<gemm::gemm_ring_kernel<S, kB, false, true>>{})
+                               : run(KernelConstant<gemm::gemm_ring_kernel<S, kB, false, false>>{});
     };
     return bias != nullptr ? with_gelu(std::true_type{}) : with_gelu(std::false_type{});
 }
@@ -86,9 +83,7 @@ hipError_t gemm_ring_f32(RingTileF32 tile, const float* a, const float* b, const
                          const GemmArgs& args, hipStream_t stream) {
     auto launch_f32 = [&](auto shape) -> hipError_t {
         using S = decltype(shape);
-        static std::atomic<std::uint64_t> opted_in{0};
-        return run_tiles<S>(gemm::gemm_ring_f32_kernel<S>, opted_in, a, b, bias, c, args, gemm::TileMap{0, 0}, true,
-                            stream);
+        return run_tiles<S, gemm::gemm_ring_f32_kernel<S>>(a, b, bias, c, args, gemm::TileMap{0, 0}, true, stream);
     };
     switch (tile) {
     case RingTileF32::k32x16Alone: return launch_f32(gemm::RingShape<float, 2, 1, 1, 1, 3, true, true>{});

@@ -159,6 +159,18 @@ int compute_units();
 /// the devices already done.
 hipError_t allow_lds(const void* kernel, std::size_t bytes, std::atomic<std::uint64_t>& devices);
 
+/// The same for @p Kernel, which is part of the bit set's name: kernels of one
+/// function type never share a set.
+template <auto Kernel> hipError_t allow_lds(std::size_t bytes) {
+    static std::atomic<std::uint64_t> devices{0};
+    return allow_lds(reinterpret_cast<const void*>(Kernel), bytes, devices);
+}
+
+/// A kernel as a type, for generic lambdas that pick one and launch it.
+template <auto Kernel> struct KernelConstant {
+    static constexpr auto kValue = Kernel;
+};
+
 /// Grid size for a grid-stride kernel: enough blocks to cover @p units of work,
 /// capped so the work-item count stays far inside the 32-bit dispatch limit.
 unsigned int stride_grid(std::int64_t units, int units_per_block, int cap_per_cu);
