@@ -17,6 +17,7 @@
 #include <ATen/core/Tensor.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/version.h>
 
 #include <climits>
 #include <cstddef>
@@ -441,4 +442,18 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", "The launchers' plain ca
 
 } // namespace
 
-PyMODINIT_FUNC PyInit__native() { return PyModule_Create(&module); }
+/// The module, with the PyTorch and Python that it was compiled for: the Python
+/// side uses it with these only.
+PyMODINIT_FUNC PyInit__native() {
+    PyObject* const created = PyModule_Create(&module);
+    if (created == nullptr) {
+        return nullptr;
+    }
+    PyObject* const built_for = Py_BuildValue("(sii)", TORCH_VERSION, PY_MAJOR_VERSION, PY_MINOR_VERSION);
+    if (built_for == nullptr || PyModule_AddObject(created, "built_for", built_for) != 0) {
+        Py_XDECREF(built_for);
+        Py_DECREF(created);
+        return nullptr;
+    }
+    return created;
+}

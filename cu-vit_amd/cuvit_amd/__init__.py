@@ -18,6 +18,7 @@ from __future__ import annotations
 import ctypes
 import os
 import sys
+import threading
 from typing import Optional
 
 __all__ = [
@@ -253,26 +254,60 @@ _NATIVE_FUNCTIONS = (
 )
 
 
+_NATIVE_CALLS = ("layer_norm", "softmax", "extract_patches", "gemm", "attention", "preprocess", "vit_forward")
+
+
+def _not_plain(*arguments) -> int:
+    return -1
+
+
+def _native_module(torch):
+    """The native module, or None (with a warning) where it is not built or was
+    built for another PyTorch or Python, whose tensors it would misread."""
+    import warnings
+
+    try:
+        from . import _native
+    except ImportError as error:
+        reason = str(error)
+    else:
+        here = (torch.__version__.split("+")[0], *sys.version_info[:2])
+        if getattr(_native, "built_for", None) == here:
+            return _native
+        reason = f"it was built for {getattr(_native, 'built_for', 'an older binding')}, this is {here}"
+    warnings.warn(f"cuvit_amd: no native binding ({reason}); calls take the slower ctypes path. "
+                  "Build it with `make python` in cu-vit_amd.", RuntimeWarning, stacklevel=4)
+    return None
+
+
 class _NativeCalls:
     """The launchers' plain case in native code (csrc/binding/native.cpp): each
     takes a launcher's arguments and returns the library's status, or -1 where
-    they are not plain GPU tensors and whole numbers that pass every check.
+    they are not plain GPU tensors and whole numbers that pass every check; the
+    Python code then takes the call, as it does every call without the module.
     The module is loaded with the first launcher that can be given a tensor:
     a program without torch has none. A LayerNorm call of 197 rows takes 4.0 us
     of a stream of calls so, 10.4 through the Python code."""
 
-    def __getattr__(self, name):
-        if "torch" not in sys.modules:
-            return lambda *arguments: -1
-        from . import _native
+    def __init__(self):
+        self._lock = threading.Lock()
 
-        lib = library()
-        _native.bind(GemmProblem, Preprocessing,
-                     *(ctypes.cast(getattr(lib, f), _P).value for f in _NATIVE_FUNCTIONS))
-        for call in ("layer_norm", "softmax", "extract_patches", "gemm", "attention", "preprocess",
-                     "vit_forward"):
-            setattr(self, call, getattr(_native, call))
-        return getattr(_native, name)
+    def __getattr__(self, name):
+        if name not in _NATIVE_CALLS:
+            raise AttributeError(name)
+        torch = sys.modules.get("torch")
+        if torch is None:
+            return _not_plain
+        with self._lock:
+            if name not in self.__dict__:
+                native = _native_module(torch)
+                if native is not None:
+                    lib = library()
+                    native.bind(GemmProblem, Preprocessing,
+                                *(ctypes.cast(getattr(lib, f), _P).value for f in _NATIVE_FUNCTIONS))
+                for call in _NATIVE_CALLS:
+                    setattr(self, call, getattr(native, call) if native is not None else _not_plain)
+        return self.__dict__[name]
 
 
 _native_calls = _NativeCalls()
