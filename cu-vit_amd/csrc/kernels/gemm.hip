@@ -15,6 +15,7 @@
 //        1024), else 64 x 64.
 // Every kernel of a type runs the same MFMA over K in the same order, so the
 // choice never changes a result.
+#include "gemm_choice.hpp"
 #include "gemm_dma.hpp"
 #include "gemm_kernel.hpp"
 #include "gemm_panel.hpp"
@@ -47,40 +48,6 @@ template <typename T> bool vector_output(const T* c, const GemmArgs& args) {
     const bool split = args.inner > 0;
     return (reinterpret_cast<std::uintptr_t>(c) % (4 * sizeof(T))) == 0 && args.ldc % 4 == 0 &&
            args.stride_c % 4 == 0 && (!split || args.outer_stride_c % 4 == 0);
-}
-
-/// The px x py split of an entry's tile grid among the 8 XCDs (px * py = 8)
-/// that moves the fewest bytes into their L2 caches, A being read once per
-/// column block and B once per row block, counting B double when its block
-/// would not fit comfortably in one XCD's 4 MB L2. Measured on the ViT-Base
-/// bf16 GEMMs: FC1 183 -> 173 us, FC2 129 -> 120 us. The fp32 ViT-Tiny GEMMs
-/// (a few MB in all) gained nothing from it, so they keep row-major order.
-gemm::TileMap tile_map(const GemmArgs& args, int bm, int bn, std::size_t element) {
-    gemm::TileMap map{0, 0};
-    const int tiles_m = (args.m + bm - 1) / bm;
-    const int tiles_n = (args.n + bn - 1) / bn;
-    if (element != 2 || static_cast<std::int64_t>(tiles_m) * tiles_n < 64) {
-        return map;
-    }
-    const double a_bytes = static_cast<double>(tiles_m) * bm * args.k * element;
-    const double b_bytes = static_cast<double>(tiles_n) * bn * args.k * element;
-    constexpr double kL2Budget = 3.0 * (1 << 20);
-    double best = 0.0;
-    for (const int px : {8, 4, 2, 1}) {
-        const int py = 8 / px;
-        if (px > tiles_m || py > tiles_n) {
-            continue;
-        }
-        double cost = py * a_bytes + px * b_bytes;
-        if (b_bytes / py > kL2Budget) {
-            cost *= 2.0;
-        }
-        if (map.px == 0 || cost < best) {
-            best = cost;
-            map = gemm::TileMap{px, py};
-        }
-    }
-    return map;
 }
 
 template <typename T, int WM, int WN, int TM, int TN, int BK, int MinWaves, bool VecA, bool VecB,
@@ -153,10 +120,6 @@ GemmArgs as_one_problem(const GemmArgs& args) {
         whole.rows_per_entry = args.m;
     }
     return whole;
-}
-
-std::int64_t tile_count(const GemmArgs& args, int bm, int bn) {
-    return static_cast<std::int64_t>((args.m + bm - 1) / bm) * ((args.n + bn - 1) / bn) * args.count;
 }
 
 } // namespace
@@ -315,111 +278,15 @@ hipError_t gemm_f32(const float* a, const float* b, const float* bias, float* c,
     return pick_flags<float, 2, 2, 1, 1, 32>(a, b, bias, c, args, stream);
 }
 
-/// The XCD split for a persistent kernel whose @p turns workgroups per XCD
-/// take an XCD's tiles in turn: fewest rounds (the largest block's tiles over
-/// @p turns), then the fewest bytes moved into the L2 caches (tile_map's
-/// measure). Measured at ViT-Base FC2 on 192 x 256 tiles: a byte-only choice
-/// left one XCD 34 tiles for its 32 workgroups, 139 against 88 us.
-gemm::TileMap balanced_map(const GemmArgs& args, int bm, int bn, int turns, int* rounds_out) {
-    const int tiles_m = (args.m + bm - 1) / bm;
-    const int tiles_n = (args.n + bn - 1) / bn;
-    const double a_bytes = static_cast<double>(tiles_m) * bm * args.k * 2;
-    const double b_bytes = static_cast<double>(tiles_n) * bn * args.k * 2;
-    constexpr double kL2Budget = 3.0 * (1 << 20);
-    gemm::TileMap best{0, 0};
-    double best_cost = 0.0;
-    int best_rounds = 0;
-    for (const int px : {8, 4, 2, 1}) {
-        const int py = 8 / px;
-        if (px > tiles_m || py > tiles_n) {
-            continue;
-        }
-        const int block = ((tiles_m + px - 1) / px) * ((tiles_n + py - 1) / py);
-        const int rounds = (block + turns - 1) / turns;
-        double cost = py * a_bytes + px * b_bytes;
-        if (b_bytes / py > kL2Budget) {
-            cost *= 2.0;
-        }
-        if (best.px == 0 || rounds < best_rounds || (rounds == best_rounds && cost < best_cost)) {
-            best = gemm::TileMap{px, py};
-            best_cost = cost;
-            best_rounds = rounds;
-        }
-    }
-    *rounds_out = best_rounds;
-    return best;
-}
-
-/// Relative times of the bf16 kernels with B as [N, K], one 64 x 64 ring tile
-/// per CU without GELU being 1, all proportional to K: a CU's row of ring tiles
-/// takes ceil(tiles / CUs) times the tile's cost, the persistent kernel rounds x
-/// BM times its cost per row of a 256-wide tile. Fitted to MI355X times at K =
-/// 384 and 768, M from 197 to 12608 (us at K = 768: a 64 x 64 tile 2.65, 128 x
-/// 64 4.4, 128 x 128 7.7, a persistent 192-row tile 16.7; at K = 384: 1.6, 2.6,
-/// 4.2). The GELU weighs more where fewer wavefronts share a SIMD.
-constexpr double kRingCost[3] = {1.0, 1.65, 2.9};
-constexpr double kRingCostGelu[3] = {1.1, 1.85, 3.3};
-/// A tile alone on its CU, with nothing beside it to cover its waits (128 x 64:
-/// 4616 x 384 x 384 5.7 us against 5.3 with two 64 x 64 tiles per CU).
-constexpr double kRingCostAlone[3] = {1.3, 2.1, 3.0};
-constexpr double kDmaRow = 0.035;
-constexpr double kDmaRowGelu = 0.043;
-
-struct RingChoice {
-    RingTile tile;
-    int bm;
-    int bn;
-    double cost;
-};
-
-/// The ring kernel's cheapest tile for a problem. Where a CU has few tiles and
-/// K is long, the tile's own loads are all there is to hide behind, and it
-/// takes three stages: 64 x 64 tiles up to two per CU (768 x 3072 on 1576 rows
-/// 24.0 -> 19.3 us; FC2 of 4616 rows, 384 x 1536, two microseconds inside its
-/// forward), 128 x 128 alone on a CU (768 x 3072 on 4616 rows 31 -> 27 us; two
-/// with two stages each beat one at a time with three, 40 against 51 us on 6304
-/// rows). Tiles that are alone on their CUs have loading wavefronts beside the
-/// computing ones (64 x 32 tiles: 197 x 768 x 768 5.3 -> 4.4 us, 197 x 768 x 3072
-/// 11.6 -> 8.5; 64 x 64 from K = 768 on: 197 x 2304 x 768 5.5 -> 4.7; at K = 384
-/// 788 x 1152 lost, 4.7 -> 5.3).
-RingChoice choose_ring(const GemmArgs& args) {
-    constexpr RingTile kTiles[3] = {RingTile::k64x64, RingTile::k128x64, RingTile::k128x128};
-    constexpr int kHeights[3] = {64, 128, 128};
-    constexpr int kWidths[3] = {64, 64, 128};
-    const std::int64_t units = compute_units();
-    RingChoice best{RingTile::k64x64, 64, 64, 0.0};
-    for (int i = 0; i < 3; ++i) {
-        const std::int64_t tiles = tile_count(args, kHeights[i], kWidths[i]);
-        const double cost = tiles <= units ? kRingCostAlone[i]
-                                           : static_cast<double>((tiles + units - 1) / units) *
-                                                 (args.gelu ? kRingCostGelu[i] : kRingCost[i]);
-        if (i == 0 || cost < best.cost) {
-            best = RingChoice{kTiles[i], kHeights[i], kWidths[i], cost};
-            if (i == 0 && tile_count(args, 64, 32) <= units) {
-                best = RingChoice{RingTile::k64x32Alone, 64, 32, cost};
-            } else if (i == 0 && tiles <= units && args.k >= 768) {
-                best.tile = RingTile::k64x64Alone;
-            } else if (i == 0 && tiles <= 2 * units && args.k >= 1024) {
-                best.tile = RingTile::k64x64Deep;
-            } else if (i == 2 && tiles <= units && args.k >= 1024) {
-                best.tile = RingTile::k128x128Deep;
-            }
-        }
-    }
-    return best;
-}
-
 /// The direct-to-LDS kernel (gemm_dma.hpp) for a problem it covers: one batch
 /// entry, B as [N, K], N a multiple of 256, K of at least 256, no addend,
 /// vector A and B, C written in 16-byte pieces, every operand tile within one
 /// descriptor's span, the CUs a multiple of 8 (one persistent workgroup per
-/// CU, eight per XCD) and BM x 256 tiles for at least half the CUs. BM is the
-/// height with the fewest rounds x BM, the rounds as balanced_map's split
-/// gives them (ViT-Base b64: 320 for FC1, 256 for QKV, 192 for FC2 and the
-/// projection). Returns hipErrorNotSupported otherwise, and where the ring
-/// kernel's @p ring_cost is the smaller one.
+/// CU, the same number on every XCD), tiles for at least half the CUs, and no
+/// @p ring tile that is the better choice. Returns hipErrorNotSupported
+/// otherwise.
 hipError_t launch_dma(const std::uint16_t* a, const std::uint16_t* b, const float* bias,
-                      std::uint16_t* c, const GemmArgs& args, double ring_cost, hipStream_t stream) {
+                      std::uint16_t* c, const GemmArgs& args, const RingChoice& ring, hipStream_t stream) {
     const int units = compute_units();
     // Entries run as one problem, each row stored back in its entry: the patch
     // embedding, with its positional addend (the instance that takes entries).
@@ -441,26 +308,8 @@ hipError_t launch_dma(const std::uint16_t* a, const std::uint16_t* b, const floa
     if (!eligible) {
         return hipErrorNotSupported;
     }
-    const int turns = units / 8;
-    int bm = 0;
-    int rounds = 0;
-    gemm::TileMap map{0, 0};
-    for (const int height : {192, 256, 320}) {
-        if (with_addend && height == 320) {
-            continue;  // the addend's registers would spill at 320 rows
-        }
-        if (2 * tile_count(args, height, 256) < units) {
-            continue;  // fewer tiles than half the CUs: the ring kernel
-        }
-        int height_rounds = 0;
-        const gemm::TileMap split = balanced_map(args, height, 256, turns, &height_rounds);
-        if (bm == 0 || height_rounds * height < rounds * bm) {
-            bm = height;
-            rounds = height_rounds;
-            map = split;
-        }
-    }
-    if (bm == 0 || ring_cost < rounds * bm * (args.gelu ? kDmaRowGelu : kDmaRow)) {
+    const DmaChoice choice = choose_dma(args, units);
+    if (ring_beats_dma(args, ring, choice)) {
         return hipErrorNotSupported;
     }
     auto run = [&](auto chosen, std::size_t lds_bytes) -> hipError_t {
@@ -468,7 +317,7 @@ hipError_t launch_dma(const std::uint16_t* a, const std::uint16_t* b, const floa
         if (const hipError_t opted = allow_lds<kernel>(lds_bytes); opted != hipSuccess) {
             return opted;
         }
-        kernel<<<units, 512, lds_bytes, stream>>>(a, b, bias, c, args, map);
+        kernel<<<units, 512, lds_bytes, stream>>>(a, b, bias, c, args, choice.map);
         return hipGetLastError();
     };
     // The epilogue's parts as template flags: bias, GELU, alpha (when not 1),
@@ -499,7 +348,7 @@ hipError_t launch_dma(const std::uint16_t* a, const std::uint16_t* b, const floa
         };
         return bias != nullptr ? with_gelu(std::true_type{}) : with_gelu(std::false_type{});
     };
-    switch (bm) {
+    switch (choice.rows) {
     case 192: return pick(std::integral_constant<int, 192>{});
     case 256: return pick(std::integral_constant<int, 256>{});
     default: return pick(std::integral_constant<int, 320>{});
@@ -525,13 +374,11 @@ hipError_t gemm_bf16(const std::uint16_t* a, const std::uint16_t* b, const float
         vector_operand(b, whole.ldb, whole.k, whole.stride_b, whole.outer_stride_b, split) &&
         static_cast<std::int64_t>(128) * whole.lda * 2 < gemm::kMaxSpan &&
         static_cast<std::int64_t>(128) * whole.ldb * 2 < gemm::kMaxSpan) {
-        const RingChoice ring = choose_ring(whole);
-        if (const hipError_t dma = launch_dma(a, b, bias, c, whole, ring.cost, stream);
-            dma != hipErrorNotSupported) {
+        const RingChoice ring = choose_ring(whole, compute_units());
+        if (const hipError_t dma = launch_dma(a, b, bias, c, whole, ring, stream); dma != hipErrorNotSupported) {
             return dma;
         }
-        const gemm::TileMap map = tile_map(whole, ring.bm, ring.bn, 2);
-        return gemm_ring_bf16(ring.tile, a, b, bias, c, whole, map.px, map.py, vector_c, stream);
+        return gemm_ring_bf16(ring.tile, a, b, bias, c, whole, ring.map, vector_c, stream);
     }
     const std::int64_t units = compute_units();
     if (tile_count(args, 128, 128) >= units * 2) {

@@ -297,17 +297,6 @@ template <typename T, int WM, int WN, int TM, int TN, int BK> struct Shape {
     }
 };
 
-/// Which tile a workgroup computes. With px * py == 8 the tile grid of an
-/// entry is split into px x py blocks and workgroup x goes to block x % 8:
-/// the MI355X dispatcher hands consecutive workgroups to its 8 XCDs in turn,
-/// so each XCD's L2 then serves one block, its A rows and its B columns,
-/// instead of every XCD streaming all of A. With px == 0 the tiles are in
-/// plain row-major order.
-struct TileMap {
-    int px;
-    int py;
-};
-
 /// Start of part @p i of @p n split into @p parts near-equal parts.
 __device__ __forceinline__ int split_point(int n, int parts, int i) { return n * i / parts; }
 

@@ -59,9 +59,8 @@ hipError_t launch(const std::uint16_t* a, const std::uint16_t* b, const float* b
 } // namespace
 
 hipError_t gemm_ring_bf16(RingTile tile, const std::uint16_t* a, const std::uint16_t* b,
-                          const float* bias, std::uint16_t* c, const GemmArgs& args, int px, int py,
-                          bool vector_c, hipStream_t stream) {
-    const gemm::TileMap map{px, py};
+                          const float* bias, std::uint16_t* c, const GemmArgs& args,
+                          const gemm::TileMap& map, bool vector_c, hipStream_t stream) {
     using T = std::uint16_t;
     switch (tile) {
     case RingTile::k64x64: return launch<gemm::RingShape<T, 2, 2, 1, 1, 2>>(a, b, bias, c, args, map, vector_c, stream);

@@ -117,13 +117,28 @@ hipError_t gemm_f32(const float* a, const float* b, const float* bias, float* c,
 hipError_t gemm_bf16(const std::uint16_t* a, const std::uint16_t* b, const float* bias,
                      std::uint16_t* c, const GemmArgs& args, hipStream_t stream);
 
+namespace gemm {
+
+/// Which tile a workgroup computes. With px * py == 8 the tile grid of an
+/// entry is split into px x py blocks and workgroup x goes to block x % 8:
+/// the MI355X dispatcher hands consecutive workgroups to its 8 XCDs in turn,
+/// so each XCD's L2 then serves one block, its A rows and its B columns,
+/// instead of every XCD streaming all of A. With px == 0 the tiles are in
+/// plain row-major order.
+struct TileMap {
+    int px;
+    int py;
+};
+
+} // namespace gemm
+
 /// gemm_ring.hip: the bf16 LDS-ring kernel on one of its tiles, for a problem
-/// gemm.hip found to fit it. px x py is the tile grid's split over the XCDs
-/// (0: none); @p vector_c tells that C may be stored in 16-byte pieces.
+/// gemm.hip found to fit it. @p vector_c tells that C may be stored in 16-byte
+/// pieces.
 enum class RingTile { k64x32Alone, k64x64, k64x64Alone, k64x64Deep, k128x64, k128x128, k128x128Deep };
 hipError_t gemm_ring_bf16(RingTile tile, const std::uint16_t* a, const std::uint16_t* b,
-                          const float* bias, std::uint16_t* c, const GemmArgs& args, int px, int py,
-                          bool vector_c, hipStream_t stream);
+                          const float* bias, std::uint16_t* c, const GemmArgs& args,
+                          const gemm::TileMap& map, bool vector_c, hipStream_t stream);
 /// Its fp32 form.
 enum class RingTileF32 { k32x16Alone, k32x32, k32x32Deep, k64x32, k64x64 };
 hipError_t gemm_ring_f32(RingTileF32 tile, const float* a, const float* b, const float* bias, float* c,

@@ -1,0 +1,53 @@
+"""Which kernel and tile a bf16 or fp32 product takes (gemm_choice.hpp), on the
+256 compute units of an MI355X."""
+
+from __future__ import annotations
+
+import ctypes
+import subprocess
+from pathlib import Path
+
+import pytest
+
+from conftest import ROOT
+
+UNITS = 256
+RING = ["64x32 alone", "64x64", "64x64 alone", "64x64 deep", "128x64", "128x128", "128x128 deep"]
+
+
+@pytest.fixture(scope="module")
+def rules():
+    library = Path(ROOT) / "tests" / "cpp" / "bin" / "libinternals.so"
+    if not library.exists():
+        subprocess.run(["make", "-s", "-C", str(library.parents[1])], check=True)
+    return ctypes.CDLL(str(library))
+
+
+def bf16(rules, m, n, k, gelu=False, count=1, persistent_fits=None):
+    fits = n % 256 == 0 and k >= 256 and count == 1 if persistent_fits is None else persistent_fits
+    choice = rules.bf16_choice(m, n, k, count, int(gelu), int(fits), UNITS)
+    return RING[choice] if choice < 100 else f"persistent {choice - 100}"
+
+
+@pytest.mark.parametrize("m,n,k,gelu,expected", [
+    # 63 of an XCD's 64 slots: 15.8 to 22.8 us by card on 128 x 128 tiles.
+    (3152, 2304, 768, False, "persistent 192"),
+    # 70 tiles for the 64 slots of one XCD, though 500 for 512 over the chip: 28.1 against 24.4 us.
+    (3200, 2560, 640, True, "persistent 192"),
+    (3152, 2560, 640, True, "persistent 192"),
+    # Three rounds: 24 to 32 us by where the operands come from, against 21 to 24.
+    (4616, 2304, 768, False, "persistent 256"),
+    # 60 and 54 of 64 slots: the ring, 14.0 against 17.4 and 16.6 against 21.3 us.
+    (4616, 1536, 384, True, "128x128"),
+    (8224, 768, 768, False, "128x128"),
+    # Short K: the ring only by more.
+    (9232, 768, 256, False, "persistent 192"),
+    (6304, 1024, 256, True, "128x128"),
+    # 128 x 64 tiles would fill every CU but leave none over.
+    (394, 4096, 1024, True, "64x64 deep"),
+    (12608, 3072, 768, True, "persistent 320"),
+    (12608, 2304, 768, False, "persistent 256"),
+    (12608, 768, 3072, False, "persistent 192"),
+])
+def test_ring_or_persistent(rules, m, n, k, gelu, expected):
+    assert bf16(rules, m, n, k, gelu) == expected
