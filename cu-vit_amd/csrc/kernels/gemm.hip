@@ -26,8 +26,6 @@ namespace {
 using cuvit::device::aligned16;
 using gemm::Shape;
 
-constexpr int kMaxGridY = 65535;
-
 /// True when every row of an operand starts on a 16-byte boundary and rows
 /// of @p depth elements (the vector direction) hold whole 16-byte chunks.
 template <typename T>

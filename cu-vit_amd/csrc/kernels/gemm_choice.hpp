@@ -13,6 +13,24 @@ namespace cuvit::detail {
 /// Dispatch order puts workgroup x on XCD x % 8.
 constexpr int kXcds = 8;
 
+/// A grid's y extent, over which batch entries are spread.
+constexpr int kMaxGridY = 65535;
+
+/// Runs launch(first, entries) over a batch of @p count entries, as many at a
+/// time as a grid takes, up to the first that fails. (`first` steps past
+/// INT_MAX behind the last entries of the largest batches.)
+template <typename Launch> hipError_t for_entries(int count, Launch&& launch) {
+    for (std::int64_t first = 0; first < count; first += kMaxGridY) {
+        const std::int64_t left = count - first;
+        const hipError_t launched =
+            launch(static_cast<int>(first), static_cast<int>(left < kMaxGridY ? left : kMaxGridY));
+        if (launched != hipSuccess) {
+            return launched;
+        }
+    }
+    return hipSuccess;
+}
+
 inline std::int64_t tile_count(const GemmArgs& args, int bm, int bn) {
     return static_cast<std::int64_t>((args.m + bm - 1) / bm) * ((args.n + bn - 1) / bn) * args.count;
 }

@@ -1,11 +1,10 @@
 // Launch of the LDS-ring GEMM (gemm_ring.hpp): its instances, one translation
 // unit of their own.
+#include "gemm_choice.hpp"
 #include "gemm_ring.hpp"
 
 namespace cuvit::detail {
 namespace {
-
-constexpr int kMaxGridY = 65535;
 
 /// Launches @p Kernel over the tile grid, one workgroup per tile (per slot of
 /// the largest XCD block with a split) and batch entry.
@@ -23,16 +22,11 @@ hipError_t run_tiles(const T* a, const T* b, const float* bias, T* c, const Gemm
     if (const hipError_t opted = allow_lds<Kernel>(S::kLdsBytes); opted != hipSuccess) {
         return opted;
     }
-    // A grid's y extent is limited: more entries than that take several launches.
-    for (int first = 0; first < args.count; first += kMaxGridY) {
-        const int entries = args.count - first < kMaxGridY ? args.count - first : kMaxGridY;
+    return for_entries(args.count, [&](int first, int entries) -> hipError_t {
         const dim3 grid(static_cast<unsigned int>(tiles), static_cast<unsigned int>(entries));
         Kernel<<<grid, S::kThreads, S::kLdsBytes, stream>>>(a, b, bias, c, args, map, vector_c, first);
-        if (const hipError_t launched = hipGetLastError(); launched != hipSuccess) {
-            return launched;
-        }
-    }
-    return hipSuccess;
+        return hipGetLastError();
+    });
 }
 
 template <typename S>

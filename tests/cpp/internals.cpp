@@ -1,6 +1,6 @@
 // Internals for the Python tests: the GEMM dispatch rules (gemm_choice.hpp) for
 // test_gemm_choice_cpu.py, which kernel and tile a problem takes on a card of
-// `units` compute units.
+// `units` compute units, and how a batch is spread over launches.
 #include "kernels/gemm_choice.hpp"
 
 using namespace cuvit::detail;
@@ -35,5 +35,21 @@ int bf16_choice(int m, int n, int k, int count, int gelu, int persistent_fits, i
         }
     }
     return static_cast<int>(ring.tile);
+}
+
+/// The launches that a batch of @p count entries takes, or -1 if they don't
+/// cover it in order, each within a grid (or are more than they can be).
+int batch_launches(int count) {
+    int launches = 0;
+    long long covered = 0;
+    const hipError_t status = for_entries(count, [&](int first, int entries) -> hipError_t {
+        ++launches;
+        if (first != covered || entries < 1 || entries > kMaxGridY || launches > 40000) {
+            return hipErrorInvalidValue;
+        }
+        covered += entries;
+        return hipSuccess;
+    });
+    return status == hipSuccess && covered == count ? launches : -1;
 }
 }

@@ -51,3 +51,10 @@ def bf16(rules, m, n, k, gelu=False, count=1, persistent_fits=None):
 ])
 def test_ring_or_persistent(rules, m, n, k, gelu, expected):
     assert bf16(rules, m, n, k, gelu) == expected
+
+
+@pytest.mark.parametrize("count,launches", [(1, 1), (65535, 1), (65536, 2), (2 ** 31 - 65537, 32768),
+                                            (2 ** 31 - 65536, 32768), (2 ** 31 - 1, 32769)])
+def test_large_batches_end(rules, count, launches):
+    """Also where the last first entry plus a grid's extent is past an int."""
+    assert rules.batch_launches(count) == launches
