@@ -364,6 +364,7 @@ hipError_t gemm_bf16(const std::uint16_t* a, const std::uint16_t* b, const float
     const bool split = whole.inner > 0;
     const bool vector_c = aligned16(c) && whole.n % 8 == 0 && whole.ldc % 8 == 0 && whole.stride_c % 8 == 0 &&
                           (!split || whole.outer_stride_c % 8 == 0);
+    const int c_run = vector_c ? 8 : whole.n % 4 == 0 && vector_output(c, whole) ? 4 : 1;
     const bool addend_ok = whole.addend == nullptr ||
                            (vector_c && bias != nullptr && !whole.gelu && !whole.accumulate &&
                             aligned16(whole.addend) && whole.ld_addend % 4 == 0);
@@ -376,7 +377,7 @@ hipError_t gemm_bf16(const std::uint16_t* a, const std::uint16_t* b, const float
         if (const hipError_t dma = launch_dma(a, b, bias, c, whole, ring, stream); dma != hipErrorNotSupported) {
             return dma;
         }
-        return gemm_ring_bf16(ring.tile, a, b, bias, c, whole, ring.map, vector_c, stream);
+        return gemm_ring_bf16(ring.tile, a, b, bias, c, whole, ring.map, c_run, stream);
     }
     const std::int64_t units = compute_units();
     if (tile_count(args, 128, 128) >= units * 2) {

@@ -10,7 +10,7 @@ namespace {
 /// the largest XCD block with a split) and batch entry.
 template <typename S, auto Kernel, typename T>
 hipError_t run_tiles(const T* a, const T* b, const float* bias, T* c, const GemmArgs& args,
-                     const gemm::TileMap& map, bool vector_c, hipStream_t stream) {
+                     const gemm::TileMap& map, int c_run, hipStream_t stream) {
     const std::int64_t tiles_m = (args.m + S::kBM - 1) / S::kBM;
     const std::int64_t tiles_n = (args.n + S::kBN - 1) / S::kBN;
     const std::int64_t tiles = map.px > 0 ? 8 * ((tiles_m + map.px - 1) / map.px) *
@@ -24,16 +24,16 @@ hipError_t run_tiles(const T* a, const T* b, const float* bias, T* c, const Gemm
     }
     return for_entries(args.count, [&](int first, int entries) -> hipError_t {
         const dim3 grid(static_cast<unsigned int>(tiles), static_cast<unsigned int>(entries));
-        Kernel<<<grid, S::kThreads, S::kLdsBytes, stream>>>(a, b, bias, c, args, map, vector_c, first);
+        Kernel<<<grid, S::kThreads, S::kLdsBytes, stream>>>(a, b, bias, c, args, map, c_run, first);
         return hipGetLastError();
     });
 }
 
 template <typename S>
 hipError_t launch(const std::uint16_t* a, const std::uint16_t* b, const float* bias, std::uint16_t* c,
-                  const GemmArgs& args, const gemm::TileMap& map, bool vector_c, hipStream_t stream) {
+                  const GemmArgs& args, const gemm::TileMap& map, int c_run, hipStream_t stream) {
     auto run = [&](auto kernel) -> hipError_t {
-        return run_tiles<S, decltype(kernel)::kValue>(a, b, bias, c, args, map, vector_c, stream);
+        return run_tiles<S, decltype(kernel)::kValue>(a, b, bias, c, args, map, c_run, stream);
     };
     if (args.addend != nullptr) {
         return run(KernelConstant<gemm::gemm_ring_kernel<S, true, false, false, true>>{});
@@ -54,21 +54,21 @@ hipError_t launch(const std::uint16_t* a, const std::uint16_t* b, const float* b
 
 hipError_t gemm_ring_bf16(RingTile tile, const std::uint16_t* a, const std::uint16_t* b,
                           const float* bias, std::uint16_t* c, const GemmArgs& args,
-                          const gemm::TileMap& map, bool vector_c, hipStream_t stream) {
+                          const gemm::TileMap& map, int c_run, hipStream_t stream) {
     using T = std::uint16_t;
     switch (tile) {
-    case RingTile::k64x64: return launch<gemm::RingShape<T, 2, 2, 1, 1, 2>>(a, b, bias, c, args, map, vector_c, stream);
+    case RingTile::k64x64: return launch<gemm::RingShape<T, 2, 2, 1, 1, 2>>(a, b, bias, c, args, map, c_run, stream);
     case RingTile::k64x32Alone:
-        return launch<gemm::RingShape<T, 2, 1, 1, 1, 4, true, true>>(a, b, bias, c, args, map, vector_c, stream);
+        return launch<gemm::RingShape<T, 2, 1, 1, 1, 4, true, true>>(a, b, bias, c, args, map, c_run, stream);
     case RingTile::k64x64Alone:
-        return launch<gemm::RingShape<T, 2, 2, 1, 1, 3, true, true>>(a, b, bias, c, args, map, vector_c, stream);
+        return launch<gemm::RingShape<T, 2, 2, 1, 1, 3, true, true>>(a, b, bias, c, args, map, c_run, stream);
     case RingTile::k64x64Deep:
-        return launch<gemm::RingShape<T, 2, 2, 1, 1, 3, true>>(a, b, bias, c, args, map, vector_c, stream);
+        return launch<gemm::RingShape<T, 2, 2, 1, 1, 3, true>>(a, b, bias, c, args, map, c_run, stream);
     case RingTile::k128x64:
-        return launch<gemm::RingShape<T, 4, 2, 1, 1, 2>>(a, b, bias, c, args, map, vector_c, stream);
+        return launch<gemm::RingShape<T, 4, 2, 1, 1, 2>>(a, b, bias, c, args, map, c_run, stream);
     case RingTile::k128x128:
-        return launch<gemm::RingShape<T, 4, 2, 1, 2, 2>>(a, b, bias, c, args, map, vector_c, stream);
-    default: return launch<gemm::RingShape<T, 4, 2, 1, 2, 3>>(a, b, bias, c, args, map, vector_c, stream);
+        return launch<gemm::RingShape<T, 4, 2, 1, 2, 2>>(a, b, bias, c, args, map, c_run, stream);
+    default: return launch<gemm::RingShape<T, 4, 2, 1, 2, 3>>(a, b, bias, c, args, map, c_run, stream);
     }
 }
 
@@ -76,7 +76,7 @@ hipError_t gemm_ring_f32(RingTileF32 tile, const float* a, const float* b, const
                          const GemmArgs& args, hipStream_t stream) {
     auto launch_f32 = [&](auto shape) -> hipError_t {
         using S = decltype(shape);
-        return run_tiles<S, gemm::gemm_ring_f32_kernel<S>>(a, b, bias, c, args, gemm::TileMap{0, 0}, true, stream);
+        return run_tiles<S, gemm::gemm_ring_f32_kernel<S>>(a, b, bias, c, args, gemm::TileMap{0, 0}, 4, stream);
     };
     switch (tile) {
     case RingTileF32::k32x16Alone: return launch_f32(gemm::RingShape<float, 2, 1, 1, 1, 3, true, true>{});

@@ -319,15 +319,16 @@ __device__ __forceinline__ void ring_multiply(const RingLoads<T, S>& loads, cons
 
 /// The epilogue's parts as in gemm_dma_kernel (alpha is always multiplied in:
 /// 1 * x is x, bit for bit). Batch entry @p first_entry + blockIdx.y; with
-/// args.rows_per_entry > 0 the rows are entries run as one problem. Without
-/// @p vector_c C's rows are not 16-byte aligned or N is no multiple of 8, and
-/// its elements are read and written one by one.
+/// args.rows_per_entry > 0 the rows are entries run as one problem. @p c_run of
+/// C's elements are read and written at once: 8, 4 where N and its rows are
+/// whole 8-byte pieces only (6304 x 2308 x 768 accumulating 72 -> 41 us against
+/// one by one, 196 x 196 x 64 in 96 entries 18.4 -> 9.4), else 1.
 template <typename S, bool kBias, bool kGelu, bool kAccumulate, bool kAddend = false>
 __global__ __launch_bounds__(S::kThreads) void gemm_ring_kernel(const std::uint16_t* __restrict__ a,
                                                                 const std::uint16_t* __restrict__ b,
                                                                 const float* __restrict__ bias,
                                                                 std::uint16_t* c, GemmArgs args,
-                                                                TileMap map, bool vector_c, int first_entry) {
+                                                                TileMap map, int c_run, int first_entry) {
     constexpr int BM = S::kBM;
     constexpr int BN = S::kBN;
     constexpr int TM = S::kTM;
@@ -381,7 +382,16 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring_kernel(const std::uint1
                 old_rows[i][k] = Vec16{{0U, 0U, 0U, 0U}};
                 if (row < args.m && store_col < args.n) {
                     const std::uint16_t* const from = c + c_offset(row) + store_col;
-                    old_rows[i][k] = vector_c ? load16(from) : load_chunk_scalar(from, 0, 0, 1, 0, args.n - store_col);
+                    if (c_run == 8) {
+                        old_rows[i][k] = load16(from);
+                    } else if (c_run == 4) {
+                        const uint2 first = *reinterpret_cast<const uint2*>(from);
+                        const uint2 second =
+                            store_col + 4 < args.n ? *reinterpret_cast<const uint2*>(from + 4) : make_uint2(0U, 0U);
+                        old_rows[i][k] = Vec16{{first.x, first.y, second.x, second.y}};
+                    } else {
+                        old_rows[i][k] = load_chunk_scalar(from, 0, 0, 1, 0, args.n - store_col);
+                    }
                 }
             }
     }
@@ -461,8 +471,13 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring_kernel(const std::uint1
             const Vec16 v = *reinterpret_cast<const Vec16*>(staged(kRowsPerStore * k + store_row, store_chunk));
             if (out_row < args.m && store_col < args.n) {
                 std::uint16_t* const to = c + c_offset(out_row) + store_col;
-                if (vector_c) {
+                if (c_run == 8) {
                     store16(to, v);
+                } else if (c_run == 4) {
+                    *reinterpret_cast<uint2*>(to) = make_uint2(v.w[0], v.w[1]);
+                    if (store_col + 4 < args.n) {
+                        *reinterpret_cast<uint2*>(to + 4) = make_uint2(v.w[2], v.w[3]);
+                    }
                 } else {
 #pragma unroll
                     for (int e = 0; e < 8; ++e) {
@@ -484,7 +499,7 @@ template <typename S>
 __global__ __launch_bounds__(S::kThreads) void gemm_ring_f32_kernel(const float* __restrict__ a,
                                                                     const float* __restrict__ b,
                                                                     const float* __restrict__ bias, float* c,
-                                                                    GemmArgs args, TileMap map, bool /* four at once: always */,
+                                                                    GemmArgs args, TileMap map, int /* c_run: always 4 */,
                                                                     int first_entry) {
     constexpr int TM = S::kTM;
     constexpr int TN = S::kTN;

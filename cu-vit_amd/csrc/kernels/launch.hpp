@@ -133,12 +133,12 @@ struct TileMap {
 } // namespace gemm
 
 /// gemm_ring.hip: the bf16 LDS-ring kernel on one of its tiles, for a problem
-/// gemm.hip found to fit it. @p vector_c tells that C may be stored in 16-byte
-/// pieces.
+/// gemm.hip found to fit it. @p c_run is how many of C's elements are stored at
+/// once: 8, 4 or 1.
 enum class RingTile { k64x32Alone, k64x64, k64x64Alone, k64x64Deep, k128x64, k128x128, k128x128Deep };
 hipError_t gemm_ring_bf16(RingTile tile, const std::uint16_t* a, const std::uint16_t* b,
                           const float* bias, std::uint16_t* c, const GemmArgs& args,
-                          const gemm::TileMap& map, bool vector_c, hipStream_t stream);
+                          const gemm::TileMap& map, int c_run, hipStream_t stream);
 /// Its fp32 form.
 enum class RingTileF32 { k32x16Alone, k32x32, k32x32Deep, k64x32, k64x64 };
 hipError_t gemm_ring_f32(RingTileF32 tile, const float* a, const float* b, const float* bias, float* c,

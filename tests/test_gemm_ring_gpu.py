@@ -34,6 +34,9 @@ CASES = [
     (63, 64, 64, True, True, False, 1.0, 0),          # a row short of a tile
     (65, 72, 136, True, False, True, 1.0, 8),         # a row and a chunk past; K past one span
     (64, 65, 128, True, False, True, 1.0, 0),         # odd N: element-wise C, accumulating
+    (65, 76, 136, True, False, True, 1.0, 0),         # C in 8-byte pieces, accumulating, half a chunk at N
+    (130, 132, 72, True, True, False, 1.0, 4),        # the same, padded rows
+    (4616, 1540, 384, True, False, True, 1.0, 0),     # the same on 128 x 128 tiles
     (130, 199, 72, False, True, False, -0.5, 3),      # odd rows of C, GELU without bias, alpha
     (197, 768, 3080, True, False, True, 1.0, 0),      # tiles alone on their CUs, long K
     (65, 2304, 128, True, True, True, 1.0, 0),        # the same at one span of K
