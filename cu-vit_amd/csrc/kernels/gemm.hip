@@ -199,40 +199,6 @@ hipError_t launch_panel(const float* a, const float* b, const float* bias, float
     return bias != nullptr ? with_gelu(std::true_type{}) : with_gelu(std::false_type{});
 }
 
-/// The fp32 ring kernel's tile for a problem, by relative times of a CU's row
-/// of tiles fitted to MI355X at K = 768 (us: 32 x 32 3.8, 64 x 32 6.9, 64 x 64
-/// 13.7 each, more for a tile alone on its CU; these are MFMA-bound, so larger
-/// tiles gain little and lose it to a last row of tiles that is not full).
-/// Three stages for 32 x 32 tiles where few of them share a CU or K is long
-/// (1576 x 192 x 768 14.3 -> 11.3 us, 394 x 768 x 3072 47 -> 35), two elsewhere
-/// (788 x 768 x 768: 13.7 against 14.3). While 32 x 16 tiles are alone on their
-/// CUs, those, with loading wavefronts beside the computing ones (197 x 192 x
-/// 768 7.6 -> 6.6, 197 x 576 x 192 4.0 -> 3.6).
-RingTileF32 choose_ring_f32(const GemmArgs& args) {
-    constexpr RingTileF32 kTiles[3] = {RingTileF32::k32x32, RingTileF32::k64x32, RingTileF32::k64x64};
-    constexpr int kHeights[3] = {32, 64, 64};
-    constexpr int kWidths[3] = {32, 32, 64};
-    constexpr double kCost[3] = {1.0, 1.8, 3.56};
-    constexpr double kAlone[3] = {1.5, 2.45, 4.0};
-    const std::int64_t units = compute_units();
-    if (tile_count(args, 32, 16) <= units) {
-        return RingTileF32::k32x16Alone;
-    }
-    RingTileF32 best = RingTileF32::k32x32;
-    double best_cost = 0.0;
-    for (int i = 0; i < 3; ++i) {
-        const std::int64_t tiles = tile_count(args, kHeights[i], kWidths[i]);
-        const double cost =
-            tiles <= units ? kAlone[i] : static_cast<double>((tiles + units - 1) / units) * kCost[i];
-        if (i == 0 || cost < best_cost) {
-            const bool deep = i == 0 && ((tiles <= 2 * units && args.k >= 512) || args.k >= 1024);
-            best = deep ? RingTileF32::k32x32Deep : kTiles[i];
-            best_cost = cost;
-        }
-    }
-    return best;
-}
-
 hipError_t gemm_f32(const float* a, const float* b, const float* bias, float* c,
                     const GemmArgs& args, hipStream_t stream) {
     // Tall single products with B as [N, K] (the model's linear layers): the
@@ -268,7 +234,8 @@ hipError_t gemm_f32(const float* a, const float* b, const float* bias, float* c,
         vector_operand(b, whole.ldb, whole.k, whole.stride_b, whole.outer_stride_b, split) &&
         static_cast<std::int64_t>(64) * whole.lda * 4 < gemm::kMaxSpan &&
         static_cast<std::int64_t>(64) * whole.ldb * 4 < gemm::kMaxSpan) {
-        return gemm_ring_f32(choose_ring_f32(whole), a, b, bias, c, whole, stream);
+        const RingChoiceF32 ring = choose_ring_f32(whole, compute_units());
+        return gemm_ring_f32(ring.tile, a, b, bias, c, whole, ring.map, stream);
     }
     if (tile_count(args, 32, 32) > static_cast<std::int64_t>(compute_units()) * 32) {
         return pick_flags<float, 2, 2, 2, 2, 32>(a, b, bias, c, args, stream);

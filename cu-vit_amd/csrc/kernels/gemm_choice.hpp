@@ -13,8 +13,9 @@ namespace cuvit::detail {
 /// Dispatch order puts workgroup x on XCD x % 8.
 constexpr int kXcds = 8;
 
-/// A grid's y extent, over which batch entries are spread.
-constexpr int kMaxGridY = 65535;
+/// Batch entries of one launch: within a grid's y extent (65535), and a multiple
+/// of the XCDs, over which entries are spread.
+constexpr int kMaxGridY = 65528;
 
 /// Runs launch(first, entries) over a batch of @p count entries, as many at a
 /// time as a grid takes, up to the first that fails. (`first` steps past
@@ -69,10 +70,26 @@ inline gemm::TileMap tile_map(const GemmArgs& args, int bm, int bn, std::size_t 
     return map;
 }
 
+/// Whether a batch of @p tiles tiles an entry has its entries dealt to the XCDs
+/// whole (TileMap, px < 0), so that each operand is read into one L2 only and
+/// lines of C that two tiles share are merged there: where no XCD gets more
+/// than a tenth above its share. Entries spread over all XCDs against this, us:
+/// bf16 577 x 168 x 384 in 192 entries 63 -> 43, 295 x 296 x 768 in 256 134 ->
+/// 77, fp32 196 x 200 x 384 in 192 118 -> 75; against it, 9 entries for 8 XCDs:
+/// fp32 562 x 128 x 768 12 -> 15.
+inline bool entries_by_xcd(int count, std::int64_t tiles) {
+    const std::int64_t dealt = (static_cast<std::int64_t>(count) + kXcds - 1) / kXcds * kXcds;
+    // (The launch's grid within 31 bits.)
+    return count > 1 && tiles < 16384 && 10 * (dealt - count) <= count;
+}
+
 /// Tiles of the XCD that @p map gives the most, over all batch entries.
 inline std::int64_t largest_share(const GemmArgs& args, const gemm::TileMap& map, int bm, int bn) {
     const std::int64_t tiles_m = (args.m + bm - 1) / bm;
     const std::int64_t tiles_n = (args.n + bn - 1) / bn;
+    if (map.px < 0) {
+        return tiles_m * tiles_n * ((static_cast<std::int64_t>(args.count) + kXcds - 1) / kXcds);
+    }
     if (map.px == 0) {
         return (tiles_m * tiles_n * args.count + kXcds - 1) / kXcds;
     }
@@ -145,6 +162,14 @@ constexpr double kFullRound = 1.15;
 constexpr double kRingMargin = 0.9;
 constexpr double kRingMarginShortK = 0.85;
 
+/// The ring kernel's XCD split: tile_map's where an entry has tiles enough for
+/// one, else whole entries where they divide evenly.
+inline gemm::TileMap ring_map(const GemmArgs& args, int bm, int bn, std::size_t element) {
+    const gemm::TileMap map = tile_map(args, bm, bn, element);
+    const std::int64_t tiles = static_cast<std::int64_t>((args.m + bm - 1) / bm) * ((args.n + bn - 1) / bn);
+    return map.px == 0 && entries_by_xcd(args.count, tiles) ? gemm::TileMap{-1, -1} : map;
+}
+
 struct RingChoice {
     RingTile tile;
     int bm;
@@ -171,7 +196,7 @@ inline RingChoice choose_ring(const GemmArgs& args, int units) {
     RingChoice best{RingTile::k64x64, 64, 64, {0, 0}, 0.0};
     for (int i = 0; i < 3; ++i) {
         const std::int64_t tiles = tile_count(args, kHeights[i], kWidths[i]);
-        const gemm::TileMap map = tile_map(args, kHeights[i], kWidths[i], 2);
+        const gemm::TileMap map = ring_map(args, kHeights[i], kWidths[i], 2);
         const std::int64_t share = largest_share(args, map, kHeights[i], kWidths[i]);
         const std::int64_t rounds = (share + slots - 1) / slots;
         double cost = rounds <= 1 ? kRingCostAlone[i]
@@ -182,7 +207,7 @@ inline RingChoice choose_ring(const GemmArgs& args, int units) {
         if (i == 0 || cost < best.cost) {
             best = RingChoice{kTiles[i], kHeights[i], kWidths[i], map, cost};
             if (i == 0 && tile_count(args, 64, 32) <= units) {
-                best = RingChoice{RingTile::k64x32Alone, 64, 32, tile_map(args, 64, 32, 2), cost};
+                best = RingChoice{RingTile::k64x32Alone, 64, 32, ring_map(args, 64, 32, 2), cost};
             } else if (i == 0 && tiles <= units && args.k >= 768) {
                 best.tile = RingTile::k64x64Alone;
             } else if (i == 0 && tiles <= 2 * units && args.k >= 1024) {
@@ -230,6 +255,49 @@ inline DmaChoice choose_dma(const GemmArgs& args, int units) {
 /// Whether the ring kernel takes a problem that the persistent one could.
 inline bool ring_beats_dma(const GemmArgs& args, const RingChoice& ring, const DmaChoice& dma) {
     return dma.rows == 0 || ring.cost < dma.cost * (args.k < 384 ? kRingMarginShortK : kRingMargin);
+}
+
+struct RingChoiceF32 {
+    RingTileF32 tile;
+    gemm::TileMap map;
+};
+
+/// The fp32 ring kernel's tile for a problem, by relative times of a CU's row
+/// of tiles fitted to MI355X at K = 768 (us: 32 x 32 3.8, 64 x 32 6.9, 64 x 64
+/// 13.7 each, more for a tile alone on its CU; these are MFMA-bound, so larger
+/// tiles gain little and lose it to a last row of tiles that is not full).
+/// While 32 x 16 tiles are alone on their CUs, those, with loading wavefronts
+/// beside the computing ones (197 x 192 x 768 7.6 -> 6.6, 197 x 576 x 192 4.0 ->
+/// 3.6).
+/// Three stages for 32 x 32 tiles where few of them share a CU or K is long
+/// (1576 x 192 x 768 14.3 -> 11.3 us, 394 x 768 x 3072 47 -> 35), two elsewhere
+/// (788 x 768 x 768: 13.7 against 14.3).
+inline RingChoiceF32 choose_ring_f32(const GemmArgs& args, int units) {
+    constexpr RingTileF32 kTiles[3] = {RingTileF32::k32x32, RingTileF32::k64x32, RingTileF32::k64x64};
+    constexpr int kHeights[3] = {32, 64, 64};
+    constexpr int kWidths[3] = {32, 32, 64};
+    constexpr double kCost[3] = {1.0, 1.8, 3.56};
+    constexpr double kAlone[3] = {1.5, 2.45, 4.0};
+    if (tile_count(args, 32, 16) <= units) {
+        return {RingTileF32::k32x16Alone, ring_map(args, 32, 16, 4)};
+    }
+    const std::int64_t slots = units >= kXcds ? units / kXcds : 1;  // CUs of an XCD
+    const gemm::TileMap map = ring_map(args, 32, 32, 4);
+    const std::int64_t small_rounds = (largest_share(args, map, 32, 32) + slots - 1) / slots;
+    RingChoiceF32 best{RingTileF32::k32x32, map};
+    double best_cost = 0.0;
+    for (int i = 0; i < 3; ++i) {
+        const std::int64_t rounds = (largest_share(args, map, kHeights[i], kWidths[i]) + slots - 1) / slots;
+        const double cost = rounds <= 1 ? kAlone[i] : static_cast<double>(rounds) * kCost[i];
+        if (i == 0 || cost < best_cost) {
+            best.tile = kTiles[i];
+            best_cost = cost;
+        }
+    }
+    if (best.tile == RingTileF32::k32x32 && (args.k >= 1024 || (args.k >= 512 && small_rounds <= 2))) {
+        best.tile = RingTileF32::k32x32Deep;
+    }
+    return best;
 }
 
 } // namespace cuvit::detail

@@ -23,7 +23,8 @@ hipError_t run_tiles(const T* a, const T* b, const float* bias, T* c, const Gemm
         return opted;
     }
     return for_entries(args.count, [&](int first, int entries) -> hipError_t {
-        const dim3 grid(static_cast<unsigned int>(tiles), static_cast<unsigned int>(entries));
+        const dim3 grid = map.px < 0 ? dim3(static_cast<unsigned int>((entries + 7) / 8 * 8 * tiles))
+                                     : dim3(static_cast<unsigned int>(tiles), static_cast<unsigned int>(entries));
         Kernel<<<grid, S::kThreads, S::kLdsBytes, stream>>>(a, b, bias, c, args, map, c_run, first);
         return hipGetLastError();
     });
@@ -73,10 +74,10 @@ hipError_t gemm_ring_bf16(RingTile tile, const std::uint16_t* a, const std::uint
 }
 
 hipError_t gemm_ring_f32(RingTileF32 tile, const float* a, const float* b, const float* bias, float* c,
-                         const GemmArgs& args, hipStream_t stream) {
+                         const GemmArgs& args, const gemm::TileMap& map, hipStream_t stream) {
     auto launch_f32 = [&](auto shape) -> hipError_t {
         using S = decltype(shape);
-        return run_tiles<S, gemm::gemm_ring_f32_kernel<S>>(a, b, bias, c, args, gemm::TileMap{0, 0}, 4, stream);
+        return run_tiles<S, gemm::gemm_ring_f32_kernel<S>>(a, b, bias, c, args, map, 4, stream);
     };
     switch (tile) {
     case RingTileF32::k32x16Alone: return launch_f32(gemm::RingShape<float, 2, 1, 1, 1, 3, true, true>{});

@@ -92,13 +92,27 @@ struct RingShape {
     __device__ __forceinline__ static int place(int row, int chunk) { return chunk ^ ((row >> 1) & 7); }
 };
 
-/// The tile of workgroup blockIdx.x, or false where its XCD's block of the
-/// tile grid (TileMap) has fewer tiles than the grid allows.
+/// The batch entry and tile of a workgroup, or false where its XCD's block of
+/// the tile grid (TileMap) has fewer tiles than the grid allows.
 template <typename S>
-__device__ __forceinline__ bool ring_tile(const GemmArgs& args, const TileMap& map, int& row0, int& col0) {
+__device__ __forceinline__ bool ring_tile(const GemmArgs& args, const TileMap& map, int& entry, int& row0, int& col0) {
     const int tiles_n = (args.n + S::kBN - 1) / S::kBN;
-    int tile_m = static_cast<int>(blockIdx.x) / tiles_n;
-    int tile_n = static_cast<int>(blockIdx.x) % tiles_n;
+    int tile = static_cast<int>(blockIdx.x);
+    if (map.px < 0) {
+        // Whole entries to an XCD: entry e's tiles on XCD e % 8.
+        const int tiles = (args.m + S::kBM - 1) / S::kBM * tiles_n;
+        const int slot = tile >> 3;
+        const int turn = slot / tiles;
+        entry += 8 * turn + (tile & 7);
+        tile = slot - turn * tiles;
+        if (entry >= args.count) {
+            return false;
+        }
+    } else {
+        entry += static_cast<int>(blockIdx.y);
+    }
+    int tile_m = tile / tiles_n;
+    int tile_n = tile - tile_m * tiles_n;
     if (map.px > 0) {
         const int tiles_m = (args.m + S::kBM - 1) / S::kBM;
         // px py = 8, both powers of two: the split points as shifts, since a
@@ -333,10 +347,6 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring_kernel(const std::uint1
     constexpr int BN = S::kBN;
     constexpr int TM = S::kTM;
     constexpr int TN = S::kTN;
-    const Offsets entry = entry_offsets(args, first_entry + static_cast<int>(blockIdx.y));
-    a += entry.a;
-    b += entry.b;
-    c += entry.c;
     extern __shared__ Vec16 lds_vectors[];
     unsigned char* const lds = reinterpret_cast<unsigned char*>(lds_vectors);
     const unsigned int lds_base = __builtin_amdgcn_readfirstlane(lds_address(lds));
@@ -349,9 +359,13 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring_kernel(const std::uint1
     const int wave_n = wave % S::kWN;
 
     int row0, col0;
-    if (!ring_tile<S>(args, map, row0, col0)) {
+    if (!ring_tile<S>(args, map, first_entry, row0, col0)) {
         return; // the whole workgroup, before any barrier
     }
+    const Offsets entry = entry_offsets(args, first_entry);
+    a += entry.a;
+    b += entry.b;
+    c += entry.c;
 
     // Old C, one 16-byte piece per lane and row group, issued ahead of the
     // stage loads (so older than they are in every wait below).
@@ -504,7 +518,6 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring_f32_kernel(const float*
     constexpr int TM = S::kTM;
     constexpr int TN = S::kTN;
     constexpr int E = S::kEdge;
-    const Offsets entry = entry_offsets(args, first_entry + static_cast<int>(blockIdx.y));
     extern __shared__ Vec16 lds_vectors[];
     unsigned char* const lds = reinterpret_cast<unsigned char*>(lds_vectors);
     const unsigned int lds_base = __builtin_amdgcn_readfirstlane(lds_address(lds));
@@ -515,9 +528,10 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring_f32_kernel(const float*
     const int wave_m = wave / S::kWN;
     const int wave_n = wave % S::kWN;
     int row0, col0;
-    if (!ring_tile<S>(args, map, row0, col0)) {
+    if (!ring_tile<S>(args, map, first_entry, row0, col0)) {
         return; // the whole workgroup, before any barrier
     }
+    const Offsets entry = entry_offsets(args, first_entry);
 
     // The epilogue's operands ahead of the stage loads: the bias of this
     // lane's runs and old C.

@@ -124,7 +124,8 @@ namespace gemm {
 /// the MI355X dispatcher hands consecutive workgroups to its 8 XCDs in turn,
 /// so each XCD's L2 then serves one block, its A rows and its B columns,
 /// instead of every XCD streaming all of A. With px == 0 the tiles are in
-/// plain row-major order.
+/// plain row-major order. With px < 0 (the ring kernel's batches) so are an
+/// entry's, and all of entry e's go to XCD e % 8.
 struct TileMap {
     int px;
     int py;
@@ -142,7 +143,7 @@ hipError_t gemm_ring_bf16(RingTile tile, const std::uint16_t* a, const std::uint
 /// Its fp32 form.
 enum class RingTileF32 { k32x16Alone, k32x32, k32x32Deep, k64x32, k64x64 };
 hipError_t gemm_ring_f32(RingTileF32 tile, const float* a, const float* b, const float* bias, float* c,
-                         const GemmArgs& args, hipStream_t stream);
+                         const GemmArgs& args, const gemm::TileMap& map, hipStream_t stream);
 
 /// Fused softmax(Q.K^T / sqrt(head_dim)).V per (image, head) from the packed
 /// [images, tokens, 3, heads, head_dim] projection into [images, tokens,

@@ -37,6 +37,14 @@ int bf16_choice(int m, int n, int k, int count, int gelu, int persistent_fits, i
     return static_cast<int>(ring.tile);
 }
 
+/// A RingTileF32's number.
+int f32_choice(int m, int n, int k, int count, int units) {
+    const GemmArgs args = problem(m, n, k, count, 0);
+    return static_cast<int>(choose_ring_f32(args, units).tile);
+}
+
+int whole_entries(int count, long long tiles) { return entries_by_xcd(count, tiles) ? 1 : 0; }
+
 /// The launches that a batch of @p count entries takes, or -1 if they don't
 /// cover it in order, each within a grid (or are more than they can be).
 int batch_launches(int count) {

@@ -53,8 +53,16 @@ def test_ring_or_persistent(rules, m, n, k, gelu, expected):
     assert bf16(rules, m, n, k, gelu) == expected
 
 
-@pytest.mark.parametrize("count,launches", [(1, 1), (65535, 1), (65536, 2), (2 ** 31 - 65537, 32768),
-                                            (2 ** 31 - 65536, 32768), (2 ** 31 - 1, 32769)])
+@pytest.mark.parametrize("count,whole", [(1, False), (3, False), (8, True), (9, False), (12, False), (24, True),
+                                         (27, False), (72, True), (73, True), (75, True), (192, True),
+                                         (65537, True)])
+def test_entries_go_to_the_xcds_whole_where_they_divide_evenly(rules, count, whole):
+    assert rules.whole_entries(count, 64) == int(whole)
+    assert rules.whole_entries(count, 16384) == 0  # a grid past 31 bits
+
+
+@pytest.mark.parametrize("count,launches", [(1, 1), (65528, 1), (65529, 2), (2 ** 31 - 65529, 32772),
+                                            (2 ** 31 - 65528, 32772), (2 ** 31 - 1, 32773)])
 def test_large_batches_end(rules, count, launches):
     """Also where the last first entry plus a grid's extent is past an int."""
     assert rules.batch_launches(count) == launches

@@ -86,10 +86,11 @@ def test_ring_equals_the_tiled_kernel(cuvit, device, m, n, k, with_bias, gelu, a
 
 
 @pytest.mark.parametrize("count,inner,m,n,k", [(3, 0, 70, 72, 64), (6, 3, 33, 64, 72), (6, 2, 65, 65, 64),
-                                                (65537, 0, 2, 8, 8)])
+                                                (65537, 0, 2, 8, 8), (8, 0, 70, 136, 64), (16, 4, 130, 65, 72),
+                                                (75, 5, 33, 76, 64), (80, 0, 257, 168, 128)])
 def test_ring_batches(cuvit, device, count, inner, m, n, k):
-    """Batch entries of their own A, B and C, flat and split, and more than one
-    launch's."""
+    """Batch entries of their own A, B and C, flat and split, more than one
+    launch's, and dealt to the XCDs whole (from 8 on, evenly or nearly so)."""
     a, b = normal(1, (count, m, k), 1.0, device), normal(2, (count, n, k), 0.1, device)
     results = []
     for transposed in (True, False):
@@ -177,7 +178,8 @@ def test_f32_ring_equals_the_tiled_kernel(cuvit, device, m, n, k, with_bias, gel
 
 
 @pytest.mark.parametrize("count,inner,m,n,k", [(3, 0, 33, 36, 68), (6, 3, 50, 50, 64), (4, 2, 17, 65, 64),
-                                                (65537, 0, 2, 8, 4)])
+                                                (65537, 0, 2, 8, 4), (8, 0, 70, 136, 64), (16, 4, 50, 65, 68),
+                                                (75, 5, 33, 76, 64), (80, 0, 257, 168, 128)])
 def test_f32_ring_batches(cuvit, device, count, inner, m, n, k):
     a, b = normal(1, (count, m, k), 1.0, device, torch.float32), normal(2, (count, n, k), 0.1, device, torch.float32)
     results = []
