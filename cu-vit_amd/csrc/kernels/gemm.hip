@@ -3,9 +3,10 @@
 //   fp32 (16 x 16 MFMA): the resident-panel kernel (gemm_panel.hpp) for
 //        tall products with B as [N, K] and K of 192, or 768 into few columns
 //        (the ViT-Tiny linear layers and patch embedding); the ring kernel
-//        (gemm_ring.hpp) for the others with B as [N, K] and 16-byte rows; else
-//        the tiled kernel (gemm_kernel.hpp), 32 x 32 tiles, 64 x 64 once a
-//        problem has work for more than 32 small tiles per compute unit.
+//        (gemm_ring.hpp) for the others with B as [N, K] and 16-byte rows, but
+//        for some of the largest; else the tiled kernel (gemm_kernel.hpp), 32 x
+//        32 tiles, 64 x 64 once a problem has work for more than 32 small tiles
+//        per compute unit.
 //   bf16 (32 x 32 MFMA): B as [N, K] with 16-byte rows runs on direct-to-LDS
 //        loads, in the persistent kernel (gemm_dma.hpp, up to 320 x 256 tiles)
 //        where its tiles fill the chip and in the ring kernel (gemm_ring.hpp,
@@ -233,7 +234,7 @@ hipError_t gemm_f32(const float* a, const float* b, const float* bias, float* c,
     if (whole.transposed && vector_operand(a, whole.lda, whole.k, whole.stride_a, whole.outer_stride_a, split) &&
         vector_operand(b, whole.ldb, whole.k, whole.stride_b, whole.outer_stride_b, split) &&
         static_cast<std::int64_t>(64) * whole.lda * 4 < gemm::kMaxSpan &&
-        static_cast<std::int64_t>(64) * whole.ldb * 4 < gemm::kMaxSpan) {
+        static_cast<std::int64_t>(64) * whole.ldb * 4 < gemm::kMaxSpan && !tiled_beats_ring_f32(whole, compute_units())) {
         const RingChoiceF32 ring = choose_ring_f32(whole, compute_units());
         return gemm_ring_f32(ring.tile, a, b, bias, c, whole, ring.map, stream);
     }

@@ -269,9 +269,15 @@ struct RingChoiceF32 {
 /// While 32 x 16 tiles are alone on their CUs, those, with loading wavefronts
 /// beside the computing ones (197 x 192 x 768 7.6 -> 6.6, 197 x 576 x 192 4.0 ->
 /// 3.6).
-/// Three stages for 32 x 32 tiles where few of them share a CU or K is long
-/// (1576 x 192 x 768 14.3 -> 11.3 us, 394 x 768 x 3072 47 -> 35), two elsewhere
-/// (788 x 768 x 768: 13.7 against 14.3).
+///
+/// Two stages hide the L2 but not HBM, which with K above 128 costs more than a
+/// larger tile gains: 9182 x 96 x 3072, operands from HBM, 90 us on 64 x 32 tiles,
+/// 78 on 32 x 32 with two stages, 66 with three (from the caches 65, 61, 62);
+/// 12608 x 320 x 384 41 us on 64 x 64, 36 on 32 x 32 with three. So three stages
+/// there, and a larger tile only with a long K and many tiles (10602 x 744 x
+/// 3072: 386 us on 64 x 64, 429 on 32 x 32). Entries dealt to the XCDs whole
+/// come from the L2 (196 x 200 x 384 in 192 entries: 75 us with two stages), and
+/// take three only for few tiles a CU.
 inline RingChoiceF32 choose_ring_f32(const GemmArgs& args, int units) {
     constexpr RingTileF32 kTiles[3] = {RingTileF32::k32x32, RingTileF32::k64x32, RingTileF32::k64x64};
     constexpr int kHeights[3] = {32, 64, 64};
@@ -283,10 +289,12 @@ inline RingChoiceF32 choose_ring_f32(const GemmArgs& args, int units) {
     }
     const std::int64_t slots = units >= kXcds ? units / kXcds : 1;  // CUs of an XCD
     const gemm::TileMap map = ring_map(args, 32, 32, 4);
+    const bool by_entry = map.px < 0;
     const std::int64_t small_rounds = (largest_share(args, map, 32, 32) + slots - 1) / slots;
+    const int candidates = by_entry || args.k <= 128 || (args.k >= 1024 && small_rounds > 6) ? 3 : 1;
     RingChoiceF32 best{RingTileF32::k32x32, map};
     double best_cost = 0.0;
-    for (int i = 0; i < 3; ++i) {
+    for (int i = 0; i < candidates; ++i) {
         const std::int64_t rounds = (largest_share(args, map, kHeights[i], kWidths[i]) + slots - 1) / slots;
         const double cost = rounds <= 1 ? kAlone[i] : static_cast<double>(rounds) * kCost[i];
         if (i == 0 || cost < best_cost) {
@@ -294,10 +302,20 @@ inline RingChoiceF32 choose_ring_f32(const GemmArgs& args, int units) {
             best_cost = cost;
         }
     }
-    if (best.tile == RingTileF32::k32x32 && (args.k >= 1024 || (args.k >= 512 && small_rounds <= 2))) {
+    if (best.tile == RingTileF32::k32x32 && (args.k >= 1024 || (args.k > 128 && (!by_entry || small_rounds <= 4)))) {
         best.tile = RingTileF32::k32x32Deep;
     }
     return best;
+}
+
+/// Whether an fp32 problem that the ring kernel could take runs on the tiled
+/// kernel: with many tiles a CU and operands that come from several XCDs' worth
+/// of L2 (12507 x 1928 x 512: 224 to 232 us against 235 to 262 by tile; 8221 x
+/// 1376 x 768 159 against 160 to 174). At K = 64 the ring is ahead, and at K of
+/// 1024 its 64 x 64 tiles are (10602 x 744 x 3072: 386 against 440).
+inline bool tiled_beats_ring_f32(const GemmArgs& args, int units) {
+    return args.k > 64 && (args.count > 1 || args.k < 1024) &&
+           tile_count(args, 32, 32) > 32 * static_cast<std::int64_t>(units) && ring_map(args, 32, 32, 4).px >= 0;
 }
 
 } // namespace cuvit::detail

@@ -37,10 +37,10 @@ int bf16_choice(int m, int n, int k, int count, int gelu, int persistent_fits, i
     return static_cast<int>(ring.tile);
 }
 
-/// A RingTileF32's number.
+/// A RingTileF32's number, or 5 for the tiled kernel.
 int f32_choice(int m, int n, int k, int count, int units) {
     const GemmArgs args = problem(m, n, k, count, 0);
-    return static_cast<int>(choose_ring_f32(args, units).tile);
+    return tiled_beats_ring_f32(args, units) ? 5 : static_cast<int>(choose_ring_f32(args, units).tile);
 }
 
 int whole_entries(int count, long long tiles) { return entries_by_xcd(count, tiles) ? 1 : 0; }

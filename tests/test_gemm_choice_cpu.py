@@ -53,6 +53,30 @@ def test_ring_or_persistent(rules, m, n, k, gelu, expected):
     assert bf16(rules, m, n, k, gelu) == expected
 
 
+RING_F32 = ["32x16 alone", "32x32", "32x32 deep", "64x32", "64x64", "tiled"]
+
+
+@pytest.mark.parametrize("m,n,k,count,expected", [
+    (197, 192, 768, 1, "32x16 alone"),
+    # Operands from HBM: three stages (90 us on 64 x 32 tiles, 66 on these).
+    (9182, 96, 3072, 1, "32x32 deep"),
+    (1576, 2304, 384, 1, "32x32 deep"),
+    (12608, 320, 384, 1, "32x32 deep"),
+    # A long K and many tiles, and a short K: the cheapest tile.
+    (10602, 744, 3072, 1, "64x64"),
+    (11603, 248, 128, 1, "64x64"),
+    # More work than that in one piece.
+    (12507, 1928, 512, 1, "tiled"),
+    (577, 608, 192, 27, "tiled"),
+    # Batches whose entries go to the XCDs whole.
+    (196, 200, 384, 192, "32x32"),
+    (54, 24, 768, 136, "32x32 deep"),
+    (577, 577, 64, 24, "64x32"),
+])
+def test_fp32_ring(rules, m, n, k, count, expected):
+    assert RING_F32[rules.f32_choice(m, n, k, count, UNITS)] == expected
+
+
 @pytest.mark.parametrize("count,whole", [(1, False), (3, False), (8, True), (9, False), (12, False), (24, True),
                                          (27, False), (72, True), (73, True), (75, True), (192, True),
                                          (65537, True)])
