@@ -74,12 +74,12 @@ inline gemm::TileMap tile_map(const GemmArgs& args, int bm, int bn, std::size_t 
 /// whole (TileMap, px < 0), so that each operand is read into one L2 only and
 /// lines of C that two tiles share are merged there: where no XCD gets more
 /// than a tenth above its share. Entries spread over all XCDs against this, us:
-/// bf16 577 x 168 x 384 in 192 entries 63 -> 43, 295 x 296 x 768 in 256 134 ->
+/// bf16 577 x 168 x 384 in 192 entries 63 -> 41, 295 x 296 x 768 in 256 134 ->
 /// 77, fp32 196 x 200 x 384 in 192 118 -> 75; against it, 9 entries for 8 XCDs:
 /// fp32 562 x 128 x 768 12 -> 15.
 inline bool entries_by_xcd(int count, std::int64_t tiles) {
     const std::int64_t dealt = (static_cast<std::int64_t>(count) + kXcds - 1) / kXcds * kXcds;
-    // (The launch's grid within 31 bits.)
+    // (Tiles within a grid's y extent.)
     return count > 1 && tiles < 16384 && 10 * (dealt - count) <= count;
 }
 

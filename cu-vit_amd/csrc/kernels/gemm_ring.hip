@@ -23,7 +23,8 @@ hipError_t run_tiles(const T* a, const T* b, const float* bias, T* c, const Gemm
         return opted;
     }
     return for_entries(args.count, [&](int first, int entries) -> hipError_t {
-        const dim3 grid = map.px < 0 ? dim3(static_cast<unsigned int>((entries + 7) / 8 * 8 * tiles))
+        const dim3 grid = map.px < 0 ? dim3(kXcds, static_cast<unsigned int>(tiles),
+                                            static_cast<unsigned int>((entries + kXcds - 1) / kXcds))
                                      : dim3(static_cast<unsigned int>(tiles), static_cast<unsigned int>(entries));
         Kernel<<<grid, S::kThreads, S::kLdsBytes, stream>>>(a, b, bias, c, args, map, c_run, first);
         return hipGetLastError();

@@ -92,27 +92,28 @@ struct RingShape {
     __device__ __forceinline__ static int place(int row, int chunk) { return chunk ^ ((row >> 1) & 7); }
 };
 
-/// The batch entry and tile of a workgroup, or false where its XCD's block of
-/// the tile grid (TileMap) has fewer tiles than the grid allows.
+/// The batch entry of a workgroup and the number of its tile there. With whole
+/// entries to an XCD (TileMap, px < 0) the grid is 8 x tiles x entries / 8, whose
+/// x is the XCD, else tiles x entries; nothing is divided.
+struct RingSpot {
+    int entry;
+    int tile;
+};
+
+__device__ __forceinline__ RingSpot ring_spot(const TileMap& map, int first_entry) {
+    const int x = static_cast<int>(blockIdx.x);
+    const int y = static_cast<int>(blockIdx.y);
+    return map.px < 0 ? RingSpot{first_entry + 8 * static_cast<int>(blockIdx.z) + x, y} : RingSpot{first_entry + y, x};
+}
+
+/// The tile of a workgroup, or false where its XCD's block of the tile grid
+/// (TileMap) has fewer tiles, or the batch fewer entries, than the grid allows.
 template <typename S>
-__device__ __forceinline__ bool ring_tile(const GemmArgs& args, const TileMap& map, int& entry, int& row0, int& col0) {
+__device__ __forceinline__ bool ring_tile(const GemmArgs& args, const TileMap& map, const RingSpot& spot, int& row0,
+                                          int& col0) {
     const int tiles_n = (args.n + S::kBN - 1) / S::kBN;
-    int tile = static_cast<int>(blockIdx.x);
-    if (map.px < 0) {
-        // Whole entries to an XCD: entry e's tiles on XCD e % 8.
-        const int tiles = (args.m + S::kBM - 1) / S::kBM * tiles_n;
-        const int slot = tile >> 3;
-        const int turn = slot / tiles;
-        entry += 8 * turn + (tile & 7);
-        tile = slot - turn * tiles;
-        if (entry >= args.count) {
-            return false;
-        }
-    } else {
-        entry += static_cast<int>(blockIdx.y);
-    }
-    int tile_m = tile / tiles_n;
-    int tile_n = tile - tile_m * tiles_n;
+    int tile_m = spot.tile / tiles_n;
+    int tile_n = spot.tile % tiles_n;
     if (map.px > 0) {
         const int tiles_m = (args.m + S::kBM - 1) / S::kBM;
         // px py = 8, both powers of two: the split points as shifts, since a
@@ -136,7 +137,7 @@ __device__ __forceinline__ bool ring_tile(const GemmArgs& args, const TileMap& m
     }
     row0 = __builtin_amdgcn_readfirstlane(tile_m * S::kBM);
     col0 = __builtin_amdgcn_readfirstlane(tile_n * S::kBN);
-    return true;
+    return spot.entry < args.count;
 }
 
 /// The stage loads of one wavefront: piece p of wavefront w holds stage rows
@@ -332,7 +333,7 @@ __device__ __forceinline__ void ring_multiply(const RingLoads<T, S>& loads, cons
 }
 
 /// The epilogue's parts as in gemm_dma_kernel (alpha is always multiplied in:
-/// 1 * x is x, bit for bit). Batch entry @p first_entry + blockIdx.y; with
+/// 1 * x is x, bit for bit). Batch entries from @p first_entry on; with
 /// args.rows_per_entry > 0 the rows are entries run as one problem. @p c_run of
 /// C's elements are read and written at once: 8, 4 where N and its rows are
 /// whole 8-byte pieces only (6304 x 2308 x 768 accumulating 72 -> 41 us against
@@ -347,6 +348,11 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring_kernel(const std::uint1
     constexpr int BN = S::kBN;
     constexpr int TM = S::kTM;
     constexpr int TN = S::kTN;
+    const RingSpot spot = ring_spot(map, first_entry);
+    const Offsets entry = entry_offsets(args, spot.entry);
+    a += entry.a;
+    b += entry.b;
+    c += entry.c;
     extern __shared__ Vec16 lds_vectors[];
     unsigned char* const lds = reinterpret_cast<unsigned char*>(lds_vectors);
     const unsigned int lds_base = __builtin_amdgcn_readfirstlane(lds_address(lds));
@@ -359,13 +365,9 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring_kernel(const std::uint1
     const int wave_n = wave % S::kWN;
 
     int row0, col0;
-    if (!ring_tile<S>(args, map, first_entry, row0, col0)) {
+    if (!ring_tile<S>(args, map, spot, row0, col0)) {
         return; // the whole workgroup, before any barrier
     }
-    const Offsets entry = entry_offsets(args, first_entry);
-    a += entry.a;
-    b += entry.b;
-    c += entry.c;
 
     // Old C, one 16-byte piece per lane and row group, issued ahead of the
     // stage loads (so older than they are in every wait below).
@@ -396,7 +398,7 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring_kernel(const std::uint1
                 old_rows[i][k] = Vec16{{0U, 0U, 0U, 0U}};
                 if (row < args.m && store_col < args.n) {
                     const std::uint16_t* const from = c + c_offset(row) + store_col;
-                    if (c_run == 8) {
+                    if (__builtin_expect(c_run == 8, 1)) {
                         old_rows[i][k] = load16(from);
                     } else if (c_run == 4) {
                         const uint2 first = *reinterpret_cast<const uint2*>(from);
@@ -485,7 +487,7 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring_kernel(const std::uint1
             const Vec16 v = *reinterpret_cast<const Vec16*>(staged(kRowsPerStore * k + store_row, store_chunk));
             if (out_row < args.m && store_col < args.n) {
                 std::uint16_t* const to = c + c_offset(out_row) + store_col;
-                if (c_run == 8) {
+                if (__builtin_expect(c_run == 8, 1)) {
                     store16(to, v);
                 } else if (c_run == 4) {
                     *reinterpret_cast<uint2*>(to) = make_uint2(v.w[0], v.w[1]);
@@ -518,6 +520,8 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring_f32_kernel(const float*
     constexpr int TM = S::kTM;
     constexpr int TN = S::kTN;
     constexpr int E = S::kEdge;
+    const RingSpot spot = ring_spot(map, first_entry);
+    const Offsets entry = entry_offsets(args, spot.entry);
     extern __shared__ Vec16 lds_vectors[];
     unsigned char* const lds = reinterpret_cast<unsigned char*>(lds_vectors);
     const unsigned int lds_base = __builtin_amdgcn_readfirstlane(lds_address(lds));
@@ -528,10 +532,9 @@ __global__ __launch_bounds__(S::kThreads) void gemm_ring_f32_kernel(const float*
     const int wave_m = wave / S::kWN;
     const int wave_n = wave % S::kWN;
     int row0, col0;
-    if (!ring_tile<S>(args, map, first_entry, row0, col0)) {
+    if (!ring_tile<S>(args, map, spot, row0, col0)) {
         return; // the whole workgroup, before any barrier
     }
-    const Offsets entry = entry_offsets(args, first_entry);
 
     // The epilogue's operands ahead of the stage loads: the bias of this
     // lane's runs and old C.

@@ -91,7 +91,7 @@ def test_fp32_ring(rules, m, n, k, count, expected):
                                          (65537, True)])
 def test_entries_go_to_the_xcds_whole_where_they_divide_evenly(rules, count, whole):
     assert rules.whole_entries(count, 64) == int(whole)
-    assert rules.whole_entries(count, 16384) == 0  # a grid past 31 bits
+    assert rules.whole_entries(count, 16384) == 0  # past a grid
 
 
 @pytest.mark.parametrize("count,launches", [(1, 1), (65528, 1), (65529, 2), (2 ** 31 - 65529, 32772),
