@@ -36,7 +36,8 @@
 // launch stores them. Error against 64 bits at 577 tokens, Q and K of standard
 // deviation 1 (0.05): fp32 4.2e-7 (3.1e-7) against the launches' 5.2e-7
 // (4.3e-7), bf16 2.3e-3 (2.0e-3) against 4.4e-3 (2.1e-3). A row of -inf logits
-// gives NaN, as the launches do.
+// gives NaN, as the launches do; a query whose sums overflow or vanish before
+// they are normalised is taken again by itself (attend_normalised).
 #include "attention_common.hpp"
 #include "launch.hpp"
 
@@ -122,12 +123,11 @@ __device__ __forceinline__ void walk_blocks(int tokens, int part, bool live, Pre
             constexpr int kPart = Keys / kSplit;
             constexpr int kTiles = kPart / Edge;
             const int left = tokens - first - part * kPart;
+            static_assert(kTiles <= 2, "a tail is one tile or all of them");
             if (left >= kPart) {
                 step(std::integral_constant<int, kTiles>{}, std::false_type{}, buffer, left);
-            } else if (kTiles > 1 && left > kPart / 2) {
+            } else if (kTiles > 1 && left > Edge) {
                 step(std::integral_constant<int, kTiles>{}, std::true_type{}, buffer, left);
-            } else if (kTiles > 2 && left > Edge) {
-                step(std::integral_constant<int, (kTiles + 1) / 2>{}, std::true_type{}, buffer, left);
             } else if (left > 0) {
                 step(std::integral_constant<int, 1>{}, std::true_type{}, buffer, left);
             }
@@ -180,13 +180,83 @@ __device__ __forceinline__ void combine_parts(float* lds, int wave, int lane, Ru
     }
 }
 
+/// Whether a query's sums are of no use: its numerators overflowed where the
+/// context would not (V within its type, but above 2^128 / (tokens 2^kHeadroom),
+/// about 2e33 here), its weights did, or they vanished (logits beyond 2^31,
+/// the type's lowest value among them: `shift` is then rounded by more than an
+/// exponent's range), or there is an infinity or NaN in it, which stays.
+template <int Count> __device__ __forceinline__ bool unusable(float sum, const float (&values)[Count]) {
+    float largest[2] = {0.F, 0.F};
+#pragma unroll
+    for (int i = 0; i < Count; ++i) { // (a NaN stays)
+        largest[i / 2 % 2] = __builtin_elementwise_maximum(largest[i / 2 % 2], fabsf(values[i]));
+    }
+    const float all = __builtin_elementwise_maximum(largest[0], largest[1]);
+    return !(all < INFINITY && sum > 0.F && sum < INFINITY);
+}
+
+/// The context of one query whose sums were unusable, by a whole wavefront: the
+/// exponent is a difference of logits, and what is accumulated stays
+/// normalised, so within max |V|, both as in the launches. @p qkv is the pair's
+/// Q of token 0. Slow, and seldom run; weights lowered for every query instead
+/// would lose as much where V is tiny, and the difference costs an instruction a
+/// logit.
+template <typename T>
+__device__ __forceinline__ void attend_normalised(const T* qkv, T* context_row, int query, int tokens,
+                                                  std::int64_t qkv_row, int embed) {
+    constexpr int kVec = Elem<T>::kPerVec;
+    const int lane = lane_id();
+    const T* const q = qkv + query * qkv_row;
+    float maximum = -INFINITY;
+    float sum = 0.F;
+    float value = 0.F; // of dim `lane`
+#pragma clang loop unroll(disable)
+    for (int first = 0; first < tokens; first += kWave) {
+        float logit = -INFINITY; // of key first + lane
+        if (first + lane < tokens) {
+            const T* const k = qkv + (first + lane) * qkv_row + embed;
+            logit = 0.F;
+#pragma clang loop unroll(disable)
+            for (int d = 0; d < kHeadDim; d += kVec) {
+                const Vec16 a = load16(q + d);
+                const Vec16 b = load16(k + d);
+#pragma unroll
+                for (int e = 0; e < kVec; ++e) {
+                    logit = fmaf(Elem<T>::get(a, e), Elem<T>::get(b, e), logit);
+                }
+            }
+        }
+        const float raised = fmaxf(maximum, wave_allreduce(logit, Max2{}));
+        if (raised == -INFINITY) {
+            continue;
+        }
+        const float weight = __builtin_amdgcn_exp2f((logit - raised) * kScaledLog2e);
+        const float kept = maximum == -INFINITY ? 0.F : sum * __builtin_amdgcn_exp2f((maximum - raised) * kScaledLog2e);
+        maximum = raised;
+        sum = kept + wave_allreduce(weight, Add2{});
+        if (sum != sum) {
+            break; // NaN, whatever follows
+        }
+        value *= kept / sum;
+        const float share = weight / sum;
+        const int keys = min(tokens - first, kWave);
+        const T* const v = qkv + first * qkv_row + 2 * static_cast<std::int64_t>(embed) + lane;
+#pragma clang loop unroll(disable)
+        for (int key = 0; key < keys; ++key) {
+            const float s = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(share), key));
+            value = fmaf(s, Elem<T>::load(v + key * qkv_row), value);
+        }
+    }
+    Elem<T>::store(context_row + lane, sum > 0.F ? value : __builtin_nanf("")); // (no logit above -inf: NaN)
+}
+
 // -- bf16 -----------------------------------------------------------------------
 
 constexpr int kEdge = 32;       // queries of a wavefront, keys of an MFMA tile
 constexpr int kBlockKeys = 64;  // keys a step
 constexpr int kKBlock = 16;     // k of one MFMA
 
-__global__ __launch_bounds__(kThreads, 2) void attention_long_bf16_kernel(
+__global__ __launch_bounds__(kThreads, 3) void attention_long_bf16_kernel(
     const std::uint16_t* __restrict__ qkv, std::uint16_t* __restrict__ context, int heads, int tokens,
     int pairs, int groups) {
     using Acc = Mma<std::uint16_t>::Acc;
@@ -362,21 +432,31 @@ __global__ __launch_bounds__(kThreads, 2) void attention_long_bf16_kernel(
     if (!live || part > 0) {
         return;
     }
-    const float inverse = 1.0F / combine_halves(running.sum, Add2{});
-    if (query >= tokens) {
-        return;
-    }
-    std::uint16_t* const destination =
-        context + (static_cast<std::int64_t>(image) * tokens + query) * embed + head * kHeadDim;
+    const float total = combine_halves(running.sum, Add2{});
+    const float inverse = 1.0F / total;
+    std::uint16_t* const rows = context + (static_cast<std::int64_t>(image) * tokens + query0) * embed + head * kHeadDim;
+    // The row anew, from the hardware's lane number: kept over the walk it would
+    // be the register that costs the third wavefront a SIMD.
+    const int out_row = static_cast<int>(__builtin_amdgcn_mbcnt_hi(~0U, __builtin_amdgcn_mbcnt_lo(~0U, 0U))) % kEdge;
+    const bool inside = query0 + out_row < tokens;
+    const std::uint64_t bad = __ballot(inside && unusable(total, sums));
+    std::uint32_t again = static_cast<std::uint32_t>(bad | (bad >> kEdge)); // bit: row of the tile
+    if (inside && (again >> out_row & 1U) == 0) {
+        std::uint16_t* const destination = rows + static_cast<std::int64_t>(out_row) * embed;
 #pragma unroll
-    for (int d = 0; d < 2; ++d) {
+        for (int d = 0; d < 2; ++d) {
 #pragma unroll
-        for (int run = 0; run < 4; ++run) {
-            uint2 bits;
-            bits.x = pack_bf16x2(sums[16 * d + 4 * run] * inverse, sums[16 * d + 4 * run + 1] * inverse);
-            bits.y = pack_bf16x2(sums[16 * d + 4 * run + 2] * inverse, sums[16 * d + 4 * run + 3] * inverse);
-            *reinterpret_cast<uint2*>(destination + d * kEdge + Mma<std::uint16_t>::column(lane, run)) = bits;
+            for (int run = 0; run < 4; ++run) {
+                uint2 bits;
+                bits.x = pack_bf16x2(sums[16 * d + 4 * run] * inverse, sums[16 * d + 4 * run + 1] * inverse);
+                bits.y = pack_bf16x2(sums[16 * d + 4 * run + 2] * inverse, sums[16 * d + 4 * run + 3] * inverse);
+                *reinterpret_cast<uint2*>(destination + d * kEdge + Mma<std::uint16_t>::column(lane, run)) = bits;
+            }
         }
+    }
+    for (; __builtin_expect(again != 0, 0); again &= again - 1) {
+        const int r = __builtin_ctz(again);
+        attend_normalised(q_base, rows + static_cast<std::int64_t>(r) * embed, query0 + r, tokens, qkv_row, embed);
     }
 }
 
@@ -558,11 +638,15 @@ __global__ __launch_bounds__(kThreads, 2) void attention_long_f32_kernel(const f
     if (!live || part > 0) {
         return;
     }
-    const float inverse = 1.0F / combine_rows<32>(combine_rows<16>(running.sum, Add2{}), Add2{});
-    if (query < tokens) {
+    const float total = combine_rows<32>(combine_rows<16>(running.sum, Add2{}), Add2{});
+    const float inverse = 1.0F / total;
+    float* const rows = context + (static_cast<std::int64_t>(image) * tokens + query0) * embed + head * kHeadDim;
+    std::uint64_t bad = __ballot(query < tokens && unusable(total, sums));
+    bad |= bad >> 32;
+    std::uint32_t again = static_cast<std::uint32_t>(bad | (bad >> kEdgeF32)) & 0xFFFFU; // bit: row of the tile
+    if (query < tokens && (again >> row & 1U) == 0) {
         // Lane holds context[query][16 dt + 4 group .. + 3].
-        float* const destination = context + (static_cast<std::int64_t>(image) * tokens + query) * embed +
-                                   head * kHeadDim + 4 * group;
+        float* const destination = rows + static_cast<std::int64_t>(row) * embed + 4 * group;
 #pragma unroll
         for (int dt = 0; dt < kHeadDim / 16; ++dt) {
             floatx4 value;
@@ -573,9 +657,13 @@ __global__ __launch_bounds__(kThreads, 2) void attention_long_f32_kernel(const f
             *reinterpret_cast<floatx4*>(destination + 16 * dt) = value;
         }
     }
+    for (; __builtin_expect(again != 0, 0); again &= again - 1) {
+        const int r = __builtin_ctz(again);
+        attend_normalised(q_base, rows + static_cast<std::int64_t>(r) * embed, query0 + r, tokens, qkv_row, embed);
+    }
 }
 
-/// Workgroups: a pair's groups of four query tiles, pairs rounded up to the
+/// Workgroups: a pair's groups of two query tiles, pairs rounded up to the
 /// XCDs (a workgroup past the last pair leaves at once).
 unsigned int grid_size(std::int64_t pairs, int groups) {
     return static_cast<unsigned int>((pairs + 7) / 8 * 8 * groups);

@@ -1,6 +1,8 @@
 // Internals for the Python tests: the GEMM dispatch rules (gemm_choice.hpp) for
 // test_gemm_choice_cpu.py, which kernel and tile a problem takes on a card of
-// `units` compute units, and how a batch is spread over launches.
+// `units` compute units, and how a batch is spread over launches; and the
+// model's attention beyond 256 tokens by itself for test_long_attention_gpu.py.
+#include "capi/status.hpp"
 #include "kernels/gemm_choice.hpp"
 
 using namespace cuvit::detail;
@@ -59,5 +61,15 @@ int batch_launches(int count) {
         return hipSuccess;
     });
     return status == hipSuccess && covered == count ? launches : -1;
+}
+
+int long_attention_f32(const void* qkv, void* context, int images, int heads, int tokens, void* stream) {
+    return cuvit::capi::attention_long(static_cast<const float*>(qkv), static_cast<float*>(context), images, heads,
+                                       tokens, static_cast<hipStream_t>(stream));
+}
+
+int long_attention_bf16(const void* qkv, void* context, int images, int heads, int tokens, void* stream) {
+    return cuvit::capi::attention_long(static_cast<const std::uint16_t*>(qkv), static_cast<std::uint16_t*>(context),
+                                       images, heads, tokens, static_cast<hipStream_t>(stream));
 }
 }
