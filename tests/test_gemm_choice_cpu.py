@@ -1,5 +1,6 @@
 """Which kernel and tile a bf16 or fp32 product takes (gemm_choice.hpp), on the
-256 compute units of an MI355X."""
+256 compute units of an MI355X, the cases of the ring kernel's GPU tests among
+them."""
 
 from __future__ import annotations
 
@@ -10,6 +11,7 @@ from pathlib import Path
 import pytest
 
 from conftest import ROOT
+from test_gemm_ring_gpu import CASES, F32_CASES
 
 UNITS = 256
 RING = ["64x32 alone", "64x64", "64x64 alone", "64x64 deep", "128x64", "128x128", "128x128 deep"]
@@ -62,6 +64,13 @@ def test_gelu_of_one_round(rules, m, n, k, count, expected):
     assert bf16(rules, m, n, k, True, count) == expected
 
 
+@pytest.mark.parametrize("case", CASES, ids=str)
+def test_each_ring_case_reaches_its_tile(rules, case):
+    m, n, k, _, gelu, _, _, pad, tile = case
+    fits = n % 256 == 0 and k >= 256 and (n + pad) % 8 == 0
+    assert bf16(rules, m, n, k, gelu, persistent_fits=fits) == tile
+
+
 RING_F32 = ["32x16 alone", "32x32", "32x32 deep", "64x32", "64x64", "tiled"]
 
 
@@ -84,6 +93,11 @@ RING_F32 = ["32x16 alone", "32x32", "32x32 deep", "64x32", "64x64", "tiled"]
 ])
 def test_fp32_ring(rules, m, n, k, count, expected):
     assert RING_F32[rules.f32_choice(m, n, k, count, UNITS)] == expected
+
+
+@pytest.mark.parametrize("case", F32_CASES, ids=str)
+def test_each_fp32_ring_case_reaches_its_tile(rules, case):
+    assert RING_F32[rules.f32_choice(*case[:3], 1, UNITS)] == case[-1]
 
 
 @pytest.mark.parametrize("count,whole", [(1, False), (3, False), (8, True), (9, False), (12, False), (24, True),

@@ -1,6 +1,7 @@
-"""The LDS-ring bf16 GEMM (64 x 64, 128 x 64 and 128 x 128 tiles), which
-products with B as [N, K] and 16-byte operand rows take where the persistent
-kernel does not.
+"""The LDS-ring GEMM in every tile that the dispatch takes (bf16 64 x 32 to 128
+x 128, fp32 32 x 16 to 64 x 64; test_gemm_choice_cpu.py checks that each case
+below reaches the tile it names), which products with B as [N, K] and 16-byte
+operand rows take where the persistent kernel and the panels do not.
 
 The tiled kernel, which B as [K, N] takes, runs the same MFMA over the same
 k-blocks in the same order and rounds every step of the epilogue alike, so the
@@ -29,29 +30,33 @@ def run(cuvit, a, b, bias, c, problem, transposed):
 
 
 CASES = [
-    # m, n, k, bias, gelu, accumulate, alpha, C's padding
-    (1, 8, 8, True, False, False, 1.0, 0),            # one tile, one row, one chunk of K
-    (63, 64, 64, True, True, False, 1.0, 0),          # a row short of a tile
-    (65, 72, 136, True, False, True, 1.0, 8),         # a row and a chunk past; K past one span
-    (64, 65, 128, True, False, True, 1.0, 0),         # odd N: element-wise C, accumulating
-    (65, 76, 136, True, False, True, 1.0, 0),         # C in 8-byte pieces, accumulating, half a chunk at N
-    (130, 132, 72, True, True, False, 1.0, 4),        # the same, padded rows
-    (4616, 1540, 384, True, False, True, 1.0, 0),     # the same on 128 x 128 tiles
-    (130, 199, 72, False, True, False, -0.5, 3),      # odd rows of C, GELU without bias, alpha
-    (197, 768, 3080, True, False, True, 1.0, 0),      # tiles alone on their CUs, long K
-    (65, 2304, 128, True, True, True, 1.0, 0),        # the same at one span of K
-    (197, 2304, 776, True, False, False, 1.0, 0),     # 64 x 64 alone, loading wavefronts
-    (1576, 1536, 200, True, False, True, 1.0, 0),     # several 64 x 64 tiles a CU
-    (1576, 768, 1032, True, False, True, 1.0, 0),     # 64 x 64 tiles with three stages
-    (1576, 2304, 200, True, False, False, 1.0, 0),    # 128 x 64 tiles
-    (1571, 3064, 64, True, True, True, 1.0, 1),       # 128 x 64 or 128 x 128, odd rows of C
-    (6304, 1152, 384, True, False, False, 1.0, 0),    # 128 x 128 tiles
-    (3152, 776, 1032, True, False, True, 1.0, 0),     # 128 x 128 with three stages, N and K off the grid
-    (4616, 1536, 384, True, True, False, 1.0, 0),     # 128 x 128 where the persistent kernel could run
+    # m, n, k, bias, gelu, accumulate, alpha, C's padding, tile
+    (1, 8, 8, True, False, False, 1.0, 0, "64x32 alone"),            # one row, one chunk of K
+    (63, 64, 64, True, True, False, 1.0, 0, "64x32 alone"),          # a row short of a tile
+    (65, 72, 136, True, False, True, 1.0, 8, "64x32 alone"),         # a row and a chunk past; K past one span
+    (64, 65, 128, True, False, True, 1.0, 0, "64x32 alone"),         # odd N: element-wise C, accumulating
+    (65, 76, 136, True, False, True, 1.0, 0, "64x32 alone"),         # C in 8-byte pieces, half a chunk at N
+    (130, 132, 72, True, True, False, 1.0, 4, "64x32 alone"),        # the same, padded rows
+    (130, 199, 72, False, True, False, -0.5, 3, "64x32 alone"),      # odd rows of C, GELU without bias, alpha
+    (197, 768, 3080, True, False, True, 1.0, 0, "64x32 alone"),      # long K
+    (65, 2304, 128, True, True, True, 1.0, 0, "64x32 alone"),        # one span of K
+    (197, 2304, 776, True, False, False, 1.0, 0, "64x64 alone"),     # loading wavefronts
+    (1576, 1536, 200, True, False, True, 1.0, 0, "64x64"),           # several tiles a CU
+    (4616, 1540, 384, True, False, True, 1.0, 0, "64x64"),           # C in 8-byte pieces
+    (3152, 776, 1032, True, False, True, 1.0, 0, "64x64"),           # N and K off the grid
+    (1576, 768, 1032, True, False, True, 1.0, 0, "64x64 deep"),      # three stages
+    (1576, 2304, 200, True, False, False, 1.0, 0, "128x64"),
+    (1571, 3064, 64, True, True, True, 1.0, 1, "128x64"),            # odd rows of C
+    (6304, 1152, 384, True, False, False, 1.0, 0, "128x128"),
+    (6301, 1145, 200, True, False, True, 1.0, 1, "128x128"),         # accumulating, odd N and rows of C
+    (6304, 1148, 384, False, False, True, 0.5, 0, "128x128"),        # C in 8-byte pieces, accumulating
+    (4616, 1536, 384, True, True, False, 1.0, 0, "128x128"),         # where the persistent kernel could run
+    (4616, 768, 1032, True, False, True, 1.0, 0, "128x128 deep"),    # three stages, accumulating
+    (4611, 757, 1032, False, True, False, 1.0, 3, "128x128 deep"),   # tails, odd rows of C
 ]
 
 
-@pytest.mark.parametrize("m,n,k,with_bias,gelu,accumulate,alpha,pad", CASES)
+@pytest.mark.parametrize("m,n,k,with_bias,gelu,accumulate,alpha,pad", [case[:-1] for case in CASES])
 def test_ring_equals_the_tiled_kernel(cuvit, device, m, n, k, with_bias, gelu, accumulate, alpha, pad):
     a = normal(m + k, (m, k), 1.0, device)
     b = normal(n + k, (n, k), 0.05, device)
@@ -131,19 +136,22 @@ def test_ring_runs_a_shared_weight_batch_as_one_problem(cuvit, device):
 
 
 F32_CASES = [
-    # m, n, k, bias, gelu, accumulate, alpha, C's padding
-    (1, 8, 4, True, False, False, 1.0, 0),           # one tile, one chunk of K
-    (31, 33, 64, True, True, False, 1.0, 3),         # odd rows of C
-    (33, 65, 68, True, False, True, 1.0, 0),         # past a tile, past a span of K; element-wise C
-    (197, 192, 772, False, False, True, -0.5, 4),    # tiles alone on their CUs
-    (230, 640, 772, True, False, False, 1.0, 0),     # 32 x 32 tiles with three stages
-    (788, 384, 320, True, True, True, 1.0, 0),       # several 32 x 32 tiles a CU
-    (1003, 1152, 100, True, False, False, 1.0, 0),   # 64 x 32 or 64 x 64 tiles with tails
-    (3151, 1540, 196, False, True, False, 2.0, 0),   # 64 x 64 tiles, GELU without bias
+    # m, n, k, bias, gelu, accumulate, alpha, C's padding, tile
+    (1, 8, 4, True, False, False, 1.0, 0, "32x16 alone"),            # one chunk of K
+    (31, 33, 64, True, True, False, 1.0, 3, "32x16 alone"),          # odd rows of C
+    (33, 65, 68, True, False, True, 1.0, 0, "32x16 alone"),          # past a tile, past a span of K; a run that N cuts
+    (197, 192, 772, False, False, True, -0.5, 4, "32x16 alone"),
+    (230, 640, 772, True, False, False, 1.0, 0, "32x32 deep"),       # three stages
+    (788, 384, 320, True, True, True, 1.0, 0, "32x32 deep"),         # several tiles a CU
+    (3151, 1540, 196, False, True, False, 2.0, 0, "32x32 deep"),     # GELU without bias
+    (1003, 1152, 100, True, False, False, 1.0, 0, "32x32"),          # two stages, tails
+    (394, 2302, 100, True, True, True, 0.5, 1, "64x32"),             # tails, odd rows of C
+    (3151, 1541, 100, False, False, True, 1.0, 0, "64x64"),          # tails, odd N
+    (5001, 1540, 1028, True, False, False, 1.0, 0, "64x64"),         # a long K
 ]
 
 
-@pytest.mark.parametrize("m,n,k,with_bias,gelu,accumulate,alpha,pad", F32_CASES)
+@pytest.mark.parametrize("m,n,k,with_bias,gelu,accumulate,alpha,pad", [case[:-1] for case in F32_CASES])
 def test_f32_ring_equals_the_tiled_kernel(cuvit, device, m, n, k, with_bias, gelu, accumulate, alpha, pad):
     a = normal(m + k, (m, k), 1.0, device, torch.float32)
     b = normal(n + k, (n, k), 0.05, device, torch.float32)

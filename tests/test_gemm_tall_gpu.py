@@ -1,17 +1,15 @@
-"""The twelve-wavefront bf16 GEMM tile (256 x 192, wavefront tiles of 64 x 64,
-64-deep stages), which products with B as [N, K] and K of at least 512 take
-when one round of such tiles covers the problem and 128 x 128 tiles would need
-more than two per compute unit: the ViT-Base FC2 and projection at batch 64
-(12608 x 768 x 3072 and 12608 x 768 x 768, accumulating into the residual
-stream).
+"""Large bf16 products with B as [N, K] into few columns, most of them
+accumulating: the ViT-Base FC2 and projection at batch 64 (12608 x 768 x 3072
+and 12608 x 768 x 768, into the residual stream) on the persistent kernel, and
+others off its grid on the 128-row ring tiles.
 
-Its results must be bitwise those of the 64 x 64 kernel that small problems
-take: both run the same MFMA over the same k-blocks in the same order and
-apply alpha, the bias, GELU and the accumulation without fusing them. Each
-case launches a problem the tall tile takes (outputs that are not accumulated
-into start as NaN), then the same rows in launches of 197 rows, and requires
-equality bit for bit over every row; the last 64 rows are also judged
-against the oracle, and the columns past N must keep their values.
+Their results must be bitwise those of the small ring tiles that launches of
+few rows take: all run the same MFMA over the same k-blocks in the same order
+and apply alpha, the bias, GELU and the accumulation without fusing them. Each
+case launches the whole problem (outputs that are not accumulated into start as
+NaN), then the same rows in launches of 197 rows, and requires equality bit for
+bit over every row; the last 64 rows are also judged against the oracle, and
+the columns past N must keep their values.
 """
 
 from __future__ import annotations
@@ -103,8 +101,8 @@ def test_tall_tile_equals_the_small_tile_kernel(cuvit, oracle, device, m, n, k, 
 
 
 def test_tall_tile_batched_entries(cuvit, oracle, device):
-    """Two batch entries of 6304 rows (one round of 200 tall tiles between
-    them), B shared: each entry equals its own launch, bit for bit."""
+    """Two batch entries of 6304 rows, B shared, which run as one problem: each
+    entry equals its own launch, bit for bit."""
     m, n, k = 6304, 768, 3072
     a_bits, _ = bf16_inputs(oracle, 91, 2 * m * k)
     w_bits, _ = bf16_inputs(oracle, 92, n * k, 0.02)
@@ -128,7 +126,7 @@ def test_tall_tile_batched_entries(cuvit, oracle, device):
 def test_tall_tile_runs_a_shared_weight_batch_as_one_problem(cuvit, oracle, device):
     """A batch of 64 entries of 196 rows with B shared and A rows following
     one another (the ViT-Base patch embedding's shape) runs as one problem of
-    12544 rows on the tall tile; each entry lands at its own C stride (197
+    12544 rows; each entry lands at its own C stride (197
     rows apart, so one row per entry is never written) and equals its own
     launch of 196 rows, bit for bit."""
     entries, m, n, k = 64, 196, 768, 768

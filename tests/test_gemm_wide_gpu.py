@@ -1,12 +1,12 @@
-"""The wide-tile bf16 GEMM (128 x 256 workgroup tiles, epilogue through LDS),
-which large B-as-[N, K] problems without accumulation take.
+"""Large bf16 products with B as [N, K] and no accumulation: the persistent
+kernel's (N a multiple of 256) and the 128 x 128 ring tiles' (the others).
 
-Its results must be bitwise those of the 64 x 64 / 128 x 128 kernel that small
-problems take: both run the same MFMA over the same k-blocks in the same order
-and apply alpha and the bias without fusing them. Each case launches a problem
-large enough for the wide kernel (output prefilled with NaN), then the same
-rows in launches of 197 rows, small enough for the other kernel, and requires
-equality bit for bit; one block of rows is also judged against the oracle.
+Their results must be bitwise those of the small ring tiles that launches of
+few rows take: all run the same MFMA over the same k-blocks in the same order
+and apply alpha and the bias without fusing them. Each case launches the whole
+problem (output prefilled with NaN), then the same rows in launches of 197
+rows, and requires equality bit for bit; one block of rows is also judged
+against the oracle.
 """
 
 from __future__ import annotations
@@ -41,8 +41,8 @@ def require_gemm_close(actual, expected, scale, context):
 
 CASES = [
     # m, n, k, bias, gelu, alpha
-    (12608, 3072, 768, True, True, 1.0),      # ViT-Base FC1
-    (12608, 2304, 768, True, False, 1.0),     # ViT-Base QKV
+    (12608, 3072, 768, True, True, 1.0),      # ViT-Base FC1 (persistent)
+    (12608, 2304, 768, True, False, 1.0),     # ViT-Base QKV (persistent)
     (12608, 1544, 776, True, True, 0.75),     # N and K off the tile grid, alpha with the bias
     (12450, 1544, 200, False, False, -1.25),  # M tail, short K, no bias
     (12608, 1320, 768, False, True, 0.5),     # GELU without a bias
