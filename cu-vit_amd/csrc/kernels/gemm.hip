@@ -221,10 +221,13 @@ hipError_t gemm_f32(const float* a, const float* b, const float* bias, float* c,
                panel != hipErrorNotSupported) {
         return panel;
     }
-    // K = 768 into wide outputs is the ring kernel's (3152 x 2304 114 -> 107 us,
-    // 3152 x 768 40 -> 37); into 192 columns the panels stay ahead (6304 rows:
-    // 23.1 against 25.0 us).
-    if (whole.n < 512) {
+    // K = 768: the panels into few columns (192 of 6304 rows: 23.1 us against the
+    // ring kernel's 25.0) and, with many tiles, into up to 1024 (768 of 4616 rows
+    // accumulating 51 against 55 to 58, of 3152 37 against 39 to 41, of 2364 31.6
+    // against 31). Wider ones, and with GELU, are the ring kernel's (3152 x 2304
+    // 101 against 101, 4616 x 3072 with GELU 216 against 190).
+    if (whole.n < 512 || (whole.n <= 1024 && !whole.gelu &&
+                          tile_count(whole, 32, 32) > 8 * static_cast<std::int64_t>(compute_units()))) {
         if (const hipError_t panel = launch_panel<48, 32, 2, 4, 12>(a, b, bias, c, whole, stream);
             panel != hipErrorNotSupported) {
             return panel;

@@ -278,10 +278,11 @@ struct RingChoiceF32 {
 /// larger tile gains: 9182 x 96 x 3072, operands from HBM, 90 us on 64 x 32 tiles,
 /// 78 on 32 x 32 with two stages, 66 with three (from the caches 65, 61, 62);
 /// 12608 x 320 x 384 41 us on 64 x 64, 36 on 32 x 32 with three. So three stages
-/// there, and a larger tile only with a long K and many tiles (10602 x 744 x
-/// 3072: 386 us on 64 x 64, 429 on 32 x 32). Entries dealt to the XCDs whole
-/// come from the L2 (196 x 200 x 384 in 192 entries: 75 us with two stages), and
-/// take three only for few tiles a CU.
+/// there, but for many tiles a CU, where more workgroups hide as much (1576 x
+/// 2304 x 768 54 us with two, 57 with three), and a larger tile only with a long
+/// K and many tiles (10602 x 744 x 3072: 386 us on 64 x 64, 429 on 32 x 32).
+/// Entries dealt to the XCDs whole come from the L2 (196 x 200 x 384 in 192
+/// entries: 75 us with two stages), and take three for few tiles a CU only.
 inline RingChoiceF32 choose_ring_f32(const GemmArgs& args, int units) {
     constexpr RingTileF32 kTiles[3] = {RingTileF32::k32x32, RingTileF32::k64x32, RingTileF32::k64x64};
     constexpr int kHeights[3] = {32, 64, 64};
@@ -306,7 +307,7 @@ inline RingChoiceF32 choose_ring_f32(const GemmArgs& args, int units) {
             best_cost = cost;
         }
     }
-    if (best.tile == RingTileF32::k32x32 && (args.k >= 1024 || (args.k > 128 && (!by_entry || small_rounds <= 4)))) {
+    if (best.tile == RingTileF32::k32x32 && (args.k >= 1024 || (args.k > 128 && small_rounds <= (by_entry ? 4 : 12)))) {
         best.tile = RingTileF32::k32x32Deep;
     }
     return best;

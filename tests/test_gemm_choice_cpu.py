@@ -78,8 +78,10 @@ RING_F32 = ["32x16 alone", "32x32", "32x32 deep", "64x32", "64x64", "tiled"]
     (197, 192, 768, 1, "32x16 alone"),
     # Operands from HBM: three stages (90 us on 64 x 32 tiles, 66 on these).
     (9182, 96, 3072, 1, "32x32 deep"),
-    (1576, 2304, 384, 1, "32x32 deep"),
-    (12608, 320, 384, 1, "32x32 deep"),
+    (3152, 384, 384, 1, "32x32 deep"),
+    # More tiles a CU than three stages leave workgroups for.
+    (1576, 2304, 768, 1, "32x32"),
+    (12608, 320, 384, 1, "32x32"),
     # A long K and many tiles, and a short K: the cheapest tile.
     (10602, 744, 3072, 1, "64x64"),
     (11603, 248, 128, 1, "64x64"),

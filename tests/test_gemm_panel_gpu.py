@@ -32,7 +32,8 @@ CASES = [
     (4099, 196, 192, False, True, True, 0.75, 8, 4),     # M and N tails, GELU + accumulate, alpha
     (5000, 300, 768, True, True, False, -1.25, 4, 0),    # 48 k-blocks, a partial last panel, alpha
     (6001, 196, 768, False, True, True, 0.75, 8, 4),     # the same with M and N tails, GELU + accumulate
-    (5000, 580, 768, True, True, False, -1.25, 4, 0),    # wide N at K = 768: the ring kernel
+    (5000, 580, 768, True, True, False, -1.25, 4, 0),    # wide N at K = 768 with GELU: the ring kernel
+    (3152, 768, 768, True, False, True, 1.0, 0, 0),      # ViT-Base projection
     (4111, 392, 192, True, False, False, 2.0, 0, 12),    # a partial last panel, padded C rows
 ]
 

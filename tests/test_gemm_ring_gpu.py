@@ -143,7 +143,7 @@ F32_CASES = [
     (197, 192, 772, False, False, True, -0.5, 4, "32x16 alone"),
     (230, 640, 772, True, False, False, 1.0, 0, "32x32 deep"),       # three stages
     (788, 384, 320, True, True, True, 1.0, 0, "32x32 deep"),         # several tiles a CU
-    (3151, 1540, 196, False, True, False, 2.0, 0, "32x32 deep"),     # GELU without bias
+    (3151, 1540, 196, False, True, False, 2.0, 0, "32x32"),          # many tiles a CU, GELU without bias
     (1003, 1152, 100, True, False, False, 1.0, 0, "32x32"),          # two stages, tails
     (394, 2302, 100, True, True, True, 0.5, 1, "64x32"),             # tails, odd rows of C
     (3151, 1541, 100, False, False, True, 1.0, 0, "64x64"),          # tails, odd N
