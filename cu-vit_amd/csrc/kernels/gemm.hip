@@ -50,9 +50,9 @@ template <typename T> bool vector_output(const T* c, const GemmArgs& args) {
 }
 
 template <typename T, int WM, int WN, int TM, int TN, int BK, int MinWaves, bool VecA, bool VecB,
-          bool TransB>
+          bool TransB, bool Unaligned>
 hipError_t launch(const T* a, const T* b, const float* bias, T* c, const GemmArgs& args,
-                  bool vector_c, bool spans_a, bool spans_b, hipStream_t stream) {
+                  bool vector_c, hipStream_t stream) {
     using S = Shape<T, WM, WN, TM, TN, BK>;
     const gemm::TileMap map = tile_map(args, S::kBM, S::kBN, sizeof(T));
     const std::int64_t tiles_m = (args.m + S::kBM - 1) / S::kBM;
@@ -68,14 +68,14 @@ hipError_t launch(const T* a, const T* b, const float* bias, T* c, const GemmArg
     // The occupancy hint caps registers; the element-wise operand paths need
     // more than it leaves, so they take the default.
     constexpr int kMinWaves = VecA && VecB ? MinWaves : 1;
-    constexpr auto kernel = gemm::gemm_kernel<T, WM, WN, TM, TN, BK, VecA, VecB, TransB, kMinWaves>;
+    constexpr auto kernel = gemm::gemm_kernel<T, WM, WN, TM, TN, BK, VecA, VecB, TransB, kMinWaves, Unaligned>;
     // Above 64 KiB of LDS a kernel has to opt in, once per device.
     if (const hipError_t opted = allow_lds<kernel>(S::kLdsBytes); opted != hipSuccess) {
         return opted;
     }
     const dim3 grid(static_cast<unsigned int>(tiles),
                     static_cast<unsigned int>(args.count < kMaxGridY ? args.count : kMaxGridY));
-    kernel<<<grid, S::kThreads, S::kLdsBytes, stream>>>(a, b, bias, c, args, map, vector_c, spans_a, spans_b);
+    kernel<<<grid, S::kThreads, S::kLdsBytes, stream>>>(a, b, bias, c, args, map, vector_c);
     return hipGetLastError();
 }
 
@@ -94,14 +94,32 @@ hipError_t pick_flags(const T* a, const T* b, const float* bias, T* c, const Gem
     const bool vec_b = spans_b && vector_operand(b, args.ldb, args.transposed ? args.k : args.n, args.stride_b,
                                                  args.outer_stride_b, split);
     const bool vec_c = vector_output(c, args);
-#define CUVIT_GEMM_LAUNCH(VA, VB)                                                                  \
-    (args.transposed                                                                               \
-         ? launch<T, WM, WN, TM, TN, BK, MinWaves, VA, VB, true>(a, b, bias, c, args, vec_c, spans_a, spans_b, stream) \
-         : launch<T, WM, WN, TM, TN, BK, MinWaves, VA, VB, false>(a, b, bias, c, args, vec_c, spans_a, spans_b, stream))
-    if (vec_a) {
-        return vec_b ? CUVIT_GEMM_LAUNCH(true, true) : CUVIT_GEMM_LAUNCH(true, false);
+#define CUVIT_GEMM_LAUNCH(VA, VB, U)                                                               \
+    (args.transposed ? launch<T, WM, WN, TM, TN, BK, MinWaves, VA, VB, true, U>(a, b, bias, c, args, vec_c, stream) \
+                     : launch<T, WM, WN, TM, TN, BK, MinWaves, VA, VB, false, U>(a, b, bias, c, args, vec_c, stream))
+    if (vec_a && vec_b) {
+        return CUVIT_GEMM_LAUNCH(true, true, false);
     }
-    return vec_b ? CUVIT_GEMM_LAUNCH(false, true) : CUVIT_GEMM_LAUNCH(false, false);
+    if constexpr (sizeof(T) == 4) {
+        // fp32 rows that start at any float, through the resources all the same
+        // (577 x 64 x 577 in 24 entries 25 us element by element, 20 so). Not where
+        // neither operand has aligned rows, most of a short K is a cut stage's four
+        // loads a chunk, and enough workgroups share a CU to hide the element-wise
+        // loads: 577 x 98 x 50 in 96 entries 28.5 us element by element, 36 so;
+        // 12000 x 577 x 65 38.5 and 43.
+        const bool element_wise = !vec_a && !vec_b && args.k < (args.transposed ? 64 : 128) &&
+                                  tile_count(args, 32, 32) > 20 * static_cast<std::int64_t>(compute_units());
+        if (spans_a && spans_b && !element_wise) {
+            return vec_a   ? CUVIT_GEMM_LAUNCH(true, false, true)
+                   : vec_b ? CUVIT_GEMM_LAUNCH(false, true, true)
+                           : CUVIT_GEMM_LAUNCH(false, false, true);
+        }
+        return CUVIT_GEMM_LAUNCH(false, false, false);
+    } else {
+        return vec_a   ? CUVIT_GEMM_LAUNCH(true, false, false)
+               : vec_b ? CUVIT_GEMM_LAUNCH(false, true, false)
+                       : CUVIT_GEMM_LAUNCH(false, false, false);
+    }
 #undef CUVIT_GEMM_LAUNCH
 }
 

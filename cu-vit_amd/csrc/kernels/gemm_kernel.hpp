@@ -306,17 +306,19 @@ __device__ __forceinline__ int split_point(int n, int parts, int i) { return n *
 /// in pairs; bf16 stages are 32 or 64 deep and run to a multiple of 128.
 template <typename T> constexpr int kSpan = sizeof(T) == 2 ? 128 : 64;
 
-/// @p spans_a, @p spans_b: an operand that is no vector operand (VecA, VecB
-/// false) still has its tile within one resource's span.
+/// @tparam Unaligned fp32 operands that are no vector operands (VecA, VecB
+/// false) have their tiles within one resource's span and are loaded through it.
+/// (An instance without both ways: with a choice between them in the kernel its
+/// registers cost a workgroup a CU.)
 /// @tparam MinWaves wavefronts per SIMD the register allocation must allow
 /// (amdgpu_waves_per_eu); 1 leaves the compiler free.
 template <typename T, int WM, int WN, int TM, int TN, int BK, bool VecA, bool VecB, bool TransB,
-          int MinWaves>
+          int MinWaves, bool Unaligned>
 __global__ __launch_bounds__(kWave * WM * WN) __attribute__((amdgpu_waves_per_eu(MinWaves))) void gemm_kernel(const T* __restrict__ a,
                                                         const T* __restrict__ b,
                                                         const float* __restrict__ bias, T* c,
-                                                        GemmArgs args, TileMap map, bool vector_c,
-                                                        bool spans_a, bool spans_b) {
+                                                        GemmArgs args, TileMap map, bool vector_c) {
+    static_assert(!Unaligned || sizeof(T) == 4, "fp32 only");
     using S = Shape<T, WM, WN, TM, TN, BK>;
     constexpr int BM = S::kBM;
     constexpr int BN = S::kBN;
@@ -397,7 +399,7 @@ __global__ __launch_bounds__(kWave * WM * WN) __attribute__((amdgpu_waves_per_eu
                         ra[p] = buffer_load16(a_resource,
                                               chunk_offset<T>(row, a_rows, args.lda, k, args.k));
                     } else {
-                        if (sizeof(T) == 4 && spans_a) {
+                        if constexpr (Unaligned) {
                             ra[p] = load_chunk_unaligned(a_resource, row, a_rows, args.lda, k, args.k,
                                                          k0 + BK <= args.k);
                         } else {
@@ -417,7 +419,7 @@ __global__ __launch_bounds__(kWave * WM * WN) __attribute__((amdgpu_waves_per_eu
                             rb[p] = buffer_load16(b_resource,
                                                   chunk_offset<T>(row, b_rows, args.ldb, k, args.k));
                         } else {
-                            if (sizeof(T) == 4 && spans_b) {
+                            if constexpr (Unaligned) {
                                 rb[p] = load_chunk_unaligned(b_resource, row, b_rows, args.ldb, k, args.k,
                                                              k0 + BK <= args.k);
                             } else {
@@ -433,7 +435,7 @@ __global__ __launch_bounds__(kWave * WM * WN) __attribute__((amdgpu_waves_per_eu
                             rb[p] = buffer_load16(b_resource,
                                                   chunk_offset<T>(k, args.k, args.ldb, n, b_rows));
                         } else {
-                            if (sizeof(T) == 4 && spans_b) {
+                            if constexpr (Unaligned) {
                                 rb[p] = load_chunk_unaligned(b_resource, k, args.k, args.ldb, n, b_rows,
                                                              BN <= b_rows);
                             } else {
