@@ -144,10 +144,10 @@ constexpr double kRingCostGelu[3] = {1.1, 1.85, 3.3};
 /// A tile alone on its CU, with nothing beside it to cover its waits (128 x 64:
 /// 4616 x 384 x 384 5.7 us against 5.3 with two 64 x 64 tiles per CU).
 constexpr double kRingCostAlone[3] = {1.3, 2.1, 3.0};
-/// With GELU two 64 x 64 tiles are the faster ones, above all where a long K
-/// gives them three stages (6504 x 240 x 3072: 30.8 us on 128 x 64, 21.9 on 64 x
-/// 64, 41 and 31 with operands from HBM).
-constexpr double kRingCostAloneGelu[3] = {1.3, 2.3, 3.0};
+/// With GELU and a long K two 64 x 64 tiles with three stages are the faster
+/// ones (6504 x 240 x 3072: 30.8 us on 128 x 64, 21.9 on 64 x 64, 41 and 31 with
+/// operands from HBM; but 6338 x 264 x 384 7.8 and 8.7).
+constexpr double kRingCostAloneGeluLongK[3] = {1.3, 2.3, 3.0};
 constexpr double kDmaRow = 0.035;
 constexpr double kDmaRowGelu = 0.043;
 /// What a round that fills an XCD's slots but for one or none costs more: a
@@ -203,7 +203,7 @@ inline RingChoice choose_ring(const GemmArgs& args, int units) {
         const gemm::TileMap map = ring_map(args, kHeights[i], kWidths[i], 2);
         const std::int64_t share = largest_share(args, map, kHeights[i], kWidths[i]);
         const std::int64_t rounds = (share + slots - 1) / slots;
-        double cost = rounds <= 1 ? (args.gelu ? kRingCostAloneGelu[i] : kRingCostAlone[i])
+        double cost = rounds <= 1 ? (args.gelu && args.k >= 1024 ? kRingCostAloneGeluLongK[i] : kRingCostAlone[i])
                                   : static_cast<double>(rounds) * (args.gelu ? kRingCostGelu[i] : kRingCost[i]);
         if (32 * share > 31 * rounds * slots) {
             cost *= kFullRound;
