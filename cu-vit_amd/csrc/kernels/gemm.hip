@@ -1,7 +1,7 @@
 // Host dispatch of the batched GEMM. The kernels, all measured on MI355X at
 // the ViT shapes and picked in this order:
 //   fp32 (16 x 16 MFMA): the resident-panel kernel (gemm_panel.hpp) for
-//        tall products with B as [N, K] and K of 192, or 768 into few columns
+//        tall products with B as [N, K] and K of 192, or 768 into up to 1024 columns
 //        (the ViT-Tiny linear layers and patch embedding); the ring kernel
 //        (gemm_ring.hpp) for the others with B as [N, K] and 16-byte rows, but
 //        for some of the largest; else the tiled kernel (gemm_kernel.hpp), 32 x

@@ -3,27 +3,30 @@
 // with too few tiles for the persistent kernel or no whole 256-column tiles. One
 // tile per workgroup, operands brought into an LDS ring by direct-to-LDS loads.
 //
-// What bounds these. Tiles are few and K is short (6 to 48 stages of 64), so
-// a tile's time is the latency of its first loads, its LDS traffic and its
-// epilogue; and a CU's LDS, not its MFMAs, is the busiest unit: a 64-deep
-// stage of a 128 x 128 tile writes 32 KB and reads 96 KB of fragments for 512
-// cycles of MFMA per SIMD. Loads through registers (gemm_kernel.hpp) hold
-// registers and add a write instruction per 16 bytes; here the loads land by
-// themselves and two stages per workgroup leave room for two (128 x 128) to
-// four (64 x 64) workgroups per CU, which cover each other's waits. Measured
-// on MI355X with two, three, four and eight stages: two are the fastest of
-// each tile, except for a tile alone on its CU with a long K, which has
-// nothing but its own loads to hide behind and takes three (4616 x 768 x
-// 3072: 31 -> 27 us). Eight wavefronts of 32 x 64 beat four of 64 x 64 on the
-// 128 x 128 tile (4616 x 2304 x 768: 24.7 against 25.7 us).
-// Before (gemm_kernel.hpp and gemm_dma.hpp) and now, bf16, us:
-//   4616 x 1152 x 384          18.0 ->  9.9    197 x 768 x 768 (+=)    8.6 -> 4.4
-//   4616 x 384 x 1536 (+=)     17.5 -> 10.6    1576 x 2304 x 768      17.4 -> 9.4
-//   4616 x 1536 x 384 (GELU)   18.2 -> 13.8    3152 x 2304 x 768      19.2 -> 16.1
-//   6304 x 192 x 768 (+=)      11.4 ->  6.5    12608 x 1152 x 384     38.2 -> 19.6
-// and fp32 (MFMA-bound from a few tiles per CU on):
-//   197 x 192 x 768 (+=)        8.5 ->  6.6    1576 x 2304 x 768      60.3 -> 54.7
-//   788 x 3072 x 768 (GELU)    45.6 -> 36.0    3152 x 768 x 3072      158  -> 126
+// What bounds these. Tiles are few and K is short (1 to 48 stages of 64), so
+// a tile's time is the latency of its first loads, its waits for a stage and its
+// epilogue: at 8224 x 768 x 768 in bf16 with operands from HBM the wavefronts
+// wait 63% of their cycles, the MFMAs are busy 15% and the LDS 14%. In fp32 with
+// several tiles a CU it is the MFMAs (58% busy at 1576 x 2304 x 768). Loads
+// through registers (gemm_kernel.hpp) hold registers and add a write instruction
+// per 16 bytes; here the loads land by themselves and two stages per workgroup
+// leave room for two (128 x 128) to four (64 x 64) workgroups per CU, which
+// cover each other's waits. So two stages are the faster of most tiles, and
+// more where little else covers the waits: bf16 three for 64 x 64 tiles alone on
+// their CUs or two a CU with a long K and for 128 x 128 tiles alone on their CUs
+// (4616 x 768 x 3072: 31 -> 27 us), four for 64 x 32 tiles alone; fp32 three for
+// 32 x 16 tiles alone and for 32 x 32 tiles with K above 128 (gemm_choice.hpp has
+// the rules). Eight wavefronts of 32 x 64 beat four of 64 x 64 on the 128 x 128
+// tile (4616 x 2304 x 768: 24.7 against 25.7 us).
+// Before (gemm_kernel.hpp and others since gone) and now, operands in the caches,
+// one card, us; bf16:
+//   4616 x 1152 x 384          18.4 -> 10.7    197 x 768 x 768 (+=)    8.9 -> 4.9
+//   4616 x 384 x 1536 (+=)     18.2 -> 12.5    1576 x 2304 x 768      17.9 -> 10.9
+//   4616 x 1536 x 384 (GELU)   18.6 -> 14.9    8224 x 768 x 768       19.0 -> 16.2
+//   6304 x 192 x 768 (+=)      11.9 ->  7.4    12608 x 1152 x 384     38.7 -> 20.5
+// and fp32:
+//   197 x 192 x 768 (+=)        8.7 ->  6.8    577 x 577 x 64 x 24    32.2 -> 21.6
+//   788 x 3072 x 768 (GELU)    43.9 -> 40.4    3152 x 768 x 3072      140  -> 128
 //
 // With kAhead a stage's fragments are read during the stage before, and its
 // loads go out between two k-blocks' MFMAs: a wavefront waits about 85 cycles
@@ -42,12 +45,12 @@
 // out too, with an offset past the descriptor's range (zeros, no traffic), so
 // that the count in flight is the same in every trip.
 //
-// Epilogue and arithmetic are gemm_dma.hpp's: 32 rows at a time through the
-// wavefront's own piece of the drained ring, stored as 16-byte pieces (single
-// elements where C's rows are not 16-byte aligned); the same MFMA over the
-// same K order, then alpha, bias, addend, GELU, old C, one rounding, so the
-// results are bitwise those of the other bf16 kernels. Old C is read before
-// the k loop.
+// Epilogue and arithmetic of the bf16 kernel are gemm_dma.hpp's: 32 rows at a
+// time through the wavefront's own piece of the drained ring, stored as 16-byte
+// pieces (8 bytes or single elements where C's rows are not so aligned); the same
+// MFMA over the same K order, then alpha, bias, addend, GELU, old C, one
+// rounding, so the results are bitwise those of the other kernels of its type,
+// as the fp32 kernel's are. Old C is read before the k loop.
 #pragma once
 
 #include "gemm_dma.hpp"
