@@ -280,7 +280,8 @@ struct RingChoiceF32 {
 /// 12608 x 320 x 384 41 us on 64 x 64, 36 on 32 x 32 with three. So three stages
 /// there, but for many tiles a CU, where more workgroups hide as much (1576 x
 /// 2304 x 768 54 us with two, 57 with three), and a larger tile only with a long
-/// K and many tiles (10602 x 744 x 3072: 386 us on 64 x 64, 429 on 32 x 32).
+/// K and many tiles (10602 x 744 x 3072: 386 us on 64 x 64, 429 on 32 x 32) or
+/// with more of them than the tiled kernel leaves to the ring.
 /// Entries dealt to the XCDs whole come from the L2 (196 x 200 x 384 in 192
 /// entries: 75 us with two stages), and take three for few tiles a CU only.
 inline RingChoiceF32 choose_ring_f32(const GemmArgs& args, int units) {
@@ -296,7 +297,8 @@ inline RingChoiceF32 choose_ring_f32(const GemmArgs& args, int units) {
     const gemm::TileMap map = ring_map(args, 32, 32, 4);
     const bool by_entry = map.px < 0;
     const std::int64_t small_rounds = (largest_share(args, map, 32, 32) + slots - 1) / slots;
-    const int candidates = by_entry || args.k <= 128 || (args.k >= 1024 && small_rounds > 6) ? 3 : 1;
+    const bool larger = by_entry || args.k <= 128 || small_rounds > (args.k >= 1024 ? 6 : 32);
+    const int candidates = larger ? 3 : 1;
     RingChoiceF32 best{RingTileF32::k32x32, map};
     double best_cost = 0.0;
     for (int i = 0; i < candidates; ++i) {
@@ -317,9 +319,12 @@ inline RingChoiceF32 choose_ring_f32(const GemmArgs& args, int units) {
 /// kernel: with many tiles a CU and operands that come from several XCDs' worth
 /// of L2 (12507 x 1928 x 512: 224 to 232 us against 235 to 262 by tile; 8221 x
 /// 1376 x 768 159 against 160 to 174). At K = 64 the ring is ahead, and at K of
-/// 1024 its 64 x 64 tiles are (10602 x 744 x 3072: 386 against 440).
+/// 1024 its 64 x 64 tiles are (10602 x 744 x 3072: 386 against 440). Entries run
+/// as one problem are the ring's unless they are whole 64-row tiles, since the
+/// tiled kernel's stop at each (768 x 588 on 64 entries of 196 rows 151 us there,
+/// 126 on the ring; of 256 rows 136 and 149).
 inline bool tiled_beats_ring_f32(const GemmArgs& args, int units) {
-    return args.k > 64 && (args.count > 1 || args.k < 1024) &&
+    return args.rows_per_entry % 64 == 0 && args.k > 64 && (args.count > 1 || args.k < 1024) &&
            tile_count(args, 32, 32) > 32 * static_cast<std::int64_t>(units) && ring_map(args, 32, 32, 4).px >= 0;
 }
 

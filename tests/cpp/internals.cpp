@@ -39,9 +39,11 @@ int bf16_choice(int m, int n, int k, int count, int gelu, int persistent_fits, i
     return static_cast<int>(ring.tile);
 }
 
-/// A RingTileF32's number, or 5 for the tiled kernel.
-int f32_choice(int m, int n, int k, int count, int units) {
-    const GemmArgs args = problem(m, n, k, count, 0);
+/// A RingTileF32's number, or 5 for the tiled kernel; @p rows_per_entry > 0:
+/// entries run as one problem.
+int f32_choice(int m, int n, int k, int count, int units, int rows_per_entry) {
+    GemmArgs args = problem(m, n, k, count, 0);
+    args.rows_per_entry = rows_per_entry;
     return tiled_beats_ring_f32(args, units) ? 5 : static_cast<int>(choose_ring_f32(args, units).tile);
 }
 
